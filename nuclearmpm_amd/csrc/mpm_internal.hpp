@@ -130,8 +130,8 @@ struct CompactArgs {
 
 namespace nclr_host {
 
-// Fewer full work items than this (the chip's CUs) make a 2D launch latency-bound: P2G and the G2P
-// adjoint then run one particle per thread.
+// Fewer full work items than this (the chip's CUs; 3D P2G: than four times this) make a launch
+// latency-bound: P2G and the 2D G2P adjoint then run one particle per thread.
 constexpr int kFewItems = 256;
 
 struct LaunchArgs {

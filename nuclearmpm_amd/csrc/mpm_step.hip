@@ -645,30 +645,31 @@ static hipError_t sort_dispatch(const LaunchArgs& a) {
     return hipGetLastError();
 }
 
-// 256 threads, chunk / 256 particles each; in 2D, when the particles fill fewer work items than
-// the chip has CUs, one particle per thread (a workgroup of chunk threads), which halves the
-// latency of a work item (the results are the same: the sums are exact and the scale is the
-// item's maximum).  Measured: the 19,600-particle 2D jelly step's P2G faster, the 1.75M-particle
-// 2D batch's slower with it.
+// 256 threads with chunk / 256 particles each, or, when the particles fill few work items, one
+// particle per thread (a workgroup of chunk threads), which shortens a work item's latency (the
+// results are the same: the sums are exact and the scale is the item's maximum).  The line:
+//   2D  fewer full work items than the chip has CUs.  The 19,600-particle 2D jelly step's P2G is
+//       faster with it, the 1.75M-particle 2D batch's slower.
+//   3D  fewer than four full work items per CU, which is what the 36 KB of accumulators lets a CU
+//       hold at 256 threads: every item is resident at once and the launch takes as long as its
+//       items.  Chunk 512: 60,007 snow particles 32.8 -> 27.2 us, 150,003 jelly 39.4 -> 35.9,
+//       24 x 9,261 jelly 51.8 -> 48.9; but 680,943 snow (accurate) 81.7 -> 85.4 and 2.1M jelly
+//       214 -> 221, where a CU's next items hide the latency and the wider barriers only cost.
+template <int D, int MAT, int PPT, int MODE>
+static void p2g_mode(const LaunchArgs& a) {
+    const unsigned g = unsigned((a.p.n + 256 * PPT - 1) / (256 * PPT) + a.p.ntiles);
+    if (a.p.n < int64_t(D == 2 ? kFewItems : 4 * kFewItems) * 256 * PPT)
+        k_p2g_tile<D, MAT, 1, MODE, 256 * PPT><<<g, 256 * PPT, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p,
+                                                                             a.slots);
+    else
+        k_p2g_tile<D, MAT, PPT, MODE><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p, a.slots);
+}
+
 template <int D, int MAT, int PPT>
 static hipError_t p2g_one(const LaunchArgs& a) {
-    const int64_t items = (a.p.n + 256 * PPT - 1) / (256 * PPT) + a.p.ntiles;
-    const unsigned g = unsigned(items);
-    if constexpr (D == 2) {
-        if (a.p.n < int64_t(kFewItems) * 256 * PPT)
-            k_p2g_tile<D, MAT, 1, kSvdExact, 256 * PPT><<<g, 256 * PPT, 0, a.stream>>>(a.state_in, a.perm,
-                                                                                     a.item_offset, a.p, a.slots);
-        else
-            k_p2g_tile<D, MAT, PPT, kSvdExact><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p,
-                                                                       a.slots);
-    } else if (a.svd_mode == kSvdFast) {
-        k_p2g_tile<D, MAT, PPT, kSvdFast><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p, a.slots);
-    } else if (a.svd_mode == kSvdAccurate) {
-        k_p2g_tile<D, MAT, PPT, kSvdAccurate><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p,
-                                                                      a.slots);
-    } else {
-        k_p2g_tile<D, MAT, PPT, kSvdExact><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p, a.slots);
-    }
+    if (D == 3 && a.svd_mode == kSvdFast) p2g_mode<D, MAT, PPT, D == 3 ? kSvdFast : kSvdExact>(a);
+    else if (D == 3 && a.svd_mode == kSvdAccurate) p2g_mode<D, MAT, PPT, D == 3 ? kSvdAccurate : kSvdExact>(a);
+    else p2g_mode<D, MAT, PPT, kSvdExact>(a);
     return hipGetLastError();
 }
 
