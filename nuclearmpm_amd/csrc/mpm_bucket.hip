@@ -255,6 +255,7 @@ __global__ __launch_bounds__(1024) void k_bucket_scan(StepParams p, uint32_t chu
         meta[0] = cp;
         meta[1] = 0;
         meta[2] = s_seen;
+        meta[kMetaGridTiles] = 0;
     }
 }
 
@@ -286,6 +287,7 @@ __global__ __launch_bounds__(1024) void k_bucket_rounds(StepParams p, uint32_t c
         item_offset[p.ntiles] = ci + ti;
         meta[0] = cp + tp;
         meta[1] = 0;
+        meta[kMetaGridTiles] = 0;
     }
 }
 
@@ -297,9 +299,18 @@ __global__ __launch_bounds__(256) void k_bucket_scatter(StepParams p, const uint
                                                         const uint32_t* __restrict__ tile_start,
                                                         const uint32_t* __restrict__ pid,
                                                         uint32_t* __restrict__ meta, uint32_t* __restrict__ perm,
-                                                        uint32_t* __restrict__ keys, uint32_t* __restrict__ status) {
+                                                        uint32_t* __restrict__ keys, uint32_t* __restrict__ status,
+                                                        uint32_t list_blocks,
+                                                        const uint32_t* __restrict__ item_offset,
+                                                        GridTile<D>* __restrict__ tiles,
+                                                        uint32_t* __restrict__ active) {
     using B = Buckets<D>;
-    const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (blockIdx.x < list_blocks) {  // the first workgroups list the node tiles (a chain of dependent
+                                     // loads: behind the particles' workgroups it made a tail of 4 us)
+        list_grid_tile<D>(p, blockIdx.x * 256 + threadIdx.x, item_offset, tiles, &meta[kMetaGridTiles], active);
+        return;
+    }
+    const int64_t j = int64_t(blockIdx.x - list_blocks) * blockDim.x + threadIdx.x;
     if (j >= p.n) return;
     const uint32_t seen = meta[2];
     uint32_t pos, key;
@@ -353,10 +364,12 @@ static hipError_t bucket_dispatch(const LaunchArgs& a) {
         k_bucket_rounds<D><<<rounds, 1024, 0, s>>>(p, uint32_t(p.chunk), a.item_offset, a.tile_start, a.tile_end,
                                                    a.ttotal, a.rtot, a.meta);
     }
-    if (p.n > 0)
-        k_bucket_scatter<D><<<unsigned((p.n + 255) / 256), 256, 0, s>>>(p, a.keys_tmp, a.perm_tmp, a.uidx, a.upref,
-                                                                        a.tile_start, a.pid_in, a.meta, a.perm,
-                                                                        a.keys, a.status);
+    const unsigned pb = unsigned((p.n + 255) / 256);
+    const unsigned tb = grid_tiles_listed(D, p) ? (p.node_tiles + 255) / 256 : 0;
+    if (pb + tb > 0)
+        k_bucket_scatter<D><<<pb + tb, 256, 0, s>>>(p, a.keys_tmp, a.perm_tmp, a.uidx, a.upref, a.tile_start, a.pid_in,
+                                                    a.meta, a.perm, a.keys, a.status, tb, a.item_offset,
+                                                    static_cast<GridTile<D>*>(a.grid_tiles), a.active);
     return hipGetLastError();
 }
 

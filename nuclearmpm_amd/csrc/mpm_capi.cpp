@@ -119,12 +119,13 @@ struct nclr_mpm_sim {
     int echunks = 1;
     float* gtmp[2] = {nullptr, nullptr};
     char* tape = nullptr;  // saved states of a backward segment
-    // The sort's outputs (keys, perm, tile bounds, item offsets, the item table, meta) live in one
+    // The sort's outputs (keys, perm, tile bounds, item offsets, the item and node tile lists, meta) live in one
     // block at fixed offsets, so a backward segment can run each recomputed step's sort in a block
     // of its own (a sort tape entry) and the adjoint kernels read it there.
     char* sort_block = nullptr;
     size_t sort_block_bytes = 0;
-    size_t so_keys = 0, so_perm = 0, so_ts = 0, so_te = 0, so_io = 0, so_items = 0, so_meta = 0;
+    size_t so_keys = 0, so_perm = 0, so_ts = 0, so_te = 0, so_io = 0, so_items = 0, so_meta = 0, so_gtiles = 0;
+    void* grid_tiles = nullptr;
     // the block the next incremental sort reads the old order's work items and meta from, when it
     // sorts into another block (nullptr: the current one)
     char* prev_sort = nullptr;
@@ -184,6 +185,7 @@ struct nclr_mpm_sim {
         a.upref = upref;
         a.ttotal = ttotal;
         a.meta = meta;
+        a.grid_tiles = grid_tiles;
         a.rtot = rtot;
         a.prev_item_offset = prev_sort ? reinterpret_cast<const uint32_t*>(prev_sort + so_io) : item_offset;
         a.prev_items = prev_sort ? reinterpret_cast<const uint4*>(prev_sort + so_items) : p.items;
@@ -690,8 +692,8 @@ struct nclr_mpm_sim {
         return echunks;
     }
 
-    // keys, perm (n each), tile_start, tile_end, item_offset (ntiles + 1 each), the item table and
-    // meta, each 256-byte aligned inside one allocation
+    // keys, perm (n each), tile_start, tile_end, item_offset (ntiles + 1 each), the item table, meta
+    // and the list of node tiles, each 256-byte aligned inside one allocation
     hipError_t alloc_sort_block(size_t nn, size_t nbins, size_t max_items) {
         size_t off = 0;
         auto take = [&](size_t bytes) {
@@ -703,6 +705,7 @@ struct nclr_mpm_sim {
         const size_t o_ts = take(nbins * sizeof(uint32_t)), o_te = take(nbins * sizeof(uint32_t));
         const size_t o_io = take(nbins * sizeof(uint32_t)), o_items = take(max_items * sizeof(uint4));
         const size_t o_meta = take(4 * sizeof(uint32_t));
+        const size_t o_gtiles = take(size_t(p.node_tiles) * nclr_host::grid_tile_bytes(dim));
         const hipError_t e = hipMalloc(reinterpret_cast<void**>(&sort_block), off);
         if (e != hipSuccess) return e;
         sort_block_bytes = off;
@@ -713,6 +716,7 @@ struct nclr_mpm_sim {
         so_io = o_io;
         so_items = o_items;
         so_meta = o_meta;
+        so_gtiles = o_gtiles;
         point_sort_block(sort_block);
         return hipSuccess;
     }
@@ -726,6 +730,7 @@ struct nclr_mpm_sim {
         item_offset = reinterpret_cast<uint32_t*>(base + so_io);
         p.items = reinterpret_cast<uint4*>(base + so_items);
         meta = reinterpret_cast<uint32_t*>(base + so_meta);
+        grid_tiles = base + so_gtiles;
     }
 
     int ensure_adjoint() {

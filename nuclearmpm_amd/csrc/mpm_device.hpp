@@ -5,6 +5,9 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <type_traits>
+
 #include "mpm_internal.hpp"
 #include "mpm_math.hpp"
 
@@ -229,6 +232,229 @@ NCLR_DI void write_items(uint4* __restrict__ items, uint32_t first, uint32_t cou
     for (uint32_t k = 0; k < count; ++k) {
         const uint32_t j0 = start + k * chunk;
         items[first + k] = make_uint4(tile, j0, min(j0 + chunk, end), 0u);
+    }
+}
+
+// The node tiles that particles reach, listed by the sort for the kernels over the grid (a batch's
+// node tiles are mostly empty: a workgroup for each costs more than the work, e.g. 39,304 for 8
+// scenes of res 128 with some 1,700 in use), with the work items whose slots reach them.  Candidate
+// c of node tile T is the particle tile T - delta, bit a of c the delta on axis a; its slot region
+// reaches the nodes of T with local coordinate < 2 on every axis with delta_a = 1.
+template <int D>
+struct GridTile {
+    int node_tile, scene;
+    int first[1 << D];  // first P2G work item of candidate c (its slot)
+    int count[1 << D];  // number of its work items
+};
+
+// Candidate c of node tile t of scene sp: its first work item and their number (0, 0 off the grid).
+template <int D>
+NCLR_DI void grid_tile_candidate(const SceneParams& sp, const int (&nto)[D], int c,
+                                 const uint32_t* __restrict__ item_offset, int& first, int& count) {
+    uint32_t k = 0;
+    bool valid = true;
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        const int ta = nto[a] - ((c >> a) & 1);
+        valid = valid && ta >= 0 && ta < sp.nt;
+        k = k * uint32_t(sp.nt) + uint32_t(ta);
+    }
+    first = valid ? int(item_offset[sp.tile_base + k]) : 0;
+    count = valid ? int(item_offset[sp.tile_base + k + 1]) - first : 0;
+}
+
+// 2D launches with few work items (kFewItems) have few node tiles too, and no list: a workgroup per node
+// tile looks its candidates up (19,600 jelly particles, forward + backward: 2.20 ms, 2.28 with a list).
+inline bool grid_tiles_listed(int dim, const StepParams& p) {
+    return dim == 3 || p.n >= int64_t(nclr_host::kFewItems) * p.chunk;
+}
+
+// Lists node tile t (t in 0 .. node_tiles - 1, one per thread of whole waves; others pass t past the end).
+// The order of the list is free: every node tile is computed by itself.
+template <int D>
+NCLR_DI void list_grid_tile(const StepParams& p, uint32_t t, const uint32_t* __restrict__ item_offset,
+                            GridTile<D>* __restrict__ out, uint32_t* count, uint32_t* __restrict__ active) {
+    GridTile<D> g;
+    bool occupied = false;
+    if (t < p.node_tiles) {
+        g.node_tile = int(t);
+        g.scene = p.nscenes == 1 ? 0 : scene_of_node_tile(p, t);
+        if (!scene_stopped(p, g.scene)) {  // a stopped scene's grid keeps its last completed step
+            const SceneParams& sp = p.scenes[g.scene];
+            int nto[D];
+            tile_coords<D>(t - sp.node_tile_base, sp.ntn, nto);
+#pragma unroll
+            for (int c = 0; c < (1 << D); ++c) {
+                grid_tile_candidate<D>(sp, nto, c, item_offset, g.first[c], g.count[c]);
+                occupied = occupied || g.count[c] > 0;
+            }
+            if (!occupied) active[t] = 0u;
+        }
+    }
+    const uint64_t m = __ballot(occupied);
+    const int lane = int(threadIdx.x) & 63;
+    uint32_t at = 0;
+    if (lane == 0 && m != 0ull) at = atomicAdd(count, uint32_t(__popcll(m)));
+    at = __shfl(at, 0) + uint32_t(__popcll(m & ((1ull << lane) - 1ull)));
+    if (occupied) out[at] = g;
+}
+
+// Entry i of this workgroup's share of the list: the k-th of XCD (block % 8)'s eighth of the list, k =
+// block / 8 + i * (grid / 8), so that neighbouring entries share an XCD's L2.  False past the share.
+NCLR_DI bool grid_tile_index(uint32_t count, uint32_t i, uint32_t& index) {
+    const uint32_t per = (count + kXcds - 1) / kXcds, k = blockIdx.x / kXcds + i * (gridDim.x / kXcds);
+    index = (blockIdx.x % kXcds) * per + k;
+    return k < per && index < count;
+}
+// Workgroups of a launch over the list: every node tile, as far as that is not mostly empty ones.
+constexpr uint32_t kMaxGridBlocks = 8192;
+inline unsigned grid_tile_blocks(uint32_t node_tiles) { return xcd_grid(std::min(node_tiles, kMaxGridBlocks)); }
+
+// The node classes of a node tile: bit a is set where the local coordinate is below 2 on axis a, and
+// class T's nodes are reached by the candidates c whose bits are all in T.  Threads take the nodes
+// class by class (interior nodes first, rows kept together), so that a wave's lanes have the same
+// slots to sum: of the 40 wave loads per work item that row order takes in 3D, 17 are left.
+template <int D>
+struct NodeOrder {
+    uint16_t node[Tile<D>::NODES];  // class << 9 | node
+};
+template <int D>
+constexpr NodeOrder<D> make_node_order() {
+    NodeOrder<D> o{};
+    int at = 0;
+    for (int bits = 0; bits <= D; ++bits)
+        for (int T = 0; T < (1 << D); ++T) {
+            int b = 0;
+            for (int a = 0; a < D; ++a) b += (T >> a) & 1;
+            if (b != bits) continue;
+            for (int l = 0; l < Tile<D>::NODES; ++l) {
+                int cls = 0;
+                for (int a = 0; a < D; ++a) {
+                    const int la = (l >> (Tile<D>::LOG * (D - 1 - a))) & (Tile<D>::S - 1);
+                    cls |= la < Tile<D>::R - Tile<D>::S ? 1 << a : 0;
+                }
+                if (cls == T) o.node[at++] = uint16_t(T << 9 | l);
+            }
+        }
+    return o;
+}
+static __constant__ const NodeOrder<2> kNodeOrder2 = make_node_order<2>();
+static __constant__ const NodeOrder<3> kNodeOrder3 = make_node_order<3>();
+template <int D>
+NCLR_DI uint32_t node_order(int t) {
+    if constexpr (D == 2) return kNodeOrder2.node[t];
+    else return kNodeOrder3.node[t];
+}
+
+NCLR_DI void add4(float4& acc, const float4 t) {
+    acc.x += t.x;
+    acc.y += t.y;
+    acc.z += t.z;
+    acc.w += t.w;
+}
+
+// The node a thread of a grid kernel computes in every node tile: local index l, class cls, the classes of
+// its wave's nodes, and its index r in the slot region of the node tile's own particle tile.
+template <int D>
+struct GridThread {
+    int l, cls, r;
+    int lc[D];
+    uint32_t wave_classes;
+    NCLR_DI GridThread() {
+        using TL = Tile<D>;
+        const uint32_t order = node_order<D>(int(threadIdx.x));
+        l = int(order & 511u);
+        cls = int(order >> 9);
+        wave_classes = 0;
+#pragma unroll
+        for (int T = 0; T < (1 << D); ++T) wave_classes |= __ballot(cls == T) != 0ull ? 1u << T : 0u;
+        r = 0;
+#pragma unroll
+        for (int a = 0; a < D; ++a) {
+            lc[a] = (l >> (TL::LOG * (D - 1 - a))) & (TL::S - 1);
+            r = r * TL::R + lc[a];
+        }
+    }
+    NCLR_DI void node(uint32_t tile, int ntn, int (&n)[D]) const {
+        tile_coords<D>(tile, ntn, n);
+#pragma unroll
+        for (int a = 0; a < D; ++a) n[a] = n[a] * Tile<D>::S + lc[a];
+    }
+};
+
+// The slots that reach each class's nodes, 64 at a time, in LDS: candidates in order, a candidate's
+// items in order.  list[T][e]: the slot's first node (shifted by the candidate's offset inside the
+// region), or -1 past the list.  GROUP 4: item it of a candidate stands at a position congruent to
+// it mod 4 (a candidate's items are padded with -1).
+template <int D>
+struct SlotLists {
+    int64_t list[1 << D][64];
+};
+
+template <int GROUP>
+NCLR_DI int list_positions(int count) {
+    return (count + GROUP - 1) / GROUP * GROUP;
+}
+
+// Positions e0 .. e0 + 63 of class T's list, by one wave.
+template <int D, int GROUP>
+NCLR_DI void build_list(int64_t* list, const int (&first)[1 << D], const int (&count)[1 << D], int T, int e0) {
+    using TL = Tile<D>;
+    const int lane = int(threadIdx.x) & 63;
+    int64_t at = -1;
+    int it = e0 + lane;  // the position, less the candidates before
+#pragma unroll
+    for (int c = 0; c < (1 << D); ++c) {
+        if ((c & ~T) != 0) continue;
+        int shift = 0;
+#pragma unroll
+        for (int a = 0; a < D; ++a) shift = shift * TL::R + ((c >> a) & 1) * TL::S;
+        if (it >= 0 && it < count[c]) at = int64_t(first[c] + it) * TL::REGION + shift;
+        it -= list_positions<GROUP>(count[c]);
+    }
+    list[lane] = at;
+}
+
+// Sums over the lists of a node tile's classes: load(u, at) for the positions u = 0 .. 7 (or 0 .. 3, or 0
+// and 1) of a round, whose loads are in flight together, then sum(positions).  The thread's nodes are
+// class t_class's; wave_classes: the classes of its wave's threads.  The whole workgroup (1 << D
+// waves) takes part.
+template <int D, int GROUP, typename Load, typename Sum>
+NCLR_DI void visit_slots(SlotLists<D>& lists, const int (&first)[1 << D], const int (&count)[1 << D], int t_class,
+                         uint32_t wave_classes, Load load, Sum sum) {
+    constexpr int NC = 1 << D;
+    int longest = 0, mine = 0;  // list lengths: every class's (the last class) and this wave's
+#pragma unroll
+    for (int T = 0; T < NC; ++T) {
+        longest = 0;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            if ((c & ~T) == 0) longest += list_positions<GROUP>(count[c]);
+        if ((wave_classes >> T) & 1u) mine = max(mine, longest);
+    }
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+    const int64_t* my_list = lists.list[t_class];
+    for (int e0 = 0; e0 < longest; e0 += 64) {
+        __syncthreads();  // the lists of the round (or tile) before have been read
+        build_list<D, GROUP>(lists.list[wave], first, count, wave, e0);
+        __syncthreads();
+        const int m = min(64, mine - e0);
+        int u0 = 0;
+        for (; u0 + 4 < m; u0 += 8) {
+#pragma unroll
+            for (int u = 0; u < 8; ++u) load(u, my_list[u0 + u]);
+            sum(std::integral_constant<int, 8>{});
+        }
+        if (u0 + 2 < m) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) load(u, my_list[u0 + u]);
+            sum(std::integral_constant<int, 4>{});
+        } else if (u0 < m) {
+            constexpr int N = GROUP > 2 ? GROUP : 2;
+#pragma unroll
+            for (int u = 0; u < N; ++u) load(u, my_list[u0 + u]);
+            sum(std::integral_constant<int, N>{});
+        }
     }
 }
 

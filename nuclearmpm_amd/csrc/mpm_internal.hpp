@@ -80,6 +80,9 @@ struct StepParams {
     uint32_t* scene_frozen;
 };
 
+// Word of the sort's meta counters that counts its list of node tiles (GridTile).
+constexpr int kMetaGridTiles = 3;
+
 // The compact step (mpm_compact.hip): dynamic LDS per workgroup for its box of nodes.
 constexpr int kCompactLdsBytes = 150 * 1024;
 constexpr int kCompactMaxWorkgroups = 256;
@@ -167,6 +170,7 @@ struct LaunchArgs {
     uint32_t* upref;           // max_items * offsets: per (old item, offset), earlier particles bound alike
     uint32_t* ttotal;          // ntiles: particles per new tile
     uint32_t* meta;            // 4 counters
+    void* grid_tiles;          // node_tiles GridTile<dim>: the node tiles the sorted particles reach (meta[kMetaGridTiles])
     uint32_t* rtot;            // 2 per round of the tile scans: particle and work-item totals
     // the incremental sort's inputs from the step before: its item offsets, item table and meta.
     // The same buffers as item_offset, p.items and meta, unless the step sorts into another block.
@@ -256,6 +260,7 @@ int set_last_error(int code, const char* msg);
 int num_fields(int dim);
 int region_nodes(int dim);
 int tile_nodes(int dim);
+size_t grid_tile_bytes(int dim);
 int tile_log(int dim);
 
 }  // namespace nclr_host

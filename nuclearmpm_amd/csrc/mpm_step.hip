@@ -103,6 +103,7 @@ __global__ __launch_bounds__(1024) void k_items(const uint32_t* __restrict__ sta
     if (threadIdx.x == 0) {
         item_offset[ntiles] = ci;
         meta[0] = cp;
+        meta[kMetaGridTiles] = 0;
     }
 }
 
@@ -129,6 +130,7 @@ __global__ __launch_bounds__(1024) void k_items_rounds(const uint32_t* __restric
     if (threadIdx.x == 0 && blockIdx.x + 1 == gridDim.x) {
         item_offset[ntiles] = ci + ti;
         meta[0] = cp + tp;
+        meta[kMetaGridTiles] = 0;
     }
 }
 
@@ -294,162 +296,123 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
 }
 
 // ---------------------------------------------------------------------------------------------
-// grid update (src/nclr.h:263-310): one workgroup per node tile (256 threads; 1024 for a 2D launch
-// with few work items).  In 3D a node sums its candidate tiles' work items in order; in 2D in four
-// partial sums, partial w over items w, w + 4, ... of every candidate tile in order, added in
-// partial order: four independent chains of additions behind the slot loads (the 256-scene 2D
-// batch 3.6 % faster; in 3D it measured slower).  The grid adjoint re-sums in the same order.
+// grid update (src/nclr.h:263-310): a workgroup per node tile that particles reach, a thread per node.
+// In 3D a node sums its candidate tiles' work items in order; in 2D in four partial sums, partial w over
+// items w, w + 4, ... of every candidate tile in order, added in partial order.  The grid adjoint
+// re-sums in the same order.
+//
+// Small launches wait on the chain of slot loads, large ones on their number.  The lists of slots
+// per class of nodes answer both: eight loads in flight across candidates, and no lane idle for a
+// candidate that reaches its neighbours only.  With the listed node tiles (empty ones cost a
+// workgroup before): 30,011 liquid particles 13.1 -> 7.4 us, 150,003 jelly 17.8 -> 9.5, 24 x 9,261
+// jelly 25.3 -> 13.6, 680,943 snow 31.9 -> 21.3, 1,048,576 spread snow 34.5 -> 27.8 (3.6 TB/s of slots
+// read and grid written, of 4.7 a copy reaches), 8 x 262,144 jelly 58 -> 36, 1.7M particles in 256
+// 2D scenes 26.2 -> 20.7.
 // ---------------------------------------------------------------------------------------------
 template <int D>
-__global__ __launch_bounds__(D == 2 ? 1024 : 256) void k_grid_tiles(const float4* __restrict__ slots,
-                                                    const uint32_t* __restrict__ item_offset, StepParams p,
-                                                    float4* __restrict__ gv, float4* __restrict__ gpre,
-                                                    uint32_t* __restrict__ stamps, uint32_t* __restrict__ active) {
+__global__ __launch_bounds__(Tile<D>::NODES) void k_grid_tiles(const float4* __restrict__ slots, StepParams p,
+                                                               const GridTile<D>* __restrict__ tiles,
+                                                               const uint32_t* __restrict__ meta,
+                                                               float4* __restrict__ gv, float4* __restrict__ gpre,
+                                                               uint32_t* __restrict__ stamps,
+                                                               uint32_t* __restrict__ active) {
     using TL = Tile<D>;
-    constexpr int NC = 1 << D;
-    __shared__ int s_first[NC];  // first P2G work item of candidate tile c (its slot), or -1
-    __shared__ int s_count[NC];  // number of work items of candidate tile c
-    __shared__ uint32_t s_active;
+    __shared__ SlotLists<D> s_lists;
+    const uint32_t listed = meta[kMetaGridTiles];
+    const GridThread<D> th;
+    uint32_t index;
+    for (uint32_t i = 0; grid_tile_index(listed, i, index); ++i) {
+        const GridTile<D> tile = tiles[index];  // uniform over the workgroup
+        if (scene_stopped(p, tile.scene)) continue;
+        const uint32_t nt_idx = uint32_t(tile.node_tile);
+        const SceneParams sp = p.scenes[tile.scene];
+        if (threadIdx.x == 0) stamps[nt_idx] = *p.stamp;
+        int n[D];
+        th.node(nt_idx - sp.node_tile_base, sp.ntn, n);
+        float4 g[D == 2 ? 4 : 1], v[8];
+#pragma unroll
+        for (int q = 0; q < (D == 2 ? 4 : 1); ++q) g[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        // a position past the node's list adds +0.0, which leaves a sum that started at +0.0 unchanged
+        visit_slots<D, D == 2 ? 4 : 1>(
+            s_lists, tile.first, tile.count, th.cls, th.wave_classes,
+            [&](int u, int64_t at) {
+                v[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (at >= 0) v[u] = slots[at + th.r];
+            },
+            [&](auto positions) {
+#pragma unroll
+                for (int u = 0; u < decltype(positions)::value; ++u) add4(g[D == 2 ? u & 3 : 0], v[u]);
+            });
+        if constexpr (D == 2)
+#pragma unroll
+            for (int q = 1; q < 4; ++q) add4(g[0], g[q]);
+        if (gpre) gpre[int64_t(nt_idx) * TL::NODES + th.l] = g[0];
+        gv[int64_t(nt_idx) * TL::NODES + th.l] = grid_node<D>(g[0], n, sp);
+        // nodes with post-P2G mass > 0, per node tile (summed on demand by mpm_active_nodes)
+        const int massive = __syncthreads_count(g[0].w > 0.0f);
+        if (threadIdx.x == 0) active[nt_idx] = uint32_t(massive);
+    }
+}
+
+// The same in 2D for a launch with few work items: a workgroup of 1024 threads per node tile, occupied or
+// not.  Quarter w of the workgroup computes partial sum w, which quarters the chain of slot loads
+// that a node waits on.
+__global__ __launch_bounds__(1024) void k_grid_tiles_few(const float4* __restrict__ slots,
+                                                         const uint32_t* __restrict__ item_offset, StepParams p,
+                                                         float4* __restrict__ gv, float4* __restrict__ gpre,
+                                                         uint32_t* __restrict__ stamps,
+                                                         uint32_t* __restrict__ active) {
+    using TL = Tile<2>;
+    constexpr int NC = 4;
+    __shared__ int s_first[NC], s_count[NC];
+    __shared__ float4 s_part[3][TL::NODES];
     const uint32_t nt_idx = xcd_block();
     if (nt_idx >= p.node_tiles) return;
     const int scene = p.nscenes == 1 ? 0 : scene_of_node_tile(p, nt_idx);
     if (scene_stopped(p, scene)) return;  // a stopped scene's grid keeps its last completed step
     const SceneParams sp = p.scenes[scene];
-    int nto[D];
-    tile_coords<D>(nt_idx - sp.node_tile_base, sp.ntn, nto);
+    int nto[2];
+    tile_coords<2>(nt_idx - sp.node_tile_base, sp.ntn, nto);
     bool occupied = false;
-    if (threadIdx.x == 0) s_active = 0;
     if (threadIdx.x < NC) {
-        int t = 0;
-        bool valid = true;
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            const int ta = nto[a] - ((threadIdx.x >> a) & 1);
-            valid = valid && ta >= 0 && ta < sp.nt;
-            t = t * sp.nt + ta;
-        }
-        const uint32_t gt = sp.tile_base + uint32_t(t);
-        const uint32_t first = valid ? item_offset[gt] : 0u;
-        const uint32_t count = valid ? item_offset[gt + 1] - first : 0u;
-        occupied = count > 0;
-        s_first[threadIdx.x] = occupied ? int(first) : -1;
-        s_count[threadIdx.x] = int(count);
+        grid_tile_candidate<2>(sp, nto, int(threadIdx.x), item_offset, s_first[threadIdx.x], s_count[threadIdx.x]);
+        occupied = s_count[threadIdx.x] > 0;
     }
     if (!__syncthreads_or(occupied)) {
         if (threadIdx.x == 0) active[nt_idx] = 0;
         return;
     }
-    const uint32_t stamp = *p.stamp;
-    if (threadIdx.x == 0) stamps[nt_idx] = stamp;
-    int first[NC], count[NC];
+    if (threadIdx.x == 0) stamps[nt_idx] = *p.stamp;
+    const int l = int(threadIdx.x) & (TL::NODES - 1), w = int(threadIdx.x) >> 8;
+    const int lc[2] = {l >> TL::LOG, l & (TL::S - 1)};
+    const int n[2] = {nto[0] * TL::S + lc[0], nto[1] * TL::S + lc[1]};
+    float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        first[c] = s_first[c];
-        count[c] = s_count[c];
+        const int r0 = lc[0] + (c & 1) * TL::S, r1 = lc[1] + ((c >> 1) & 1) * TL::S;
+        if (r0 >= TL::R || r1 >= TL::R) continue;
+        const float4* q = slots + int64_t(s_first[c]) * TL::REGION + (r0 * TL::R + r1);
+        for (int it = w; it < s_count[c]; it += 4) add4(g, q[int64_t(it) * TL::REGION]);
     }
-    uint32_t massive_nodes = 0;
-    auto add = [](float4& acc, const float4 v) {
-        acc.x += v.x;
-        acc.y += v.y;
-        acc.z += v.z;
-        acc.w += v.w;
-    };
-    if constexpr (D == 2) {
-        // With 1024 threads (a launch with few work items) quarter w of the workgroup computes
-        // partial sum w, which quarters the chain of slot loads a node waits on; with 256 threads
-        // each thread computes all four.  Both give the same sums.
-        static_assert(TL::NODES == 256, "one node per thread of a 2D node tile");
-        __shared__ float4 s_part[3][TL::NODES];
-        const int l = int(threadIdx.x) & (TL::NODES - 1);
-        const int n[2] = {nto[0] * TL::S + (l >> TL::LOG), nto[1] * TL::S + (l & (TL::S - 1))};
-        const bool split = blockDim.x == 4 * TL::NODES;
-        const int w = split ? int(threadIdx.x) >> 8 : 0;
-        float4 g0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), g1 = g0, g2 = g0, g3 = g0;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            if (first[c] < 0) continue;
-            const int r0 = n[0] - (nto[0] - (c & 1)) * TL::S, r1 = n[1] - (nto[1] - ((c >> 1) & 1)) * TL::S;
-            if (r0 >= TL::R || r1 >= TL::R) continue;
-            const float4* q = slots + int64_t(first[c]) * TL::REGION + (r0 * TL::R + r1);
-            if (split) {
-                for (int it = w; it < count[c]; it += 4) add(g0, q[int64_t(it) * TL::REGION]);
-            } else {
-                int it = 0;
-                for (; it + 4 <= count[c]; it += 4) {
-                    const float4 s0 = q[int64_t(it) * TL::REGION], s1 = q[int64_t(it + 1) * TL::REGION],
-                                 s2 = q[int64_t(it + 2) * TL::REGION], s3 = q[int64_t(it + 3) * TL::REGION];
-                    add(g0, s0);
-                    add(g1, s1);
-                    add(g2, s2);
-                    add(g3, s3);
-                }
-                if (it < count[c]) add(g0, q[int64_t(it) * TL::REGION]);
-                if (it + 1 < count[c]) add(g1, q[int64_t(it + 1) * TL::REGION]);
-                if (it + 2 < count[c]) add(g2, q[int64_t(it + 2) * TL::REGION]);
-            }
-        }
-        if (split) {
-            if (w > 0) s_part[w - 1][l] = g0;
-            __syncthreads();
-            if (w == 0) {
-                g1 = s_part[0][l];
-                g2 = s_part[1][l];
-                g3 = s_part[2][l];
-            }
-        }
-        if (w == 0) {
-            float4 g = g0;
-            add(g, g1);
-            add(g, g2);
-            add(g, g3);
-            massive_nodes += g.w > 0.0f ? 1u : 0u;
-            if (gpre) gpre[int64_t(nt_idx) * TL::NODES + l] = g;
-            gv[int64_t(nt_idx) * TL::NODES + l] = grid_node<D>(g, n, sp);
-        }
-    } else
-    for (int l = threadIdx.x; l < TL::NODES; l += blockDim.x) {
-        int n[D];
-        {
-            int rem = l;
-#pragma unroll
-            for (int a = D - 1; a >= 0; --a) {
-                n[a] = nto[a] * TL::S + (rem & (TL::S - 1));
-                rem >>= TL::LOG;
-            }
-        }
-        float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            if (first[c] < 0) continue;
-            bool inside = true;
-            int r = 0;
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                const int ra = n[a] - (nto[a] - ((c >> a) & 1)) * TL::S;
-                inside = inside && ra < TL::R;
-                r = r * TL::R + ra;
-            }
-            if (!inside) continue;
-            // items in order; four loads in flight before their (ordered) sums
-            const float4* q = slots + int64_t(first[c]) * TL::REGION + r;
-            int it = 0;
-            for (; it + 4 <= count[c]; it += 4, q += 4 * TL::REGION) {
-                const float4 s0 = q[0], s1 = q[TL::REGION], s2 = q[2 * TL::REGION], s3 = q[3 * TL::REGION];
-                add(g, s0);
-                add(g, s1);
-                add(g, s2);
-                add(g, s3);
-            }
-            for (; it < count[c]; ++it, q += TL::REGION) add(g, q[0]);
-        }
-        massive_nodes += g.w > 0.0f ? 1u : 0u;
-        if (gpre) gpre[int64_t(nt_idx) * TL::NODES + l] = g;
-        gv[int64_t(nt_idx) * TL::NODES + l] = grid_node<D>(g, n, sp);
-    }
-    // nodes with post-P2G mass > 0, per node tile (summed on demand by mpm_active_nodes)
-    if (massive_nodes) atomicAdd(&s_active, massive_nodes);
+    if (w > 0) s_part[w - 1][l] = g;
     __syncthreads();
-    if (threadIdx.x == 0) active[nt_idx] = s_active;
+    if (w == 0) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) add4(g, s_part[q][l]);
+        if (gpre) gpre[int64_t(nt_idx) * TL::NODES + l] = g;
+        gv[int64_t(nt_idx) * TL::NODES + l] = grid_node<2>(g, n, sp);
+    }
+    const int massive = __syncthreads_count(w == 0 && g.w > 0.0f);
+    if (threadIdx.x == 0) active[nt_idx] = uint32_t(massive);
+}
+
+// The node tiles the particles reach, after a radix sort (the incremental sort's scatter kernel lists
+// them itself).
+template <int D>
+__global__ __launch_bounds__(256) void k_list_grid_tiles(StepParams p, const uint32_t* __restrict__ item_offset,
+                                                         GridTile<D>* __restrict__ tiles, uint32_t* meta,
+                                                         uint32_t* __restrict__ active) {
+    list_grid_tile<D>(p, blockIdx.x * 256 + threadIdx.x, item_offset, tiles, &meta[kMetaGridTiles], active);
 }
 
 // Sum of v[first .. first+n) into *out (one workgroup).
@@ -642,6 +605,9 @@ static hipError_t sort_dispatch(const LaunchArgs& a) {
         k_items_rounds<<<rounds, 1024, 0, s>>>(a.tile_start, a.tile_end, p.ntiles, uint32_t(p.chunk), a.item_offset,
                                                p.items, a.rtot, a.meta);
     }
+    if (p.node_tiles > 0 && grid_tiles_listed(D, p))
+        k_list_grid_tiles<D><<<blocks_for(p.node_tiles, 256), 256, 0, s>>>(
+            p, a.item_offset, static_cast<GridTile<D>*>(a.grid_tiles), a.meta, a.active);
     return hipGetLastError();
 }
 
@@ -725,14 +691,16 @@ hipError_t launch_p2g(const LaunchArgs& a) { return a.dim == 2 ? p2g_dispatch<2>
 hipError_t launch_g2p(const LaunchArgs& a) { return a.dim == 2 ? g2p_dispatch<2>(a) : g2p_dispatch<3>(a); }
 
 hipError_t launch_grid(const LaunchArgs& a) {
-    const unsigned tiles = a.p.node_tiles;
-    if (tiles == 0) return hipSuccess;
-    if (a.dim == 2)  // few work items: four threads per node (the same sums)
-        k_grid_tiles<2><<<xcd_grid(tiles), a.p.n < int64_t(kFewItems) * a.p.chunk ? 1024 : 256, 0, a.stream>>>(
-            a.slots, a.item_offset, a.p, a.gv, a.gpre, a.stamps, a.active);
+    if (a.p.node_tiles == 0) return hipSuccess;
+    if (!grid_tiles_listed(a.dim, a.p))
+        k_grid_tiles_few<<<xcd_grid(a.p.node_tiles), 1024, 0, a.stream>>>(a.slots, a.item_offset, a.p, a.gv, a.gpre,
+                                                                         a.stamps, a.active);
+    else if (a.dim == 2)
+        k_grid_tiles<2><<<grid_tile_blocks(a.p.node_tiles), Tile<2>::NODES, 0, a.stream>>>(
+            a.slots, a.p, static_cast<const GridTile<2>*>(a.grid_tiles), a.meta, a.gv, a.gpre, a.stamps, a.active);
     else
-        k_grid_tiles<3><<<xcd_grid(tiles), 256, 0, a.stream>>>(a.slots, a.item_offset, a.p, a.gv, a.gpre, a.stamps,
-                                                                a.active);
+        k_grid_tiles<3><<<grid_tile_blocks(a.p.node_tiles), Tile<3>::NODES, 0, a.stream>>>(
+            a.slots, a.p, static_cast<const GridTile<3>*>(a.grid_tiles), a.meta, a.gv, a.gpre, a.stamps, a.active);
     return hipGetLastError();
 }
 
@@ -790,6 +758,7 @@ int64_t max_items(int64_t n, uint32_t ntiles) { return (n + kMinChunk - 1) / kMi
 int num_fields(int dim) { return dim == 2 ? Layout<2>::NF : Layout<3>::NF; }
 int region_nodes(int dim) { return dim == 2 ? Tile<2>::REGION : Tile<3>::REGION; }
 int tile_nodes(int dim) { return dim == 2 ? Tile<2>::NODES : Tile<3>::NODES; }
+size_t grid_tile_bytes(int dim) { return dim == 2 ? sizeof(GridTile<2>) : sizeof(GridTile<3>); }
 int tile_log(int dim) { return dim == 2 ? Tile<2>::LOG : Tile<3>::LOG; }
 
 }  // namespace nclr_host

@@ -4,6 +4,9 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
+import oracle as O
+from parity import assert_parity
+
 from nuclearmpm_amd import MaterialModel, MPMBatch, MPMSimulation, Particles
 from nuclearmpm_amd.sim import SceneSpec
 
@@ -34,3 +37,34 @@ def test_3d_p2g_one_particle_per_thread_is_bitwise_the_same(material, svd):
         ref = sim.particles()
     for k in ("x", "v", "F", "C", "Jp"):
         assert np.array_equal(getattr(got, k), getattr(ref, k)), k
+
+
+@pytest.mark.parametrize("dim,n,res,lo,hi,chunk", [
+    (2, 70000, 128, 0.40, 0.50, 256),   # lists of a node tile longer than one round of 64 slots, four partial sums
+    (3, 40000, 64, 0.40, 0.55, 256),    # the same in 3D, candidates on both sides of the tiles' faces
+    (3, 12000, 200, 0.05, 0.95, 256),   # more node tiles in use than workgroups: each takes several
+    (3, 513, 37, 0.10, 0.80, 512),      # a grid that does not fill its last node tiles
+])
+def test_grid_update_over_listed_node_tiles(dim, n, res, lo, hi, chunk):
+    """One step against the oracle, particles and grid (the step's own bound), after a radix sort and
+    after an incremental one."""
+    rng = np.random.default_rng(n)
+    p = Particles.from_positions((lo + (hi - lo) * rng.random((n, dim))).astype(np.float32), identity_mode=1)
+    p.v = rng.normal(0, 1.0, p.v.shape).astype(np.float32)
+    p.C = rng.normal(0, 2.0, p.C.shape).astype(np.float32)
+    p.F = (p.F + rng.normal(0, 0.005, p.F.shape)).astype(np.float32)
+    kw = dict(res=res, E=1e3, identity_mode=1)
+    with MPMSimulation(p, MaterialModel.kJelly, res, E=1e3, identity_mode=1, p2g_chunk=chunk) as sim:
+        before = p
+        for kind in ("radix", "incremental"):
+            sim.advance(1)
+            got = sim.particles().copy()
+            vel, mass = sim.grid()
+            st = O.State(x=before.x, v=before.v, F=before.F, C=before.C, Jp=before.Jp, mass=before.mass,
+                         volume=before.volume)
+            assert_parity(got, O.run(st, O.JELLY, steps=1, **kw), inv_dx=float(res), label=f"{kind} sort")
+            ref = O.p2g(st, O.JELLY, res=res, E=1e3)
+            ref_vel, ref_mass = O.grid_op(ref[0], ref[1], dim, res)
+            assert np.abs(mass.ravel() - ref_mass).max() <= 1e-5 * ref_mass.max()
+            assert sim.active_nodes() == int((ref[1] > 0).sum())
+            before = got
