@@ -35,13 +35,6 @@
 
 namespace nclr_dev {
 
-// d w_k / d fx of the quadratic B-spline weights (src/nclr.h:124-127)
-NCLR_DI void bspline_dweights(float fx, float (&dw)[3]) {
-    dw[0] = fx - 1.5f;
-    dw[1] = -2.0f * (fx - 1.0f);
-    dw[2] = fx - 0.5f;
-}
-
 // d det(A) / dA
 NCLR_DI M<2> cofactor(const M<2>& a) {
     M<2> c;
@@ -246,6 +239,110 @@ NCLR_DI void material_backward(int material, const M<D>& Fh, float Jp, const M<D
 
 NCLR_DI float ldg(const float* __restrict__ g, int64_t gstride, int c, int64_t j) { return g[int64_t(c) * gstride + j]; }
 
+// The stencil sums both particle adjoints take, over the 3^D nodes i of a particle with weights W_i and
+// values g_i, in cell units around the middle node: u = off - 1, phi = fx - 1, and at every node the
+// bracket b_i = k + B u (a polynomial in the node's offset, as the scattered and gathered affine velocities
+// are):
+//   m0_r = sum W_i g_ir      T_rc = sum W_i g_ir u_c      fxb_a = sum S_i dW_i / dfx_a
+// with S_i = g_i . b_i (MASS: + cm g_i.w).  The weights are products over the axes, so the sums are nested
+// per axis: about 20 multiply-adds a node where the sums node by node took 55 (3D).  emit(o, W_i, b_i)
+// is called at every node.  These derivatives have no bitwise counterpart: fused multiply-adds, and
+// the error against 64 bits is that of the sums node by node (gradients within 6e-7 of theirs).
+// 3D: one plane of nine nodes' loads in flight (27 spill).  Both kernels are bound by VALU issue:
+// 8 x 262,144 jelly particles, G2P adjoint 259 -> 189 us, P2G adjoint 342 -> 258 (60,007 snow
+// particles 36.6 -> 33.2 and 27.4 -> 19.0).
+template <int D, bool MASS, typename Node, typename Emit>
+NCLR_DI void adjoint_stencil(const float (&fx)[D], const M<D>& B, const float (&k)[D], float cm, const Node& node,
+                             Emit emit, float (&m0)[D], M<D>& T, float (&fxb)[D]) {
+    constexpr int L = D - 1;  // the innermost axis
+    // the weights' derivatives are f, -2 f - 1 and f + 1 with f = fx - 1.5: their sum against S_0, S_1, S_2
+    // is f ((S_0 - S_1) + (S_2 - S_1)) + (S_2 - S_1)
+    float w[D][3], lo = 0.0f, hi = 0.0f;  // axis 0: S_0 - S_1 and S_2 - S_1 over the planes
+#pragma unroll
+    for (int a = 0; a < D; ++a) {
+        bspline_weights(fx[a], w[a]);
+        m0[a] = 0.0f;
+        fxb[a] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < D; ++c) T.a[a][c] = 0.0f;
+    }
+    auto dsum = [](float f, float s0, float s1, float s2) { return fmaf(f - 1.5f, (s0 - s1) + (s2 - s1), s2 - s1); };
+    // one row of three nodes along the innermost axis: r0 = sum w g, r2 = sum w u g, rs = sum w S,
+    // rd = sum dw S
+    auto row = [&](int o0, int o1, const float (&b)[D], float wo, float (&r0)[D], float (&r2)[D], float& rs, float& rd) {
+        float So[3];
+#pragma unroll
+        for (int o = 0; o < 3; ++o) {
+            int off[D];
+            off[0] = o0;
+            if constexpr (D == 3) off[1] = o1;
+            off[L] = o;
+            const float4 g = node(off);
+            const float gr[3] = {g.x, g.y, g.z};
+            float bi[D];
+            float S = MASS ? g.w * cm : 0.0f;
+#pragma unroll
+            for (int r = 0; r < D; ++r) {
+                bi[r] = o == 1 ? b[r] : (o == 0 ? b[r] - B.a[r][L] : b[r] + B.a[r][L]);
+                S = !MASS && r == 0 ? gr[r] * bi[r] : fmaf(gr[r], bi[r], S);
+                const float p = w[L][o] * gr[r];
+                r0[r] = o == 0 ? p : r0[r] + p;
+                if (o == 0) r2[r] = -p;
+                if (o == 2) r2[r] = r2[r] + p;
+            }
+            rs = o == 0 ? w[L][o] * S : fmaf(w[L][o], S, rs);
+            So[o] = S;
+            emit(off, wo * w[L][o], bi);
+        }
+        rd = dsum(fx[L], So[0], So[1], So[2]);
+    };
+#pragma unroll(D == 3 ? 1 : 3)
+    for (int o0 = 0; o0 < 3; ++o0) {
+        const float w0 = pick3(w[0], o0);
+        float b0[D], q0[D], q2[D], qs, qd;
+#pragma unroll
+        for (int r = 0; r < D; ++r) b0[r] = o0 == 1 ? k[r] : (o0 == 0 ? k[r] - B.a[r][0] : k[r] + B.a[r][0]);
+        if constexpr (D == 2) {
+            row(o0, 0, b0, w0, q0, q2, qs, qd);
+        } else {
+            float q1[3], ro[3];
+#pragma unroll
+            for (int o1 = 0; o1 < 3; ++o1) {
+                float b1[3], r0[3], r2[3], rs, rd;
+#pragma unroll
+                for (int r = 0; r < 3; ++r)
+                    b1[r] = o1 == 1 ? b0[r] : (o1 == 0 ? b0[r] - B.a[r][1] : b0[r] + B.a[r][1]);
+                row(o0, o1, b1, w0 * w[1][o1], r0, r2, rs, rd);
+                ro[o1] = rs;
+                const float w1 = w[1][o1];
+#pragma unroll
+                for (int r = 0; r < 3; ++r) {
+                    q0[r] = o1 == 0 ? w1 * r0[r] : fmaf(w1, r0[r], q0[r]);
+                    if (o1 == 0) q1[r] = -q0[r];
+                    if (o1 == 2) q1[r] = fmaf(w1, r0[r], q1[r]);
+                    q2[r] = o1 == 0 ? w1 * r2[r] : fmaf(w1, r2[r], q2[r]);
+                }
+                qs = o1 == 0 ? w1 * rs : fmaf(w1, rs, qs);
+                qd = o1 == 0 ? w1 * rd : fmaf(w1, rd, qd);
+            }
+#pragma unroll
+            for (int r = 0; r < 3; ++r) T.a[r][1] = fmaf(w0, q1[r], T.a[r][1]);
+            fxb[1] = fmaf(w0, dsum(fx[1], ro[0], ro[1], ro[2]), fxb[1]);
+        }
+#pragma unroll
+        for (int r = 0; r < D; ++r) {
+            const float wq = w0 * q0[r];
+            m0[r] = m0[r] + wq;
+            T.a[r][0] = T.a[r][0] + (o0 == 1 ? 0.0f : (o0 == 0 ? -wq : wq));
+            T.a[r][L] = fmaf(w0, q2[r], T.a[r][L]);
+        }
+        lo += o0 == 0 ? qs : (o0 == 1 ? -qs : 0.0f);
+        hi += o0 == 2 ? qs : (o0 == 1 ? -qs : 0.0f);
+        fxb[L] = fmaf(w0, qd, fxb[L]);
+    }
+    fxb[0] = fmaf(fx[0] - 1.5f, lo + hi, hi);
+}
+
 // ---------------------------------------------------------------------------------------------
 // G2P adjoint (src/nclr.h:167-258).  GENERAL: any material (the scene's, at run time); otherwise
 // every scene is jelly.  A work item of TPB * PPT particles, PPT per thread.  At least two waves per
@@ -283,7 +380,7 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(D == 3 && P
 
     // pass 1: cotangents of the gathered velocity (vb = v' + dt x') and affine matrix
     // (Cb = C' + dt F' F^T) and a bound of the scattered sums per channel
-    bool valid[PPT];
+    bool valid[PPT], finite[PPT];
     int bases[PPT][D];
     float fxs[PPT][D], vb[PPT][D];
     M<D> Cb[PPT];
@@ -390,6 +487,7 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(D == 3 && P
             for (int b = 0; b < D; ++b) s += fabsf(Cb[k].a[a][b]);
             // |off - fx| <= 1.5 on every axis
             const float bc = wsum * (fabsf(vb[k][a]) + 1.5f * four_inv_dx * s);
+            finite[k] = (a == 0 || finite[k]) && bc < 3.0e38f;
             if (bc < 3.0e38f) bound[a] = fmaxf(bound[a], bc);
         }
     }
@@ -420,75 +518,58 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(D == 3 && P
     for (int k = 0; k < PPT; ++k) {
         if (!valid[k]) continue;
         const uint32_t j = j0 + uint32_t(k) * TPB + threadIdx.x;
-        float w[D][3], dw[D][3];
         int rb = 0;
+        M<D> Bm, Tm;
+        float kb[D], m0[D], fxbar[D];
 #pragma unroll
         for (int a = 0; a < D; ++a) {
-            bspline_weights(fxs[k][a], w[a]);
-            bspline_dweights(fxs[k][a], dw[a]);
             rb = rb * TL::R + (bases[k][a] - torg[a]);
-        }
-        M<D> Cn;
-        float fxbar[D];
-#pragma unroll
-        for (int a = 0; a < D; ++a) {
-            fxbar[a] = 0.0f;
-#pragma unroll
-            for (int b = 0; b < D; ++b) Cn.a[a][b] = 0.0f;
-        }
-        const StencilRows<D> node(gv, bases[k], sp.ntn, sp.node_tile_base);
-        // 3D: unrolled by rows of three nodes (fully unrolled, the early node loads spill)
-#pragma unroll(D == 3 ? 3 : K)
-        for (int o = 0; o < K; ++o) {
-            // products and sums contract to fused multiply-adds here (the kernel is bound by its
-            // VALU issue; these derivatives have no bitwise counterpart to match)
-#pragma clang fp contract(fast)
-            int off[D];
-            offsets<D>(o, off);
-            float d[D];
-            int ro = 0;
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                d[a] = float(off[a]) - fxs[k][a];
-                ro = ro * TL::R + off[a];
-            }
-            const float4 g = node(off);
-            const float gvel[3] = {g.x, g.y, g.z};
-            float weight = pick3(w[0], off[0]);
-#pragma unroll
-            for (int a = 1; a < D; ++a) weight *= pick3(w[a], off[a]);
-            float wbar = 0.0f;
-            const int r = rb + ro;
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                float cd = 0.0f;
-#pragma unroll
-                for (int b = 0; b < D; ++b) {
-                    cd += Cb[k].a[a][b] * d[b];
-                    Cn.a[a][b] += four_inv_dx * weight * gvel[a] * d[b];
-                }
-                const float val = weight * (vb[k][a] + four_inv_dx * cd);
-                wbar += gvel[a] * (vb[k][a] + four_inv_dx * cd);
-                const float y = val * scale[a];
-                if (fabsf(y) < kFixedLimit) atomicAdd(&acc[a * REG + r], fixed_point(y));
-                else atomicOr(&nonfinite[r], 1u << a);
-            }
+            kb[a] = vb[k][a];
 #pragma unroll
             for (int b = 0; b < D; ++b) {
-                float ctv = 0.0f;
-#pragma unroll
-                for (int a = 0; a < D; ++a) ctv += Cb[k].a[a][b] * gvel[a];
-                fxbar[b] -= four_inv_dx * weight * ctv;
-            }
-#pragma unroll
-            for (int a = 0; a < D; ++a) {
-                float dwa = pick3(dw[a], off[a]);
-#pragma unroll
-                for (int b = 0; b < D; ++b)
-                    if (b != a) dwa *= pick3(w[b], off[b]);
-                fxbar[a] += wbar * dwa;
+                Bm.a[a][b] = four_inv_dx * Cb[k].a[a][b];
+                kb[a] = fmaf(-Bm.a[a][b], fxs[k][b] - 1.0f, kb[a]);
             }
         }
+        const StencilRows<D> node(gv, bases[k], sp.ntn, sp.node_tile_base);
+        // a particle whose bound is finite has every |contribution * scale| below 2^50 (up to the
+        // rounding of the bracket, and the conversion holds to 2^51)
+        if (finite[k]) {
+            adjoint_stencil<D, false>(
+                fxs[k], Bm, kb, 0.0f, node,
+                [&](const int (&off)[D], float weight, const float (&bi)[D]) {
+                    int r = 0;
+#pragma unroll
+                    for (int a = 0; a < D; ++a) r = r * TL::R + off[a];
+#pragma unroll
+                    for (int a = 0; a < D; ++a)
+                        atomicAdd(&acc[a * REG + rb + r], fixed_point(weight * bi[a], double(scale[a])));
+                },
+                m0, Tm, fxbar);
+        } else {
+            adjoint_stencil<D, false>(
+                fxs[k], Bm, kb, 0.0f, node,
+                [&](const int (&off)[D], float weight, const float (&bi)[D]) {
+                    int r = 0;
+#pragma unroll
+                    for (int a = 0; a < D; ++a) r = r * TL::R + off[a];
+#pragma unroll
+                    for (int a = 0; a < D; ++a) {
+                        const float y = weight * bi[a] * scale[a];
+                        if (fabsf(y) < kFixedLimit) atomicAdd(&acc[a * REG + rb + r], fixed_point(y));
+                        else atomicOr(&nonfinite[rb + r], 1u << a);
+                    }
+                },
+                m0, Tm, fxbar);
+        }
+        M<D> Cn;
+#pragma unroll
+        for (int b = 0; b < D; ++b)
+#pragma unroll
+            for (int a = 0; a < D; ++a) {
+                fxbar[b] = fmaf(-Bm.a[a][b], m0[a], fxbar[b]);
+                Cn.a[a][b] = four_inv_dx * fmaf(-m0[a], fxs[k][b] - 1.0f, Tm.a[a][b]);
+            }
         const int64_t i = perm[j];
 #pragma unroll
         for (int a = 0; a < D; ++a)
@@ -649,7 +730,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
                                                      float* __restrict__ gin, int64_t gstride,
                                                      float* __restrict__ epart) {
     using L = Layout<D>;
-    constexpr int K = D == 2 ? 9 : 27;
     const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (j >= p.n) return;
     const int64_t i = perm[j];
@@ -680,9 +760,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         epart[j] = 0.0f;
         return;
     }
-    float dw[D][3];
-#pragma unroll
-    for (int a = 0; a < D; ++a) bspline_dweights(fx[a], dw[a]);
     // the forward's affine matrix from one polar factor: in the accurate mode its F - R is kept,
     // and the stress backward below takes R = F - (F - R) (within one float rounding of the
     // iteration's R) instead of a second Newton iteration; in the other modes R itself is kept and
@@ -698,57 +775,28 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             for (int b = 0; b < D; ++b) FmR.a[a][b] = F.a[a][b] - R.a[a][b];
     }
     A = fused_affine_from<D>(sp.material, F, FmR, C, Jp, mass, vol, sp);
-    M<D> Abar;
-    float fxbar[D], vin[D];
+    // the bracket m v + A dpos of P2G's contributions in cell units around the middle node
+    M<D> Bm, Abar;
+    float kb[D], m0[D], fxbar[D];
 #pragma unroll
-    for (int a = 0; a < D; ++a) {
-        fxbar[a] = 0.0f;
-        vin[a] = 0.0f;
-#pragma unroll
-        for (int b = 0; b < D; ++b) Abar.a[a][b] = 0.0f;
-    }
-    const StencilRows<D> node(gbar, base, sp.ntn, sp.node_tile_base);
-    // 3D: unrolled by rows of three nodes (fully unrolled, the early node loads spill)
-#pragma unroll(D == 3 ? 3 : K)
-    for (int o = 0; o < K; ++o) {
-        // fused multiply-adds here, as in the G2P adjoint's stencil loop
-#pragma clang fp contract(fast)
-        int off[D];
-        offsets<D>(o, off);
-        float dpos[D];
-#pragma unroll
-        for (int a = 0; a < D; ++a) dpos[a] = (float(off[a]) - fx[a]) * sp.dx;
-        const float4 g = node(off);
-        const float gm[3] = {g.x, g.y, g.z};
-        float weight = pick3(w[0], off[0]);
-#pragma unroll
-        for (int a = 1; a < D; ++a) weight *= pick3(w[a], off[a]);
-        float wbar = g.w * mass;
-#pragma unroll
-        for (int r = 0; r < D; ++r) {
-            float ad = 0.0f;
-#pragma unroll
-            for (int c = 0; c < D; ++c) {
-                ad += A.a[r][c] * dpos[c];
-                Abar.a[r][c] += weight * gm[r] * dpos[c];
-            }
-            wbar += gm[r] * (mass * v[r] + ad);
-            vin[r] += weight * mass * gm[r];
-        }
+    for (int r = 0; r < D; ++r) {
+        kb[r] = mass * v[r];
 #pragma unroll
         for (int c = 0; c < D; ++c) {
-            float atm = 0.0f;
-#pragma unroll
-            for (int r = 0; r < D; ++r) atm += A.a[r][c] * gm[r];
-            fxbar[c] -= sp.dx * weight * atm;
+            Bm.a[r][c] = A.a[r][c] * sp.dx;
+            kb[r] = fmaf(-Bm.a[r][c], fx[c] - 1.0f, kb[r]);
         }
+    }
+    const StencilRows<D> node(gbar, base, sp.ntn, sp.node_tile_base);
+    adjoint_stencil<D, true>(fx, Bm, kb, mass, node, [](const int (&)[D], float, const float (&)[D]) {}, m0, Abar, fxbar);
+    float vin[D];
 #pragma unroll
-        for (int a = 0; a < D; ++a) {
-            float dwa = pick3(dw[a], off[a]);
+    for (int r = 0; r < D; ++r) {
+        vin[r] = mass * m0[r];
 #pragma unroll
-            for (int b = 0; b < D; ++b)
-                if (b != a) dwa *= pick3(w[b], off[b]);
-            fxbar[a] += wbar * dwa;
+        for (int c = 0; c < D; ++c) {
+            fxbar[c] = fmaf(-Bm.a[r][c], m0[r], fxbar[c]);
+            Abar.a[r][c] = sp.dx * fmaf(-m0[r], fx[c] - 1.0f, Abar.a[r][c]);
         }
     }
     // A = -(dt V0) Dinv PF + m C  ->  G = dL/dPF

@@ -585,6 +585,14 @@ NCLR_DI unsigned long long fixed_point(float y) {
     return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
 
+// y * scale likewise, scale a power of two (y * scale exact): one fused multiply-add.
+NCLR_DI unsigned long long fixed_point(float y, double scale) {
+    const double t = fma(double(y), scale, 6755399441055744.0);
+    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(t));
+    const uint32_t lo = uint32_t(b), hi = uint32_t(b >> 32) - 0x43380000u;
+    return (static_cast<unsigned long long>(hi) << 32) | lo;
+}
+
 NCLR_DI float fixed_point_value(unsigned long long q, double inv_scale) {
     return float(double((long long)q) * inv_scale);
 }

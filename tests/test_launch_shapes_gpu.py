@@ -68,3 +68,33 @@ def test_grid_update_over_listed_node_tiles(dim, n, res, lo, hi, chunk):
             assert np.abs(mass.ravel() - ref_mass).max() <= 1e-5 * ref_mass.max()
             assert sim.active_nodes() == int((ref[1] > 0).sum())
             before = got
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 1e37])
+def test_a_cotangent_out_of_range_stays_with_its_neighbours(dim, bad):
+    """The G2P adjoint deposits a particle whose bound is not finite with a check per contribution: its
+    nodes' cotangents are lost (NaN), those of a far cluster are bit for bit what they are without it."""
+    import torch
+
+    from nuclearmpm_amd import autodiff
+
+    rng = np.random.default_rng(dim)
+    n = 300
+    x = np.concatenate([0.2 + 0.1 * rng.random((n, dim)), 0.6 + 0.1 * rng.random((n, dim))]).astype(np.float32)
+    p = Particles.from_positions(x, identity_mode=1)
+    p.F = (p.F + rng.normal(0, 0.01, p.F.shape)).astype(np.float32)
+    cot = torch.from_numpy(rng.normal(size=(autodiff.channels(dim), 2 * n)).astype(np.float32)).cuda()
+    grads = []
+    with MPMSimulation(p, MaterialModel.kJelly, 64, identity_mode=1) as sim:
+        for value in (None, bad):
+            c = cot.clone()
+            if value is not None:
+                c[2 * dim + dim * dim, 7] = value  # C_00 of particle 7
+            s0 = sim.state_image().requires_grad_(True)
+            out = autodiff.rollout(sim, s0, torch.tensor([1e4]), steps=1, checkpoint_every=1)
+            grads.append(torch.autograd.grad(out, s0, c)[0].cpu().numpy())
+    far = slice(n, 2 * n)
+    assert np.isfinite(grads[0]).all()
+    assert np.array_equal(grads[0][:, far], grads[1][:, far])
+    assert np.isnan(grads[1][:, 7]).any()
