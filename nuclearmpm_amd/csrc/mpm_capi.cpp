@@ -1514,8 +1514,9 @@ int mpm_sort_keys(const uint32_t* keys, int64_t n, int bits, uint32_t* perm, int
     if (e == hipSuccess) e = dmalloc(&tk, size_t(n));
     if (e == hipSuccess) e = dmalloc(&tv, size_t(n));
     if (e == hipSuccess) e = dmalloc(&hist, size_t(256) * size_t(nclr_host::sort_tiles(n)) + 256);
-    if (e == hipSuccess) e = hipMemcpyAsync(dk, keys, size_t(n) * 4, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = nclr_host::radix_sort_pairs(dk, dv, tk, tv, hist, n, bits, true, s);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(nclr_host::radix_keys_in(dk, tk, bits), keys, size_t(n) * 4, hipMemcpyHostToDevice, s);
+    if (e == hipSuccess) e = nclr_host::radix_sort_pairs(dk, dv, tk, tv, hist, n, bits, s);
     if (e == hipSuccess) e = hipMemcpyAsync(perm, dv, size_t(n) * 4, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     void* bufs[] = {dk, dv, tk, tv, hist};

@@ -966,11 +966,12 @@ hipError_t launch_compact_order(int dim, const float* st, const uint32_t* pid, f
     while ((1 << bpa) < sp.res + 1 && bpa < 16) ++bpa;
     bpa = dim == 3 ? (bpa < 10 ? bpa : 10) : bpa;  // at most 32 key bits
     const unsigned b = unsigned((n + 255) / 256);
-    if (dim == 2) k_cell_keys<2><<<b, 256, 0, s>>>(st, stride, n, sp.inv_dx, bpa, keys);
-    else k_cell_keys<3><<<b, 256, 0, s>>>(st, stride, n, sp.inv_dx, bpa, keys);
+    uint32_t* in = radix_keys_in(keys, keys_tmp, dim * bpa);
+    if (dim == 2) k_cell_keys<2><<<b, 256, 0, s>>>(st, stride, n, sp.inv_dx, bpa, in);
+    else k_cell_keys<3><<<b, 256, 0, s>>>(st, stride, n, sp.inv_dx, bpa, in);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    e = radix_sort_pairs(keys, perm, keys_tmp, perm_tmp, hist, n, dim * bpa, true, s);
+    e = radix_sort_pairs(keys, perm, keys_tmp, perm_tmp, hist, n, dim * bpa, s);
     if (e != hipSuccess) return e;
     k_gather_state<<<b, 256, 0, s>>>(st, pid, perm, st_out, pid_out, fields, stride, n);
     return hipGetLastError();

@@ -220,8 +220,11 @@ hipError_t launch_iota_u32(uint32_t* p, int64_t n, hipStream_t s);
 hipError_t launch_bump_u32(uint32_t* p, hipStream_t s);  // *p += 1 on the device
 hipError_t launch_zero_f4(float4* p, int64_t n, hipStream_t s);
 hipError_t launch_active_sum(const LaunchArgs& a, uint32_t first_tile, uint32_t tiles, unsigned long long* out);
+// Stable sort by the low `bits` bits of n keys that lie in radix_keys_in(keys, keys_tmp, bits) (the pass
+// count's parity decides, so that no copy is needed): sorted keys in `keys`, input positions in `vals`.
+uint32_t* radix_keys_in(uint32_t* keys, uint32_t* keys_tmp, int bits);
 hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t* keys_tmp, uint32_t* vals_tmp, uint32_t* hist,
-                            int64_t n, int bits, bool identity_values, hipStream_t s);
+                            int64_t n, int bits, hipStream_t s);
 int64_t sort_tiles(int64_t n);
 // scene generators and the viewer projection (mpm_scene.hip)
 void rand_jump(uint32_t state[4], uint64_t k);

@@ -13,7 +13,8 @@
 namespace {
 
 constexpr int64_t kNoAllocMaxKeys = int64_t(1) << 20;
-// keys copy, keys_tmp, vals_tmp (kNoAllocMaxKeys each) + the histogram of the largest sort
+// keys copy, keys_tmp, vals_tmp (kNoAllocMaxKeys each) + the histogram: at most 256 tiles, of 4096
+// keys or, up to 2^18 keys, of 1024
 constexpr int64_t kHistWords = 256 * ((kNoAllocMaxKeys + 4095) / 4096) + 256;
 constexpr int64_t kScratchWords = 3 * kNoAllocMaxKeys + kHistWords;
 
@@ -62,8 +63,9 @@ extern "C" int mpm_sort_keys_noalloc(const uint32_t* keys, int64_t n, int bits, 
     uint32_t* hist = base + 3 * kNoAllocMaxKeys;
     // every histogram entry and digit total is written by its pass before it is read: nothing
     // carried over from an earlier call is used
-    e = hipMemcpyAsync(kcopy, keys, size_t(n) * sizeof(uint32_t), hipMemcpyDeviceToDevice, s);
-    if (e == hipSuccess) e = nclr_host::radix_sort_pairs(kcopy, perm, ktmp, vtmp, hist, n, bits, true, s);
+    e = hipMemcpyAsync(nclr_host::radix_keys_in(kcopy, ktmp, bits), keys, size_t(n) * sizeof(uint32_t),
+                       hipMemcpyDeviceToDevice, s);
+    if (e == hipSuccess) e = nclr_host::radix_sort_pairs(kcopy, perm, ktmp, vtmp, hist, n, bits, s);
     if (e != hipSuccess)
         return nclr_host::set_last_error(MPM_ERR_HIP, (std::string("mpm_sort_keys_noalloc: ") + hipGetErrorString(e)).c_str());
     return MPM_OK;

@@ -588,11 +588,11 @@ static hipError_t sort_dispatch(const LaunchArgs& a) {
     const auto& p = a.p;
     const int64_t nb = int64_t(p.ntiles) + 1;
     hipStream_t s = a.stream;
+    const int bits = key_bits(p.ntiles);
     k_keys<D><<<blocks_for(std::max<int64_t>(std::max<int64_t>(p.n, nb), 1), 256), 256, 0, s>>>(
-        a.state_in, a.pid_in, p, a.stamp, a.keys, a.status, a.tile_start, a.tile_end);
+        a.state_in, a.pid_in, p, a.stamp, radix_keys_in(a.keys, a.keys_tmp, bits), a.status, a.tile_start, a.tile_end);
     if (p.n > 0) {
-        hipError_t e = radix_sort_pairs(a.keys, a.perm, a.keys_tmp, a.perm_tmp, a.hist, p.n, key_bits(p.ntiles),
-                                        true, s);
+        hipError_t e = radix_sort_pairs(a.keys, a.perm, a.keys_tmp, a.perm_tmp, a.hist, p.n, bits, s);
         if (e != hipSuccess) return e;
         k_tile_bounds<<<blocks_for(p.n, 256), 256, 0, s>>>(a.keys, p.n, a.tile_start, a.tile_end);
     }

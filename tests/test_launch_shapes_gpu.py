@@ -98,3 +98,18 @@ def test_a_cotangent_out_of_range_stays_with_its_neighbours(dim, bad):
     assert np.isfinite(grads[0]).all()
     assert np.array_equal(grads[0][:, far], grads[1][:, far])
     assert np.isnan(grads[1][:, 7]).any()
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 1024, 1025, 4097, 65536, 65537, 262144, 262145, 300001])
+@pytest.mark.parametrize("bits", [0, 1, 7, 8, 9, 20, 32])
+def test_radix_sort_at_the_edges_of_its_tiles(n, bits):
+    """1024-key tiles up to 2^18 keys, 4096 above; digit offsets summed in the scatter up to 64 tiles;
+    odd and even pass counts (the input buffer alternates)."""
+    from nuclearmpm_amd._lib import sort_keys
+
+    rng = np.random.default_rng(n + bits)
+    for keys in (rng.integers(0, 1 << 32, n, dtype=np.uint32),                   # random order
+                 np.sort(rng.integers(0, 1 << min(bits, 10), n).astype(np.uint32)),  # sorted, many equal
+                 np.full(n, 0xA5A5A5A5, np.uint32)):                              # all equal
+        low = keys if bits == 32 else keys & np.uint32((1 << bits) - 1)
+        assert np.array_equal(sort_keys(keys, bits), np.argsort(low, kind="stable").astype(np.uint32))
