@@ -262,10 +262,12 @@ int mpm_backward_segment(mpm_handle h, int nsteps, const float* grad_out, float*
 /* Device bytes of the tape mpm_backward_segment keeps for segments of `nsteps` steps (-1 for a
  * NULL handle or nsteps < 1): nsteps - 1 entries of one state snapshot (mpm_state_bytes) and one
  * sort (8 bytes per particle, 12 bytes per particle tile of every scene for its bounds and work
- * item offset, 16 bytes per possible work item, 256-byte aligned), and nsteps entries of the
- * forward grid and its pre-update {momentum, mass} (32 bytes per node of every scene's node tiles;
- * kept only while it leaves a quarter of the free device memory, else each adjoint step
- * recomputes its grid). */
+ * item offset, 16 bytes per possible work item, 40 / 72 bytes (2D / 3D) per node tile, 256-byte
+ * aligned), and nsteps entries of the
+ * forward grid and its pre-update {momentum, mass} (32 bytes per node of every scene's node tiles)
+ * with, in 3D, nsteps - 1 entries of the particles' polar factors (36 bytes per particle); kept
+ * only while they leave a quarter of the free device memory, else each adjoint step recomputes
+ * them. */
 int64_t mpm_tape_bytes(mpm_handle h, int nsteps);
 
 /* Recorded segments: no counterpart in the reference (whose checkpointing recomputes every
@@ -273,7 +275,7 @@ int64_t mpm_tape_bytes(mpm_handle h, int nsteps);
  *
  * mpm_record_bytes: device bytes of the tape of one recorded segment of `nsteps` steps (-1 for a
  * NULL handle or nsteps < 1): nsteps - 1 state snapshots and sorts as in mpm_tape_bytes, and with
- * with_grid != 0 nsteps forward grids and pre-update sums.
+ * with_grid != 0 nsteps forward grids and pre-update sums (and the 3D polar factors).
  *
  * mpm_advance_recorded: advances `nsteps` steps from the current state like mpm_advance (on the
  * tiled step) and records into `tape` (caller-owned device memory of mpm_record_bytes bytes,

@@ -248,10 +248,11 @@ NCLR_DI float ldg(const float* __restrict__ g, int64_t gstride, int c, int64_t j
 // per axis: about 20 multiply-adds a node where the sums node by node took 55 (3D).  emit(o, W_i, b_i)
 // is called at every node.  These derivatives have no bitwise counterpart: fused multiply-adds, and
 // the error against 64 bits is that of the sums node by node (gradients within 6e-7 of theirs).
-// 3D: one plane of nine nodes' loads in flight (27 spill).  Both kernels are bound by VALU issue:
-// 8 x 262,144 jelly particles, G2P adjoint 259 -> 189 us, P2G adjoint 342 -> 258 (60,007 snow
-// particles 36.6 -> 33.2 and 27.4 -> 19.0).
-template <int D, bool MASS, typename Node, typename Emit>
+// 3D: one plane of nine nodes' loads in flight (27 spill).  FMA_PLANE: the bracket moves to a plane by a
+// multiply-add instead of selects; the form that leaves the caller's kernel without spills.  Both kernels are bound by VALU issue:
+// 8 x 262,144 jelly particles, G2P adjoint 259 -> 187 us, P2G adjoint 342 -> 258 (60,007 snow
+// particles 36.6 -> 29.6 and 27.4 -> 19.0).
+template <int D, bool MASS, bool FMA_PLANE, typename Node, typename Emit>
 NCLR_DI void adjoint_stencil(const float (&fx)[D], const M<D>& B, const float (&k)[D], float cm, const Node& node,
                              Emit emit, float (&m0)[D], M<D>& T, float (&fxb)[D]) {
     constexpr int L = D - 1;  // the innermost axis
@@ -301,7 +302,8 @@ NCLR_DI void adjoint_stencil(const float (&fx)[D], const M<D>& B, const float (&
         const float w0 = pick3(w[0], o0);
         float b0[D], q0[D], q2[D], qs, qd;
 #pragma unroll
-        for (int r = 0; r < D; ++r) b0[r] = o0 == 1 ? k[r] : (o0 == 0 ? k[r] - B.a[r][0] : k[r] + B.a[r][0]);
+        for (int r = 0; r < D; ++r) b0[r] = FMA_PLANE ? fmaf(B.a[r][0], float(o0 - 1), k[r])
+                              : (o0 == 1 ? k[r] : (o0 == 0 ? k[r] - B.a[r][0] : k[r] + B.a[r][0]));
         if constexpr (D == 2) {
             row(o0, 0, b0, w0, q0, q2, qs, qd);
         } else {
@@ -535,7 +537,7 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(D == 3 && P
         // a particle whose bound is finite has every |contribution * scale| below 2^50 (up to the
         // rounding of the bracket, and the conversion holds to 2^51)
         if (finite[k]) {
-            adjoint_stencil<D, false>(
+            adjoint_stencil<D, false, !GENERAL>(
                 fxs[k], Bm, kb, 0.0f, node,
                 [&](const int (&off)[D], float weight, const float (&bi)[D]) {
                     int r = 0;
@@ -547,7 +549,7 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(D == 3 && P
                 },
                 m0, Tm, fxbar);
         } else {
-            adjoint_stencil<D, false>(
+            adjoint_stencil<D, false, !GENERAL>(
                 fxs[k], Bm, kb, 0.0f, node,
                 [&](const int (&off)[D], float weight, const float (&bi)[D]) {
                     int r = 0;
@@ -719,18 +721,21 @@ __global__ __launch_bounds__(Tile<D>::NODES) void k_grid_adjoint(const float4* _
 }
 
 // ---------------------------------------------------------------------------------------------
-// P2G adjoint (src/nclr.h:104-165, 313-372) per sorted position j.  Two waves per SIMD, as the
-// G2P adjoint (1.38x faster than one).
+// P2G adjoint (src/nclr.h:104-165, 313-372) per sorted position j, XCD-local block order.  In 3D the
+// forward P2G leaves the particle's polar factor in `rot` (36 bytes a particle; its exact SVD was a third of
+// this kernel's instructions), and F and the factor are read again behind the stencil instead of
+// held through it, which fits four waves per SIMD: 8 x 262,144 jelly particles 258 -> 180 us (296
+// bytes a particle, 3.4 TB/s), P2G 214 -> 216 with the factor's stores; 60,007 snow 19.0 -> 13.
 // ---------------------------------------------------------------------------------------------
 template <int D, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_p2g_adjoint(const float* __restrict__ st, const uint32_t* __restrict__ pid,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_p2g_adjoint(const float* __restrict__ st, const uint32_t* __restrict__ pid,
                                                      const uint32_t* __restrict__ perm,
                                                      const uint32_t* __restrict__ keys, StepParams p,
                                                      const float4* __restrict__ gbar, const float* __restrict__ gout,
                                                      float* __restrict__ gin, int64_t gstride,
-                                                     float* __restrict__ epart) {
+                                                     float* __restrict__ epart, const float* __restrict__ rot) {
     using L = Layout<D>;
-    const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t j = int64_t(xcd_block()) * blockDim.x + threadIdx.x;
     if (j >= p.n) return;
     const int64_t i = perm[j];
     const int64_t s = p.stride;
@@ -760,19 +765,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         epart[j] = 0.0f;
         return;
     }
-    // the forward's affine matrix from one polar factor: in the accurate mode its F - R is kept,
-    // and the stress backward below takes R = F - (F - R) (within one float rounding of the
-    // iteration's R) instead of a second Newton iteration; in the other modes R itself is kept and
-    // F - R formed as the forward forms it
+    // the forward's polar factor: in 3D P2G kept it (a third of this kernel's instructions were its SVD),
+    // F - R in the accurate mode and R in the others; F - R is formed as the forward forms it
     M<D> A, FmR, R;
-    if constexpr (D == 3 && MODE == kSvdAccurate) {
-        FmR = f_minus_rotation<MODE, D>(F);
-    } else {
-        R = rotation_mode<MODE, D>(F);
+    if constexpr (D == 3) {
 #pragma unroll
         for (int a = 0; a < D; ++a)
 #pragma unroll
-            for (int b = 0; b < D; ++b) FmR.a[a][b] = F.a[a][b] - R.a[a][b];
+            for (int b = 0; b < D; ++b) {
+                const float q = rot[int64_t(a * D + b) * s + j];
+                R.a[a][b] = MODE == kSvdAccurate ? F.a[a][b] - q : q;
+                FmR.a[a][b] = MODE == kSvdAccurate ? q : F.a[a][b] - q;
+            }
+    } else {
+        FmR = f_minus_rotation<MODE, D>(F, R);
     }
     A = fused_affine_from<D>(sp.material, F, FmR, C, Jp, mass, vol, sp);
     // the bracket m v + A dpos of P2G's contributions in cell units around the middle node
@@ -788,7 +794,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         }
     }
     const StencilRows<D> node(gbar, base, sp.ntn, sp.node_tile_base);
-    adjoint_stencil<D, true>(fx, Bm, kb, mass, node, [](const int (&)[D], float, const float (&)[D]) {}, m0, Abar, fxbar);
+    adjoint_stencil<D, true, false>(fx, Bm, kb, mass, node, [](const int (&)[D], float, const float (&)[D]) {}, m0, Abar, fxbar);
+    if constexpr (D == 3) {  // F and R again (they would hold 18 registers through the stencil)
+        const float* st2 = st;
+        const float* rot2 = rot;
+        asm volatile("" : "+s"(st2), "+s"(rot2));
+#pragma unroll
+        for (int a = 0; a < D; ++a)
+#pragma unroll
+            for (int b = 0; b < D; ++b) {
+                F.a[a][b] = ldf(st2, s, L::F + a * D + b, i);
+                const float q = rot2[int64_t(a * D + b) * s + j];
+                R.a[a][b] = MODE == kSvdAccurate ? F.a[a][b] - q : q;
+            }
+    }
     float vin[D];
 #pragma unroll
     for (int r = 0; r < D; ++r) {
@@ -813,12 +832,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
             sG += G.a[a][b];
         }
     // PF = 2 mu (F - R) F^T + lambda (J - 1) J on every entry
-    if constexpr (D == 3 && MODE == kSvdAccurate) {
-#pragma unroll
-        for (int a = 0; a < D; ++a)
-#pragma unroll
-            for (int b = 0; b < D; ++b) R.a[a][b] = F.a[a][b] - FmR.a[a][b];
-    }
     const float J = det(F);
     M<D> Fbar, Rbar;
     float mubar = 0.0f;
@@ -1055,18 +1068,14 @@ hipError_t launch_grid_adjoint(const LaunchArgs& a, const AdjointArgs& b) {
 
 hipError_t launch_p2g_adjoint(const LaunchArgs& a, const AdjointArgs& b) {
     if (a.p.n > 0) {
-        if (a.dim == 2)
-            k_p2g_adjoint<2, kSvdExact><<<blocks_of(a.p.n, 256), 256, 0, a.stream>>>(
-                a.state_in, a.pid_in, a.perm, a.keys, a.p, b.gbar, b.grad_out, b.grad_in, b.gstride, b.epart);
-        else if (a.svd_mode == kSvdAccurate)
-            k_p2g_adjoint<3, kSvdAccurate><<<blocks_of(a.p.n, 256), 256, 0, a.stream>>>(
-                a.state_in, a.pid_in, a.perm, a.keys, a.p, b.gbar, b.grad_out, b.grad_in, b.gstride, b.epart);
-        else if (a.svd_mode != kSvdFast)
-            k_p2g_adjoint<3, kSvdExact><<<blocks_of(a.p.n, 256), 256, 0, a.stream>>>(
-                a.state_in, a.pid_in, a.perm, a.keys, a.p, b.gbar, b.grad_out, b.grad_in, b.gstride, b.epart);
-        else
-            k_p2g_adjoint<3, kSvdFast><<<blocks_of(a.p.n, 256), 256, 0, a.stream>>>(
-                a.state_in, a.pid_in, a.perm, a.keys, a.p, b.gbar, b.grad_out, b.grad_in, b.gstride, b.epart);
+        const unsigned blocks = xcd_grid(blocks_of(a.p.n, 256));
+        auto launch = [&](auto kernel) {
+            kernel<<<blocks, 256, 0, a.stream>>>(a.state_in, a.pid_in, a.perm, a.keys, a.p, b.gbar, b.grad_out, b.grad_in,
+                                                 b.gstride, b.epart, a.rot);
+        };
+        if (a.dim == 2) launch(k_p2g_adjoint<2, kSvdExact>);
+        else if (a.svd_mode == kSvdAccurate) launch(k_p2g_adjoint<3, kSvdAccurate>);
+        else launch(k_p2g_adjoint<3, kSvdExact>);  // R from either method
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

@@ -137,6 +137,10 @@ struct nclr_mpm_sim {
     float4 *tape_gv = nullptr, *tape_gpre = nullptr;
     int64_t tape_grid_states = 0;
     float4* gpre = nullptr;  // the grid kernel's pre-update output (nullptr: not kept)
+    // 3D polar factors (LaunchArgs::rot): kept beside the grids on the tape, so that the P2G adjoint does
+    // not decompose F again; an adjoint step that recomputes P2G keeps them in rot_own
+    float *tape_rot = nullptr, *rot_own = nullptr;
+    float* rot = nullptr;
     int g2p_threads = 256;
     // compact step (single scene; mpm_compact.hip): particles per thread, 0 = off; its buffers are
     // allocated by the first compact launch
@@ -177,6 +181,7 @@ struct nclr_mpm_sim {
         a.slots = slots;
         a.gv = gv;
         a.gpre = gpre;
+        a.rot = rot;
         a.stamps = stamps;
         a.status = status;
         a.active = active;
@@ -742,6 +747,7 @@ struct nclr_mpm_sim {
             dmalloc(&epart, size_t(std::max<int64_t>(p.n, 1))) != hipSuccess ||
             dmalloc(&erange, 2 * scenes.size()) != hipSuccess ||
             dmalloc(&epartial, scenes.size() * size_t(echunks_for_scenes())) != hipSuccess ||
+            dmalloc(&rot_own, rot_floats()) != hipSuccess ||
             dmalloc(&gtmp[0], gfl) != hipSuccess || dmalloc(&gtmp[1], gfl) != hipSuccess)
             return fail(MPM_ERR_HIP, "hipMalloc of the adjoint buffers failed (out of device memory?)");
         return MPM_OK;
@@ -756,7 +762,8 @@ struct nclr_mpm_sim {
     int backward_step(const float* gout, float* gin, double* grad_E, bool presorted = false, bool grid_kept = false) {
         RC_TRY(ensure_adjoint());
         if (p.n == 0) return MPM_OK;
-        const nclr_host::LaunchArgs a = args(cur);
+        nclr_host::LaunchArgs a = args(cur);
+        if (!(presorted && grid_kept)) a.rot = rot_own;  // P2G is recomputed below
         const nclr_host::AdjointArgs b{gout, gin, p.n, slots_b, gbar, epart, grad_E, erange, epartial, echunks};
         PendingEvent pe{};
         if (opts.timing) RC_TRY(record_start(pe, kBackward));
@@ -790,14 +797,17 @@ struct nclr_mpm_sim {
     // laid out as save_state writes it (state 0 stays in the engine's own buffer); step t's sort
     // block (t < nsteps - 1) at sorts + t * sort_block_bytes; with a grid tape (gv non-null), step
     // t's forward grid and pre-update sums at gv + t * gv_nodes and gpre + t * gv_nodes (nsteps
-    // entries each: the last step's adjoint recomputes its grid into its entry).
+    // entries each: the last step's adjoint recomputes its grid into its entry) and, in 3D, its
+    // polar factors at rot + t * rot_floats (nsteps - 1 entries).
     struct SegTape {
         char* states;
         char* sorts;
         float4* gv;
         float4* gpre;
+        float* rot;
     };
 
+    size_t rot_floats() const { return dim == 3 ? 9 * size_t(p.stride) : 0; }
     size_t gv_nodes() const { return size_t(p.node_tiles) * nclr_host::tile_nodes(dim); }
 
     // The engine's own buffers and pointers for the length of a segment (graph replay off: graphs
@@ -833,6 +843,7 @@ struct nclr_mpm_sim {
             e.sorted_valid = advanced;  // the own sort block holds the last step's sort
             e.gv = gv;
             e.gpre = nullptr;
+            e.rot = nullptr;
             e.point_sort_block(e.sort_block);
         }
     };
@@ -864,6 +875,7 @@ struct nclr_mpm_sim {
             point_state(cur ^ 1, t + 1, T, g);
             gv = T.gv ? T.gv + size_t(t) * gn : g.gv;
             gpre = T.gv ? T.gpre + size_t(t) * gn : nullptr;
+            rot = T.gv && dim == 3 ? T.rot + size_t(t) * rot_floats() : nullptr;
             char* entry = T.sorts + sort_block_bytes * size_t(t);
             prev_sort = t == 0 ? sort_block : T.sorts + sort_block_bytes * size_t(t - 1);
             point_sort_block(entry);
@@ -890,6 +902,7 @@ struct nclr_mpm_sim {
             point_sort_block(kept ? T.sorts + sort_block_bytes * size_t(t) : sort_block);
             gv = T.gv && t != 0 ? T.gv + size_t(t) * gn : g.gv;
             gpre = T.gv ? T.gpre + size_t(t) * gn : nullptr;
+            rot = T.gv && dim == 3 && kept ? T.rot + size_t(t) * rot_floats() : nullptr;
             RC_TRY(backward_step(gtmp[c], gtmp[c ^ 1], grad_E, kept, kept && T.gv && t > 0));
             c ^= 1;
         }
@@ -922,25 +935,28 @@ struct nclr_mpm_sim {
             HIP_TRY(hipStreamSynchronize(stream));
             if (tape_gv) (void)hipFree(tape_gv);
             if (tape_gpre) (void)hipFree(tape_gpre);
+            if (tape_rot) (void)hipFree(tape_rot);
             tape_gv = tape_gpre = nullptr;
+            tape_rot = nullptr;
             tape_grid_states = 0;
             size_t free_b = 0, total_b = 0;
             HIP_TRY(hipMemGetInfo(&free_b, &total_b));
-            const size_t need = 2 * size_t(nsteps) * gn * sizeof(float4);
-            if (need <= free_b / 4 * 3 && dmalloc(&tape_gv, size_t(nsteps) * gn) == hipSuccess) {
-                if (dmalloc(&tape_gpre, size_t(nsteps) * gn) == hipSuccess) {
-                    tape_grid_states = nsteps;
-                } else {
-                    (void)hipFree(tape_gv);
-                    tape_gv = nullptr;
-                    (void)hipGetLastError();
-                }
+            const size_t nrot = size_t(nsteps - 1) * rot_floats();
+            const size_t need = 2 * size_t(nsteps) * gn * sizeof(float4) + nrot * sizeof(float);
+            if (need <= free_b / 4 * 3 && dmalloc(&tape_gv, size_t(nsteps) * gn) == hipSuccess &&
+                dmalloc(&tape_gpre, size_t(nsteps) * gn) == hipSuccess && dmalloc(&tape_rot, nrot) == hipSuccess) {
+                tape_grid_states = nsteps;
             } else {
+                if (tape_gv) (void)hipFree(tape_gv);
+                if (tape_gpre) (void)hipFree(tape_gpre);
+                tape_gv = tape_gpre = nullptr;
+                tape_rot = nullptr;
                 (void)hipGetLastError();
             }
         }
         const bool grid_tape = tape_grid_states >= nsteps;
-        const SegTape T{tape, sort_tape, grid_tape ? tape_gv : nullptr, grid_tape ? tape_gpre : nullptr};
+        const SegTape T{tape, sort_tape, grid_tape ? tape_gv : nullptr, grid_tape ? tape_gpre : nullptr,
+                        grid_tape ? tape_rot : nullptr};
         SegGuard g(*this);
         RC_TRY(record_steps(nsteps, T, g));
         return adjoint_steps(nsteps, T, g, gout, gin, grad_E);
@@ -959,10 +975,12 @@ struct nclr_mpm_sim {
         const size_t o_sorts = take(sort_block_bytes * size_t(nsteps - 1));
         const size_t grid_bytes = with_grid ? size_t(nsteps) * gv_nodes() * sizeof(float4) : 0;
         const size_t o_gv = take(grid_bytes), o_gpre = take(grid_bytes);
+        const size_t o_rot = take(with_grid ? size_t(nsteps - 1) * rot_floats() * sizeof(float) : 0);
         if (T)
             *T = SegTape{base + o_states, base + o_sorts,
                          with_grid ? reinterpret_cast<float4*>(base + o_gv) : nullptr,
-                         with_grid ? reinterpret_cast<float4*>(base + o_gpre) : nullptr};
+                         with_grid ? reinterpret_cast<float4*>(base + o_gpre) : nullptr,
+                         with_grid ? reinterpret_cast<float*>(base + o_rot) : nullptr};
         return std::max<size_t>(off, 256);  // a one-step segment without grids keeps nothing
     }
 
@@ -1007,6 +1025,7 @@ struct nclr_mpm_sim {
             pid[cur ^ 1] = g.pid[own];
             gv = g.gv;
             gpre = nullptr;
+            rot = nullptr;
             // the last step sorts into the engine's own block, from the step before's
             prev_sort = nsteps > 1 ? T.sorts + sort_block_bytes * size_t(nsteps - 2) : nullptr;
             point_sort_block(sort_block);
@@ -1091,7 +1110,10 @@ struct nclr_mpm_sim {
         tape_states = 0;
         if (tape_gv) (void)hipFree(tape_gv);
         if (tape_gpre) (void)hipFree(tape_gpre);
+        if (tape_rot) (void)hipFree(tape_rot);
+        if (rot_own) (void)hipFree(rot_own);
         tape_gv = tape_gpre = nullptr;
+        tape_rot = rot_own = nullptr;
         tape_grid_states = 0;
         state[0] = state[1] = nullptr;
         pid[0] = pid[1] = nullptr;
@@ -1633,7 +1655,8 @@ int mpm_backward_segment(mpm_handle h, int nsteps, const float* grad_out, float*
 int64_t mpm_tape_bytes(mpm_handle h, int nsteps) {
     if (!h || nsteps < 1) return -1;
     const int64_t grid = 2 * int64_t(h->p.node_tiles) * int64_t(nclr_host::tile_nodes(h->dim)) * int64_t(sizeof(float4));
-    return int64_t(nsteps - 1) * int64_t(h->state_bytes() + h->sort_block_bytes) + int64_t(nsteps) * grid;
+    const int64_t rot = int64_t(h->rot_floats() * sizeof(float));
+    return int64_t(nsteps - 1) * (int64_t(h->state_bytes() + h->sort_block_bytes) + rot) + int64_t(nsteps) * grid;
 }
 
 int64_t mpm_record_bytes(mpm_handle h, int nsteps, int with_grid) {

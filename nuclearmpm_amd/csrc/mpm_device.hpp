@@ -116,7 +116,8 @@ NCLR_DI M<D> fused_affine_from(int material, const M<D>& F, const M<D>& diff, co
 template <int D, int MODE>
 NCLR_DI M<D> fused_affine(int material, const M<D>& F, const M<D>& C, float Jp, float mass, float vol,
                           const SceneParams& sp) {
-    return fused_affine_from<D>(material, F, f_minus_rotation<MODE, D>(F), C, Jp, mass, vol, sp);
+    M<D> keep;
+    return fused_affine_from<D>(material, F, f_minus_rotation<MODE, D>(F, keep), C, Jp, mass, vol, sp);
 }
 
 template <int D>
@@ -565,12 +566,13 @@ NCLR_DI void round_carries(const uint32_t* __restrict__ rtot, uint32_t round, ui
 // contributions at or beyond kFixedLimit flag their node channel (NaN) instead.
 constexpr float kFixedLimit = 1.12589991e15f;  // 2^50
 
+// (Uniform over the workgroup: kept in scalar registers, up to 12 vector registers through the deposits.)
 NCLR_DI void fixed_point_scale(float bound_max, float& scale, double& inv_scale) {
     int ex = 0;
     (void)frexpf(bound_max > 0.0f && bound_max < 3.0e38f ? bound_max : 1.0f, &ex);  // bound_max < 2^ex
-    const int e = min(127, 50 - ex);                                                  // in [-78, 127]
-    scale = ldexpf(1.0f, e);
-    inv_scale = ldexp(1.0, -e);
+    const int e = __builtin_amdgcn_readfirstlane(min(127, 50 - ex));                  // in [-78, 127]
+    scale = __int_as_float((e + 127) << 23);
+    inv_scale = __hiloint2double((1023 - e) << 20, 0);
 }
 
 // y (|y| < 2^51) rounded to the nearest integer (ties to even), as a two's complement 64-bit

@@ -161,6 +161,8 @@ struct LaunchArgs {
     float4* gv;                // node tiles * NODES, updated grid
     float4* gpre;              // optional (nullptr): node tiles * NODES, the grid's {momentum, mass} before
                                // the update (written by the grid kernel, read by the grid adjoint)
+    float* rot;                // optional (nullptr): 9 * stride, 3D: per sorted particle its polar factor (R; F - R
+                               // in the accurate mode), written by P2G and read by the P2G adjoint
     uint32_t* stamps;          // node tiles
     uint32_t* status;
     uint32_t* active;          // node tiles: nodes with post-P2G mass > 0

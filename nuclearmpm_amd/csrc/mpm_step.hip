@@ -142,7 +142,7 @@ __global__ __launch_bounds__(1024) void k_items_rounds(const uint32_t* __restric
 template <int D, int MAT, int PPT, int MODE, int TPB = 256>
 __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, const uint32_t* __restrict__ perm,
                                                   const uint32_t* __restrict__ item_offset, StepParams p,
-                                                  float4* __restrict__ slots) {
+                                                  float4* __restrict__ slots, float* __restrict__ rot) {
     using TL = Tile<D>;
     using L = Layout<D>;
     constexpr int REG = TL::REGION;
@@ -206,7 +206,14 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
         float fx[D], w[D][3];
         if (!stencil<D>(x, sp, base, fx, w)) continue;  // keyed into this tile, so never taken
         valid[k] = true;
-        As[k] = fused_affine<D, MODE>(material, F, C, Jp, mass, vol, sp);
+        M<D> keep;
+        const M<D> FmR = f_minus_rotation<MODE, D>(F, keep);
+        if (D == 3 && rot)  // a recorded or adjoint step: the polar factor, for the P2G adjoint
+#pragma unroll
+            for (int a = 0; a < D; ++a)
+#pragma unroll
+                for (int b = 0; b < D; ++b) rot[int64_t(a * D + b) * p.stride + j] = keep.a[a][b];
+        As[k] = fused_affine_from<D>(material, F, FmR, C, Jp, mass, vol, sp);
         ms[k] = mass;
         float wsum = 1.0f;
 #pragma unroll
@@ -626,9 +633,9 @@ static void p2g_mode(const LaunchArgs& a) {
     const unsigned g = unsigned((a.p.n + 256 * PPT - 1) / (256 * PPT) + a.p.ntiles);
     if (a.p.n < int64_t(D == 2 ? kFewItems : 4 * kFewItems) * 256 * PPT)
         k_p2g_tile<D, MAT, 1, MODE, 256 * PPT><<<g, 256 * PPT, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p,
-                                                                             a.slots);
+                                                                             a.slots, a.rot);
     else
-        k_p2g_tile<D, MAT, PPT, MODE><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p, a.slots);
+        k_p2g_tile<D, MAT, PPT, MODE><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p, a.slots, a.rot);
 }
 
 template <int D, int MAT, int PPT>
