@@ -111,12 +111,14 @@ struct nclr_mpm_sim {
     int64_t stamp_host = 0;  // mirror of the device step stamp (one increment per step and per adjoint step)
     bool sorted_valid = false;
     // adjoint buffers, allocated by the first backward call
+    bool adjoint_ready = false;
     float4* slots_b = nullptr;
     float4* gbar = nullptr;
     float* epart = nullptr;
     int64_t* erange = nullptr;  // adjoint: per scene, its sorted range
     double* epartial = nullptr; // adjoint: per scene, partial sums of dL/dE
     int echunks = 1;
+    int e_steps = 0;            // adjoint steps that epart, erange and epartial hold
     float* gtmp[2] = {nullptr, nullptr};
     char* tape = nullptr;  // saved states of a backward segment
     // The sort's outputs (keys, perm, tile bounds, item offsets, the item and node tile lists, meta) live in one
@@ -738,58 +740,80 @@ struct nclr_mpm_sim {
         grid_tiles = base + so_gtiles;
     }
 
-    int ensure_adjoint() {
-        if (slots_b) return MPM_OK;
-        const size_t slot_nodes = size_t(nclr_host::max_items(p.n, p.ntiles)) * nclr_host::region_nodes(dim);
-        const size_t gv_nodes = size_t(p.node_tiles) * nclr_host::tile_nodes(dim);
-        const size_t gfl = size_t(grad_channels()) * size_t(std::max<int64_t>(p.n, 1));
-        if (dmalloc(&slots_b, slot_nodes) != hipSuccess || dmalloc(&gbar, gv_nodes) != hipSuccess ||
-            dmalloc(&epart, size_t(std::max<int64_t>(p.n, 1))) != hipSuccess ||
-            dmalloc(&erange, 2 * scenes.size()) != hipSuccess ||
-            dmalloc(&epartial, scenes.size() * size_t(echunks_for_scenes())) != hipSuccess ||
-            dmalloc(&rot_own, rot_floats()) != hipSuccess ||
-            dmalloc(&gtmp[0], gfl) != hipSuccess || dmalloc(&gtmp[1], gfl) != hipSuccess)
-            return fail(MPM_ERR_HIP, "hipMalloc of the adjoint buffers failed (out of device memory?)");
-        return MPM_OK;
+    // Room for the dL/dE contributions of `steps` adjoint steps between two sums.
+    hipError_t grow_e_steps(int steps) {
+        if (e_steps >= steps) return hipSuccess;
+        if (epart) (void)hipFree(epart);
+        if (erange) (void)hipFree(erange);
+        if (epartial) (void)hipFree(epartial);
+        epart = nullptr;
+        erange = nullptr;
+        epartial = nullptr;
+        e_steps = 0;
+        hipError_t e = dmalloc(&epart, size_t(steps) * size_t(std::max<int64_t>(p.n, 1)));
+        if (e == hipSuccess) e = dmalloc(&erange, size_t(steps) * 2 * scenes.size());
+        if (e == hipSuccess) e = dmalloc(&epartial, size_t(steps) * scenes.size() * size_t(echunks_for_scenes()));
+        if (e == hipSuccess) e_steps = steps;
+        return e;
     }
 
+    int ensure_adjoint() {
+        if (adjoint_ready) return MPM_OK;
+        const size_t slot_nodes = size_t(nclr_host::max_items(p.n, p.ntiles)) * nclr_host::region_nodes(dim);
+        const size_t gfl = size_t(grad_channels()) * size_t(std::max<int64_t>(p.n, 1));
+        auto alloc = [](auto** q, size_t count) { return *q ? hipSuccess : dmalloc(q, count); };
+        if (alloc(&slots_b, slot_nodes) != hipSuccess || alloc(&gbar, gv_nodes()) != hipSuccess ||
+            grow_e_steps(1) != hipSuccess || alloc(&rot_own, rot_floats()) != hipSuccess ||
+            alloc(&gtmp[0], gfl) != hipSuccess || alloc(&gtmp[1], gfl) != hipSuccess)
+            return fail(MPM_ERR_HIP, "hipMalloc of the adjoint buffers failed (out of device memory?)");
+        adjoint_ready = true;
+        return MPM_OK;
+    }
 
     // One adjoint step of the current state: recompute sort, P2G and the grid update, then run the
     // adjoint kernels.  The state and the step counter are left unchanged.
     // presorted: the sort block already holds this state's sort (a backward segment restored it);
     // only the device step stamp advances.  grid_kept: gv and gpre already hold this state's
     // forward grid (a backward segment's recomputed step wrote them): only the adjoint kernels run.
-    int backward_step(const float* gout, float* gin, double* grad_E, bool presorted = false, bool grid_kept = false) {
+    // order_kept: the state is stored in the order of prev_sort's sort (a segment's last state): the
+    // sort is the incremental one.  slot: where the step's dL/dE contributions go (sum_e adds them up).
+    int backward_step(const float* gout, float* gin, bool presorted = false, bool grid_kept = false,
+                      bool order_kept = false, int slot = 0) {
         RC_TRY(ensure_adjoint());
         if (p.n == 0) return MPM_OK;
         nclr_host::LaunchArgs a = args(cur);
         if (!(presorted && grid_kept)) a.rot = rot_own;  // P2G is recomputed below
-        const nclr_host::AdjointArgs b{gout, gin, p.n, slots_b, gbar, epart, grad_E, erange, epartial, echunks};
+        const nclr_host::AdjointArgs b{gout, gin, p.n, slots_b, gbar, epart + int64_t(slot) * p.n};
         PendingEvent pe{};
         if (opts.timing) RC_TRY(record_start(pe, kBackward));
-        if (presorted && grid_kept) {
-            RC_TRY(timed(kG2PAdj, [&] { return nclr_host::launch_g2p_adjoint(a, b); }));
-            RC_TRY(timed(kGridAdj, [&] { return nclr_host::launch_grid_adjoint(a, b); }));
-            RC_TRY(timed(kP2GAdj, [&] { return nclr_host::launch_p2g_adjoint(a, b); }));
-            if (opts.timing) RC_TRY(record_stop(pe));
-            return MPM_OK;
+        if (!(presorted && grid_kept)) {
+            if (presorted) {
+                HIP_TRY(nclr_host::launch_bump_u32(stamp, stream));
+            } else {
+                // the sort rewrites the sort block (keys, tile bounds, work items) for the current
+                // state, whose slots are still in the previous step's order: the next step must sort
+                // from scratch, not incrementally from that block
+                if (order_kept) RC_TRY(timed(kSort, [&] { return nclr_host::launch_sort_incremental(a); }));
+                else RC_TRY(timed(kSort, [&] { return nclr_host::launch_sort(a); }));
+                sorted_valid = false;
+            }
+            RC_TRY(timed(kP2G, [&] { return nclr_host::launch_p2g(a); }));
+            RC_TRY(timed(kGrid, [&] { return nclr_host::launch_grid(a); }));
+            stamp_host += 1;
         }
-        if (presorted) {
-            HIP_TRY(nclr_host::launch_bump_u32(stamp, stream));
-        } else {
-            // the radix sort rewrites the sort block (keys, tile bounds, work items) for the current
-            // state, whose slots are still in the previous step's order: the next step must sort
-            // from scratch, not incrementally from that block
-            RC_TRY(timed(kSort, [&] { return nclr_host::launch_sort(a); }));
-            sorted_valid = false;
-        }
-        RC_TRY(timed(kP2G, [&] { return nclr_host::launch_p2g(a); }));
-        RC_TRY(timed(kGrid, [&] { return nclr_host::launch_grid(a); }));
         RC_TRY(timed(kG2PAdj, [&] { return nclr_host::launch_g2p_adjoint(a, b); }));
         RC_TRY(timed(kGridAdj, [&] { return nclr_host::launch_grid_adjoint(a, b); }));
         RC_TRY(timed(kP2GAdj, [&] { return nclr_host::launch_p2g_adjoint(a, b); }));
         if (opts.timing) RC_TRY(record_stop(pe));
-        stamp_host += 1;
+        return MPM_OK;
+    }
+
+    // grad_E += the contributions of the `steps` adjoint steps first, first - 1, ... of a segment of nsteps
+    // steps whose sorts are at `sorts` (the last step's in the own block), held in slots 0, 1, ...
+    int sum_e(int first, int steps, int nsteps, const char* sorts, double* grad_E) {
+        const nclr_dev::ESteps es{epart, p.n, sorts, sort_block, int64_t(sort_block_bytes), int64_t(so_keys),
+                                  int64_t(so_meta), first, nsteps - 1};
+        HIP_TRY(nclr_host::launch_e_sum(p, es, steps, erange, epartial, echunks, grad_E, stream));
         return MPM_OK;
     }
 
@@ -894,7 +918,19 @@ struct nclr_mpm_sim {
         const size_t gn = gv_nodes();
         const size_t gbytes = size_t(grad_channels()) * size_t(p.n) * sizeof(float);
         HIP_TRY(hipMemcpyAsync(gtmp[0], gout, gbytes, hipMemcpyDeviceToDevice, stream));
-        int c = 0;
+        int c = 0, held = 0;
+        const int room = std::min(nsteps, nclr_dev::kESteps);
+        if (grad_E && e_steps < room) {
+            HIP_TRY(hipStreamSynchronize(stream));
+            if (grow_e_steps(room) != hipSuccess) {  // no room: sums step by step
+                (void)hipGetLastError();
+                HIP_TRY(grow_e_steps(1));
+            }
+        }
+        struct PrevReset {
+            char*& prev;
+            ~PrevReset() { prev = nullptr; }
+        } reset{prev_sort};
         for (int t = nsteps - 1; t >= 0; --t) {
             point_state(cur, t, T, g);
             sorted_valid = false;
@@ -903,8 +939,15 @@ struct nclr_mpm_sim {
             gv = T.gv && t != 0 ? T.gv + size_t(t) * gn : g.gv;
             gpre = T.gv ? T.gpre + size_t(t) * gn : nullptr;
             rot = T.gv && dim == 3 && kept ? T.rot + size_t(t) * rot_floats() : nullptr;
-            RC_TRY(backward_step(gtmp[c], gtmp[c ^ 1], grad_E, kept, kept && T.gv && t > 0));
+            // the last state is stored in the order of the step before's sort
+            const bool order_kept = !kept && t > 0;
+            prev_sort = order_kept ? T.sorts + sort_block_bytes * size_t(t - 1) : nullptr;
+            RC_TRY(backward_step(gtmp[c], gtmp[c ^ 1], kept, kept && T.gv && t > 0, order_kept, held));
             c ^= 1;
+            if (grad_E && (++held == e_steps || held == nclr_dev::kESteps || t == 0)) {
+                RC_TRY(sum_e(t + held - 1, held, nsteps, T.sorts, grad_E));
+                held = 0;
+            }
         }
         HIP_TRY(hipMemcpyAsync(gin, gtmp[c], gbytes, hipMemcpyDeviceToDevice, stream));
         return MPM_OK;
@@ -1642,7 +1685,8 @@ int mpm_backward_step(mpm_handle h, const float* grad_out, float* grad_in, doubl
     if (grad_out == grad_in && h->p.n > 0) return fail(MPM_ERR_INVALID, "grad_out and grad_in must not alias");
     HIP_TRY(hipSetDevice(h->opts.device));
     RC_TRY(h->require_live());
-    return h->backward_step(grad_out, grad_in, grad_E);
+    RC_TRY(h->backward_step(grad_out, grad_in));
+    return h->p.n > 0 && grad_E ? h->sum_e(0, 1, 1, nullptr, grad_E) : MPM_OK;
 }
 
 int mpm_backward_segment(mpm_handle h, int nsteps, const float* grad_out, float* grad_in, double* grad_E) {

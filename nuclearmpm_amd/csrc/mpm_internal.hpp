@@ -106,6 +106,23 @@ enum CompactReason : int {
     kCompactStopped = 2    // a particle left the grid: the scene stopped (the stamp counts every step)
 };
 
+// The adjoint steps whose dL/dE contributions one launch sums: step k of the launch (k = 0 first in time of the
+// backward pass) is step `first` - k of the segment, its contributions at epart + k * stride and
+// its sort block (keys and meta at fixed offsets) on the sort tape, or, for the segment's last
+// step, the engine's own.
+constexpr int kESteps = 32;
+struct ESteps {
+    const float* epart;
+    int64_t stride;
+    const char *sorts, *own_sort;
+    int64_t sort_bytes;
+    int64_t keys, meta;
+    int first, last;  // the segment's step of k = 0; the segment's last step
+    __host__ __device__ const char* sort(int k) const {
+        return first - k == last ? own_sort : sorts + sort_bytes * (first - k);
+    }
+};
+
 // Arguments of the compact step kernel (one scene, many steps per launch).
 struct CompactArgs {
     float* st;             // SoA state, updated in place
@@ -190,12 +207,13 @@ struct AdjointArgs {
     int64_t gstride;
     float4* slots_b;        // max_items * REGION: per work item, the G2P adjoint's grid cotangent
     float4* gbar;           // node tiles * NODES: cotangent of the pre-update grid {momentum, mass}
-    float* epart;           // n: per sorted particle, its contribution to dL/dE of its scene
-    double* grad_E;         // nscenes: accumulated dL/dE
-    int64_t* erange;        // 2 nscenes: each scene's sorted range [lo, hi)
-    double* epartial;       // nscenes * echunks: partial sums of dL/dE
-    int echunks;            // e_chunks(largest scene)
+    float* epart;           // n: per sorted particle, its contribution to dL/dE of its scene (launch_e_sum)
 };
+// grad_E[s] += the contributions of `steps` adjoint steps (at most kESteps), in order.  erange: 2 nscenes per
+// step, each scene's sorted range [lo, hi); epartial: nscenes * echunks partial sums per step; echunks:
+// e_chunks(largest scene).
+hipError_t launch_e_sum(const nclr_dev::StepParams& p, const nclr_dev::ESteps& es, int steps, int64_t* erange,
+                        double* epartial, int echunks, double* grad_E, hipStream_t s);
 
 // Chunks of the fixed-order dL/dE sum for a scene of n particles.
 int e_chunks(int64_t n);

@@ -113,3 +113,27 @@ def test_radix_sort_at_the_edges_of_its_tiles(n, bits):
                  np.full(n, 0xA5A5A5A5, np.uint32)):                              # all equal
         low = keys if bits == 32 else keys & np.uint32((1 << bits) - 1)
         assert np.array_equal(sort_keys(keys, bits), np.argsort(low, kind="stable").astype(np.uint32))
+
+
+@pytest.mark.parametrize("dim,scenes", [(2, 1), (3, 2)])
+def test_segments_longer_than_one_sum_of_the_elasticity_gradient(dim, scenes):
+    """dL/dE is summed up to 32 adjoint steps at a time, and a segment's last state is sorted from the
+    step before's order: the same gradients, bit for bit, for segments of 1, 7 and 70 steps."""
+    import torch
+
+    from nuclearmpm_amd import autodiff
+
+    specs = [SceneSpec(_cloud(dim, 900 + 700 * s, 5 + s), MaterialModel.kJelly, 48, E=1e3) for s in range(scenes)]
+    cot = None
+    grads = []
+    with MPMBatch(specs, identity_mode=1) as sim:
+        image = sim.state_image()
+        for every in (1, 7, 70):
+            s0 = image.clone().requires_grad_(True)
+            E = torch.tensor([1e3 + 100.0 * s for s in range(scenes)], dtype=torch.float64, requires_grad=True)
+            out = autodiff.rollout(sim, s0, E, steps=70, checkpoint_every=every)
+            if cot is None:
+                cot = torch.randn(out.shape, generator=torch.Generator("cuda").manual_seed(1), device="cuda")
+            grads.append(torch.autograd.grad(out, (s0, E), cot))
+    for g in grads[1:]:
+        assert torch.equal(g[0], grads[0][0]) and torch.equal(g[1], grads[0][1])
