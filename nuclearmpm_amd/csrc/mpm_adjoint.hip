@@ -997,20 +997,6 @@ __global__ __launch_bounds__(1024) void k_scene_e_final(ESteps es, const double*
     if (threadIdx.x == 0) grad_E[sc] = sum;
 }
 
-// dst[c][to(i)] = src[c][from(i)]: with to_particle_order, slot i goes to particle pid[i];
-// otherwise slot i takes particle pid[i].
-__global__ __launch_bounds__(256) void k_permute_channels(const uint32_t* __restrict__ pid, const float* __restrict__ src,
-                                                          int64_t src_stride, float* __restrict__ dst,
-                                                          int64_t dst_stride, int channels, int64_t n,
-                                                          int to_particle_order) {
-    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int64_t u = pid[i];
-    const int64_t si = to_particle_order ? i : u;
-    const int64_t di = to_particle_order ? u : i;
-    for (int c = 0; c < channels; ++c) dst[int64_t(c) * dst_stride + di] = src[int64_t(c) * src_stride + si];
-}
-
 }  // namespace nclr_dev
 
 namespace nclr_host {
@@ -1110,14 +1096,5 @@ hipError_t launch_e_sum(const StepParams& p, const ESteps& es, int steps, int64_
 }
 
 int e_chunks(int64_t n) { return int(std::max<int64_t>(1, (n + kEChunk - 1) / kEChunk)); }
-
-hipError_t launch_permute_channels(const uint32_t* pid, const float* src, int64_t src_stride, float* dst,
-                                   int64_t dst_stride, int channels, int64_t n, bool to_particle_order,
-                                   hipStream_t s) {
-    if (n <= 0) return hipSuccess;
-    k_permute_channels<<<blocks_of(n, 256), 256, 0, s>>>(pid, src, src_stride, dst, dst_stride, channels, n,
-                                                         to_particle_order ? 1 : 0);
-    return hipGetLastError();
-}
 
 }  // namespace nclr_host

@@ -102,14 +102,17 @@ struct nclr_mpm_sim {
     // tile bounds / work items of that sort are intact (cleared by uploads, loads, re-tuning)
     uint32_t *uidx = nullptr, *ucnt = nullptr, *upref = nullptr, *ttotal = nullptr, *meta = nullptr;
     uint32_t* rtot = nullptr;
+    uint32_t* line_changes = nullptr;  // one word: how incoherent an order is (mpm_order.hip)
     uint32_t *tile_scene = nullptr, *node_tile_scene = nullptr;  // scene maps (batches only)
     // per scene (device): status bits raised since the last read, and the stamp of the step that
     // stopped the scene (StepParams::scene_flags / scene_frozen); host: every bit reported since
     // the state was last set
     uint32_t *scene_flags = nullptr, *scene_frozen = nullptr;
+    uint32_t* off_grid = nullptr;  // per scene: a sorted image had a particle off its grid
     std::vector<uint32_t> scene_seen;
     int64_t stamp_host = 0;  // mirror of the device step stamp (one increment per step and per adjoint step)
     bool sorted_valid = false;
+    bool slots_sorted = false;  // the current state's own sort stands (a sorted image): the step needs none
     // adjoint buffers, allocated by the first backward call
     bool adjoint_ready = false;
     float4* slots_b = nullptr;
@@ -186,6 +189,7 @@ struct nclr_mpm_sim {
         a.rot = rot;
         a.stamps = stamps;
         a.status = status;
+        a.off_grid = off_grid;
         a.active = active;
         a.uidx = uidx;
         a.ucnt = ucnt;
@@ -260,7 +264,8 @@ struct nclr_mpm_sim {
     }
 
     int launch_step_kernels(const nclr_host::LaunchArgs& a) {
-        if (sorted_valid) RC_TRY(timed(kSort, [&] { return nclr_host::launch_sort_incremental(a); }));
+        if (sorted_valid && slots_sorted) RC_TRY(timed(kSort, [&] { return nclr_host::launch_sorted_step(a); }));
+        else if (sorted_valid) RC_TRY(timed(kSort, [&] { return nclr_host::launch_sort_incremental(a); }));
         else RC_TRY(timed(kSort, [&] { return nclr_host::launch_sort(a); }));
         RC_TRY(timed(kP2G, [&] { return nclr_host::launch_p2g(a); }));
         RC_TRY(timed(kGrid, [&] { return nclr_host::launch_grid(a); }));
@@ -298,7 +303,7 @@ struct nclr_mpm_sim {
     int step() {
         // graphs hold the incremental sort; a step after an upload or load runs eagerly with the
         // full radix sort, which also rebuilds the tile bounds and work items
-        const bool use_graph = opts.graph && !opts.timing && sorted_valid;
+        const bool use_graph = opts.graph && !opts.timing && sorted_valid && !slots_sorted;
         if (use_graph) {
             if (!graph_exec[cur]) RC_TRY(capture(cur));
             HIP_TRY(hipGraphLaunch(graph_exec[cur], stream));
@@ -310,6 +315,7 @@ struct nclr_mpm_sim {
         }
         if (p.n > 0) cur ^= 1;
         sorted_valid = true;
+        slots_sorted = false;
         steps += 1;
         stamp_host += 1;
         return MPM_OK;
@@ -851,6 +857,7 @@ struct nclr_mpm_sim {
             : e(s), state{s.state[0], s.state[1]}, pid{s.pid[0], s.pid[1]}, cur(s.cur), steps(s.steps),
               graph(s.opts.graph), gv(s.gv) {
             s.opts.graph = 0;
+            s.slots_sorted = false;  // the segment's first step sorts into its tape entry
         }
         ~SegGuard() {
             for (int k = 0; k < 2; ++k) {
@@ -1128,7 +1135,7 @@ struct nclr_mpm_sim {
         void* bufs[] = {state[0], state[1], pid[0],  pid[1],   sort_block, keys_tmp, perm_tmp,
                         hist,     slots, gv, stamps, status,
                         active,   active_sum, stamp,    d_scenes, slots_b, gbar, epart, erange, epartial, gtmp[0],
-                        gtmp[1],  tape,       sort_tape, uidx,     ucnt,        upref, ttotal, rtot,
+                        gtmp[1],  tape,       sort_tape, uidx,     ucnt,        upref, ttotal, rtot, line_changes, off_grid,
                         tile_scene, node_tile_scene, scene_flags, scene_frozen, cslots, cgrid, cmassive, cbox, cinfo,
                         csubbox, cbar};
         for (void* b : bufs)
@@ -1280,6 +1287,7 @@ int create_impl(int dim, int nscenes, const mpm_scene* sc, const float* x, const
         dmalloc(&h->ucnt, bucket_cells) != hipSuccess || dmalloc(&h->upref, bucket_cells) != hipSuccess ||
         dmalloc(&h->ttotal, nbins) != hipSuccess ||
         dmalloc(&h->rtot, 2 * (size_t(tiles) / nclr_dev::kScanRound + 2)) != hipSuccess ||
+        dmalloc(&h->line_changes, 1) != hipSuccess || dmalloc(&h->off_grid, size_t(nscenes)) != hipSuccess ||
         dmalloc(&h->scene_flags, size_t(nscenes)) != hipSuccess || dmalloc(&h->scene_frozen, size_t(nscenes)) != hipSuccess)
         return cleanup(fail(MPM_ERR_HIP, "hipMalloc failed (out of device memory?)"));
     p.scenes = h->d_scenes;
@@ -1640,7 +1648,8 @@ int mpm_get_state_device(mpm_handle h, float* dst) {
     if (!h || (!dst && h->p.n > 0)) return fail(MPM_ERR_INVALID, "NULL argument");
     HIP_TRY(hipSetDevice(h->opts.device));
     HIP_TRY(nclr_host::launch_permute_channels(h->pid[h->cur], h->state[h->cur], h->p.stride, dst, h->p.n,
-                                               h->grad_channels(), h->p.n, true, h->stream));
+                                               h->grad_channels(), h->p.n, true, h->state[h->cur ^ 1], h->line_changes,
+                                               h->stream));
     return MPM_OK;
 }
 
@@ -1650,15 +1659,23 @@ int mpm_set_state_device(mpm_handle h, const float* src) {
     const int64_t n = h->p.n, stride = h->p.stride;
     if (n == 0) return MPM_OK;
     const int o = h->cur ^ 1, ng = h->grad_channels();
-    // Jp, mass and volume into particle order, then x, v, F, C from the caller; slots = particles
-    HIP_TRY(nclr_host::launch_permute_channels(h->pid[h->cur], h->state[h->cur] + int64_t(ng) * stride, stride,
-                                               h->state[o] + int64_t(ng) * stride, stride, h->nf() - ng, n, true,
-                                               h->stream));
-    HIP_TRY(hipMemcpy2DAsync(h->state[o], size_t(stride) * sizeof(float), src, size_t(n) * sizeof(float),
-                             size_t(n) * sizeof(float), size_t(ng), hipMemcpyDeviceToDevice, h->stream));
-    HIP_TRY(nclr_host::launch_iota_u32(h->pid[o], stride, h->stream));
+    if (nclr_host::image_goes_sorted(n)) {
+        // stored in tile order, with the sort's tables: the next step sorts incrementally
+        const nclr_host::LaunchArgs a = h->args(h->cur);
+        HIP_TRY(nclr_host::launch_image_keys(a, src, nclr_host::key_sort_input(a)));
+        HIP_TRY(nclr_host::launch_key_sort(a));
+        HIP_TRY(nclr_host::launch_image_to_slots(a, src, ng, h->state[o], h->pid[o], h->line_changes));
+    } else {
+        // Jp, mass and volume into particle order, then x, v, F, C from the caller; slots = particles
+        HIP_TRY(nclr_host::launch_permute_channels(h->pid[h->cur], h->state[h->cur] + int64_t(ng) * stride, stride,
+                                                   h->state[o] + int64_t(ng) * stride, stride, h->nf() - ng, n, true,
+                                                   nullptr, nullptr, h->stream));
+        HIP_TRY(hipMemcpy2DAsync(h->state[o], size_t(stride) * sizeof(float), src, size_t(n) * sizeof(float),
+                                 size_t(n) * sizeof(float), size_t(ng), hipMemcpyDeviceToDevice, h->stream));
+        HIP_TRY(nclr_host::launch_iota_u32(h->pid[o], stride, h->stream));
+    }
     h->cur = o;
-    h->sorted_valid = false;
+    h->sorted_valid = h->slots_sorted = nclr_host::image_goes_sorted(n);
     return h->clear_scene_state();
 }
 
@@ -1667,7 +1684,7 @@ int mpm_grad_from_particle_order(mpm_handle h, const float* src, float* dst) {
     if (src == dst && h->p.n > 0) return fail(MPM_ERR_INVALID, "src and dst must not alias");
     HIP_TRY(hipSetDevice(h->opts.device));
     HIP_TRY(nclr_host::launch_permute_channels(h->pid[h->cur], src, h->p.n, dst, h->p.n, h->grad_channels(), h->p.n,
-                                               false, h->stream));
+                                               false, h->state[h->cur ^ 1], h->line_changes, h->stream));
     return MPM_OK;
 }
 
@@ -1676,7 +1693,7 @@ int mpm_grad_to_particle_order(mpm_handle h, const float* src, float* dst) {
     if (src == dst && h->p.n > 0) return fail(MPM_ERR_INVALID, "src and dst must not alias");
     HIP_TRY(hipSetDevice(h->opts.device));
     HIP_TRY(nclr_host::launch_permute_channels(h->pid[h->cur], src, h->p.n, dst, h->p.n, h->grad_channels(), h->p.n,
-                                               true, h->stream));
+                                               true, h->state[h->cur ^ 1], h->line_changes, h->stream));
     return MPM_OK;
 }
 

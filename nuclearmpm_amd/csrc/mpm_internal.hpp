@@ -182,6 +182,7 @@ struct LaunchArgs {
                                // in the accurate mode), written by P2G and read by the P2G adjoint
     uint32_t* stamps;          // node tiles
     uint32_t* status;
+    uint32_t* off_grid;        // nscenes: a sorted image had a particle off the scene's grid
     uint32_t* active;          // node tiles: nodes with post-P2G mass > 0
     // incremental sort (mpm_bucket.hip)
     uint32_t* uidx;            // n: old work item of each slot
@@ -221,9 +222,23 @@ int e_chunks(int64_t n);
 hipError_t launch_g2p_adjoint(const LaunchArgs& a, const AdjointArgs& b);
 hipError_t launch_grid_adjoint(const LaunchArgs& a, const AdjointArgs& b);
 hipError_t launch_p2g_adjoint(const LaunchArgs& a, const AdjointArgs& b);
+// dst[c][pid[i]] = src[c][i], or with !to_particle_order dst[c][i] = src[c][pid[i]].  rows (n * channels floats)
+// and changes (one word) are scratch for a large set whose order is found incoherent; rows may be nullptr.
 hipError_t launch_permute_channels(const uint32_t* pid, const float* src, int64_t src_stride, float* dst,
-                                   int64_t dst_stride, int channels, int64_t n, bool to_particle_order,
-                                   hipStream_t s);
+                                   int64_t dst_stride, int channels, int64_t n, bool to_particle_order, float* rows,
+                                   uint32_t* changes, hipStream_t s);
+// A large state image is stored in tile order when it is set: its keys and cleared tile bounds
+// (into the radix sort's input), and after launch_key_sort the slots from the sorted order.  a.state_in / a.pid_in:
+// the state before, whose constants (mass, volume) the new one keeps and whose buffer is scratch.
+bool image_goes_sorted(int64_t n);
+hipError_t launch_image_keys(const LaunchArgs& a, const float* image, uint32_t* keys);
+hipError_t launch_image_to_slots(const LaunchArgs& a, const float* image, int channels, float* st, uint32_t* pid,
+                                 uint32_t* changes);
+// The sort of the first step after that (perm is the identity, the tables stand).
+hipError_t launch_sorted_step(const LaunchArgs& a);
+// The radix sort of a.p.n tile keys (in radix_keys_in's buffer), tile bounds (cleared) and work items.
+hipError_t launch_key_sort(const LaunchArgs& a);
+uint32_t* key_sort_input(const LaunchArgs& a);
 hipError_t launch_sort(const LaunchArgs& a);
 // The stable sort by tile for a state that is stored in the order of the previous sort, whose
 // tile bounds and work items are still in tile_start / tile_end / item_offset (same chunk size).

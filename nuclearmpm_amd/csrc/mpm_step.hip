@@ -590,16 +590,13 @@ static int key_bits(uint32_t max_key) {
     return b;
 }
 
-template <int D>
-static hipError_t sort_dispatch(const LaunchArgs& a) {
+uint32_t* key_sort_input(const LaunchArgs& a) { return radix_keys_in(a.keys, a.keys_tmp, key_bits(a.p.ntiles)); }
+
+hipError_t launch_key_sort(const LaunchArgs& a) {
     const auto& p = a.p;
-    const int64_t nb = int64_t(p.ntiles) + 1;
     hipStream_t s = a.stream;
-    const int bits = key_bits(p.ntiles);
-    k_keys<D><<<blocks_for(std::max<int64_t>(std::max<int64_t>(p.n, nb), 1), 256), 256, 0, s>>>(
-        a.state_in, a.pid_in, p, a.stamp, radix_keys_in(a.keys, a.keys_tmp, bits), a.status, a.tile_start, a.tile_end);
     if (p.n > 0) {
-        hipError_t e = radix_sort_pairs(a.keys, a.perm, a.keys_tmp, a.perm_tmp, a.hist, p.n, bits, s);
+        hipError_t e = radix_sort_pairs(a.keys, a.perm, a.keys_tmp, a.perm_tmp, a.hist, p.n, key_bits(p.ntiles), s);
         if (e != hipSuccess) return e;
         k_tile_bounds<<<blocks_for(p.n, 256), 256, 0, s>>>(a.keys, p.n, a.tile_start, a.tile_end);
     }
@@ -612,6 +609,18 @@ static hipError_t sort_dispatch(const LaunchArgs& a) {
         k_items_rounds<<<rounds, 1024, 0, s>>>(a.tile_start, a.tile_end, p.ntiles, uint32_t(p.chunk), a.item_offset,
                                                p.items, a.rtot, a.meta);
     }
+    return hipGetLastError();
+}
+
+template <int D>
+static hipError_t sort_dispatch(const LaunchArgs& a) {
+    const auto& p = a.p;
+    const int64_t nb = int64_t(p.ntiles) + 1;
+    hipStream_t s = a.stream;
+    k_keys<D><<<blocks_for(std::max<int64_t>(std::max<int64_t>(p.n, nb), 1), 256), 256, 0, s>>>(
+        a.state_in, a.pid_in, p, a.stamp, key_sort_input(a), a.status, a.tile_start, a.tile_end);
+    const hipError_t e = launch_key_sort(a);
+    if (e != hipSuccess) return e;
     if (p.node_tiles > 0 && grid_tiles_listed(D, p))
         k_list_grid_tiles<D><<<blocks_for(p.node_tiles, 256), 256, 0, s>>>(
             p, a.item_offset, static_cast<GridTile<D>*>(a.grid_tiles), a.meta, a.active);

@@ -137,3 +137,59 @@ def test_segments_longer_than_one_sum_of_the_elasticity_gradient(dim, scenes):
             grads.append(torch.autograd.grad(out, (s0, E), cot))
     for g in grads[1:]:
         assert torch.equal(g[0], grads[0][0]) and torch.equal(g[1], grads[0][1])
+
+
+@pytest.mark.parametrize("dim,n", [(2, 262144), (3, 300007)])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_large_state_images_in_any_order(dim, n, mixed):
+    """A state image of 2^18 particles or more is stored in tile order, and the channels go by rows where
+    the order is incoherent (mixed): the image comes back as it was, the steps are bit for bit those
+    of an engine built from the same particles, and cotangents survive both orders."""
+    import torch
+
+    from nuclearmpm_amd import autodiff
+    from nuclearmpm_amd._lib import check, lib
+
+    rng = np.random.default_rng(n)
+    side = int(np.ceil(n ** (1.0 / dim)))
+    idx = np.stack(np.unravel_index(np.arange(n), (side,) * dim), 1)
+    x = (0.2 + 0.5 * idx / side + 0.001 * rng.random((n, dim))).astype(np.float32)
+    p = Particles.from_positions(x[rng.permutation(n)] if mixed else x, identity_mode=1)
+    p.v = rng.normal(0, 1.0, p.v.shape).astype(np.float32)
+    p.C = rng.normal(0, 1.0, p.C.shape).astype(np.float32)
+    p.mass = (1.0 + rng.random(n)).astype(np.float32)
+    p.volume = (1.0 + rng.random(n)).astype(np.float32)
+    image = autodiff.pack(*(torch.from_numpy(getattr(p, k)).cuda() for k in ("x", "v", "F", "C", "Jp")))
+    cot = torch.randn(image.shape, generator=torch.Generator("cuda").manual_seed(3), device="cuda")
+    with MPMSimulation(p, MaterialModel.kJelly, 64, E=1e3, identity_mode=1) as a, \
+            MPMSimulation(p, MaterialModel.kJelly, 64, E=1e3, identity_mode=1) as b:
+        b.advance(2)
+        b.set_state_image(image)
+        assert torch.equal(b.state_image(), image)
+        a.advance(3)
+        b.advance(3)
+        pa, pb = a.particles(), b.particles()
+        for k in ("x", "v", "F", "C", "Jp", "mass", "volume"):
+            assert np.array_equal(getattr(pa, k), getattr(pb, k)), k
+        s = torch.cat([torch.from_numpy(getattr(pb, k)).reshape(n, -1) for k in ("x", "v", "F", "C", "Jp")], 1).t()
+        assert torch.equal(b.state_image().cpu(), s)
+        torch.cuda.synchronize()
+        slots, back = torch.empty_like(cot), torch.empty_like(cot)
+        check(lib().mpm_grad_from_particle_order(b._handle(), cot.data_ptr(), slots.data_ptr()))
+        check(lib().mpm_grad_to_particle_order(b._handle(), slots.data_ptr(), back.data_ptr()))
+        b.synchronize()
+        assert torch.equal(back, cot) and not torch.equal(slots, cot)
+        b.advance(1)  # the other state buffer was scratch
+        a.advance(1)
+        assert np.array_equal(a.particles().x, b.particles().x)
+        # a particle off its grid is found by the step, not by the call that sets the state
+        bad = image.clone()
+        bad[0, 12345] = 2.0
+        b.set_state_image(bad)
+        assert torch.equal(b.state_image(), bad)
+        b.advance(1)
+        with pytest.raises(IndexError):
+            b.synchronize()
+        b.set_state_image(image)
+        b.advance(1)
+        b.synchronize()
