@@ -241,6 +241,12 @@ int mpm_set_state_device(mpm_handle h, const float* src);
 /* Re-indexes a cotangent between particle order and the current slot order (src != dst). */
 int mpm_grad_from_particle_order(mpm_handle h, const float* src, float* dst);
 int mpm_grad_to_particle_order(mpm_handle h, const float* src, float* dst);
+/* The current slot order by itself (mpm_order_bytes(h) bytes of device memory), and a cotangent in
+ * particle order re-indexed to a saved order: the start of a backward pass from a state that is not
+ * kept. */
+int64_t mpm_order_bytes(mpm_handle h);
+int mpm_save_order(mpm_handle h, void* dst);
+int mpm_grad_to_saved_order(mpm_handle h, const void* order, const float* src, float* dst);
 
 /* The adjoint entry points below return MPM_ERR_OUT_OF_RANGE while a scene is stopped.
  *

@@ -150,6 +150,12 @@ def lib() -> ctypes.CDLL:
     for name in ("mpm_save_state", "mpm_load_state", "mpm_get_state_device", "mpm_set_state_device"):
         getattr(L, name).argtypes = [H, _vp]
         getattr(L, name).restype = i32
+    L.mpm_order_bytes.argtypes = [H]
+    L.mpm_order_bytes.restype = i64
+    L.mpm_save_order.argtypes = [H, _vp]
+    L.mpm_save_order.restype = i32
+    L.mpm_grad_to_saved_order.argtypes = [H, _vp, _vp, _vp]
+    L.mpm_grad_to_saved_order.restype = i32
     for name in ("mpm_grad_from_particle_order", "mpm_grad_to_particle_order"):
         getattr(L, name).argtypes = [H, _vp, _vp]
         getattr(L, name).restype = i32

@@ -130,15 +130,16 @@ class _Rollout(torch.autograd.Function):
                 check(L.mpm_advance_recorded(h, k, rec.data_ptr(), mode))
             ckpts.append((buf, k, rec, mode))
             done += k
-        final = torch.empty(sb, dtype=torch.uint8, device=state0.device)
-        check(L.mpm_save_state(h, final.data_ptr()))
+        # the final state's slot order, in which its cotangent is wanted
+        order = torch.empty(int(L.mpm_order_bytes(h)), dtype=torch.uint8, device=state0.device)
+        check(L.mpm_save_order(h, order.data_ptr()))
         out = torch.empty_like(state0)
         check(L.mpm_get_state_device(h, out.data_ptr()))
         check(L.mpm_synchronize(h))
         sim._cache = None
         ctx.sim = sim
         ctx.ckpts = ckpts
-        ctx.final = final
+        ctx.order = order
         ctx.E_meta = (E.dtype, E.device, E.shape)
         ctx.E_vals = E_vals
         ctx.nu_vals = list(sim._nus)
@@ -156,8 +157,7 @@ class _Rollout(torch.autograd.Function):
         for s, (e, nu) in enumerate(zip(ctx.E_vals, ctx.nu_vals)):
             sim.set_elasticity(s, e, nu)
         g = torch.empty_like(g_user)
-        check(L.mpm_load_state(h, ctx.final.data_ptr()))
-        check(L.mpm_grad_from_particle_order(h, g_user.data_ptr(), g.data_ptr()))
+        check(L.mpm_grad_to_saved_order(h, ctx.order.data_ptr(), g_user.data_ptr(), g.data_ptr()))
         for buf, k, rec, mode in reversed(ctx.ckpts):
             check(L.mpm_load_state(h, buf.data_ptr()))
             if rec is None:

@@ -108,6 +108,20 @@ struct nclr_mpm_sim {
     // stopped the scene (StepParams::scene_flags / scene_frozen); host: every bit reported since
     // the state was last set
     uint32_t *scene_flags = nullptr, *scene_frozen = nullptr;
+    // status, scene_flags and scene_frozen are one block (2 * nscenes + 1 words), so that a check reads
+    // them with one copy into pinned memory on the stream it waits for anyway: 15 us with the wait; three
+    // blocking copies after it took 47
+    uint32_t* host_words = nullptr;
+    // Exports no larger than kReadBlock go to pinned memory (kept, grown to the largest) with the
+    // status words, so that one wait serves both; larger ones straight to the caller's arrays, as the
+    // runtime's own staging is then as fast.  All particles, pinned and direct: 0.9 MiB 92 and 144 us,
+    // 6 MiB 374 and 530, 27 MiB 1614 and 1668 (with the reordering on the host 250, 1872 and 22154);
+    // a grid of 6 MiB 361 and 490, of 33 MiB 2345 and 2308.
+    static constexpr size_t kReadBlock = size_t(8) << 20;
+    char* host_read = nullptr;
+    size_t host_read_bytes = 0;
+    float* grid_out = nullptr;  // a scene's exported grid (kept, grown to the largest scene read)
+    int64_t grid_out_floats = 0;
     uint32_t* off_grid = nullptr;  // per scene: a sorted image had a particle off its grid
     std::vector<uint32_t> scene_seen;
     int64_t stamp_host = 0;  // mirror of the device step stamp (one increment per step and per adjoint step)
@@ -429,18 +443,25 @@ struct nclr_mpm_sim {
         return MPM_OK;
     }
 
+    // Device words status[1], scene_flags[nscenes], scene_frozen[nscenes] and their pinned copy.
+    hipError_t alloc_words(size_t ns) {
+        hipError_t e = dmalloc(&status, 2 * ns + 1);
+        if (e != hipSuccess) return e;
+        scene_flags = status + 1;
+        scene_frozen = scene_flags + ns;
+        return hipHostMalloc(reinterpret_cast<void**>(&host_words), (2 * ns + 1) * sizeof(uint32_t), 0);
+    }
+
     // Waits for the stream, checks the engine-wide status word and reads the per-scene words;
     // the scenes' new status bits move into scene_seen (and are cleared on the device).
     int sync_read(std::vector<uint32_t>& flags, std::vector<uint32_t>& frozen) {
         HIP_TRY(hipSetDevice(opts.device));
-        HIP_TRY(hipStreamSynchronize(stream));
         const size_t ns = scenes.size();
-        uint32_t st = 0;
-        flags.assign(ns, 0u);
-        frozen.assign(ns, 0u);
-        HIP_TRY(hipMemcpy(&st, status, sizeof(st), hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(flags.data(), scene_flags, ns * sizeof(uint32_t), hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(frozen.data(), scene_frozen, ns * sizeof(uint32_t), hipMemcpyDeviceToHost));
+        HIP_TRY(hipMemcpyAsync(host_words, status, (2 * ns + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
+        HIP_TRY(hipStreamSynchronize(stream));
+        const uint32_t st = host_words[0];
+        flags.assign(host_words + 1, host_words + 1 + ns);
+        frozen.assign(host_words + 1 + ns, host_words + 1 + 2 * ns);
         if (opts.timing) RC_TRY(resolve_events());
         bool any = false;
         for (size_t s = 0; s < ns; ++s) {
@@ -499,8 +520,7 @@ struct nclr_mpm_sim {
 
     // Clears the per-scene words (the state was replaced: every scene runs again).
     int clear_scene_state() {
-        HIP_TRY(nclr_host::launch_fill_u32(scene_flags, int64_t(scenes.size()), 0u, stream));
-        HIP_TRY(nclr_host::launch_fill_u32(scene_frozen, int64_t(scenes.size()), 0u, stream));
+        HIP_TRY(nclr_host::launch_fill_u32(scene_flags, 2 * int64_t(scenes.size()), 0u, stream));  // and scene_frozen
         std::fill(scene_seen.begin(), scene_seen.end(), 0u);
         compact_overflowed = false;
         return MPM_OK;
@@ -516,6 +536,64 @@ struct nclr_mpm_sim {
                                                       " is stopped (out_of_range); the adjoint needs every scene live: "
                                                       "set or load a state first");
         return MPM_OK;
+    }
+
+    struct HostPart {
+        void* host;  // nullptr: skipped
+        size_t bytes;
+    };
+    // sync(), then an export on the device (written by work already queued) -> the caller's arrays,
+    // its consecutive parts.  Nothing is written if sync() fails.
+    int read_back(const void* device, std::initializer_list<HostPart> parts) {
+        size_t bytes = 0;
+        for (const auto& q : parts) bytes += q.bytes;
+        const bool staged = bytes <= kReadBlock;
+        if (staged && bytes > host_read_bytes) {
+            if (host_read) HIP_TRY(hipHostFree(host_read));
+            host_read = nullptr;
+            host_read_bytes = 0;
+            HIP_TRY(hipHostMalloc(reinterpret_cast<void**>(&host_read), bytes, 0));
+            host_read_bytes = bytes;
+        }
+        if (staged && bytes) HIP_TRY(hipMemcpyAsync(host_read, device, bytes, hipMemcpyDeviceToHost, stream));
+        RC_TRY(sync());
+        size_t at = 0;
+        for (const auto& q : parts) {
+            if (q.host && q.bytes) {
+                if (staged) std::memcpy(q.host, host_read + at, q.bytes);
+                else HIP_TRY(hipMemcpyAsync(q.host, static_cast<const char*>(device) + at, q.bytes,
+                                            hipMemcpyDeviceToHost, stream));
+            }
+            at += q.bytes;
+        }
+        if (!staged) HIP_TRY(hipStreamSynchronize(stream));
+        return MPM_OK;
+    }
+
+    int get_particles(float* x, float* v, float* F, float* C, float* Jp, float* mass, float* volume) {
+        HIP_TRY(hipSetDevice(opts.device));
+        const size_t n = size_t(p.n), f = sizeof(float), d = size_t(dim);
+        float* out = state[cur ^ 1];  // free between steps
+        HIP_TRY(nclr_host::launch_particles_out(dim, state[cur], pid[cur], p.n, p.stride, out, stream));
+        return read_back(out, {{x, n * d * f}, {v, n * d * f}, {F, n * d * d * f}, {C, n * d * d * f}, {Jp, n * f},
+                               {mass, n * f}, {volume, n * f}});
+    }
+
+    int get_grid(int scene, float* velocity, float* mass) {
+        HIP_TRY(hipSetDevice(opts.device));
+        const auto& sp = scenes[size_t(scene)];
+        const int64_t total = scene_nodes(scene), floats = total * (dim + 1);
+        if (floats > grid_out_floats) {
+            if (grid_out) HIP_TRY(hipFree(grid_out));
+            grid_out = nullptr;
+            grid_out_floats = 0;
+            HIP_TRY(dmalloc(&grid_out, size_t(floats)));
+            grid_out_floats = floats;
+        }
+        HIP_TRY(nclr_host::launch_export_grid(args(cur), scene, sp.res, sp.node_tile_base, sp.ntn, grid_out,
+                                              grid_out + total * dim, total));
+        return read_back(grid_out, {{velocity, size_t(total) * size_t(dim) * sizeof(float)},
+                                    {mass, size_t(total) * sizeof(float)}});
     }
 
     // Device state -> host SoA image (physical slot order) and the slot -> particle map.
@@ -1111,11 +1189,10 @@ struct nclr_mpm_sim {
     int set_elasticity(int s, float E, float nu) {
         if (!(std::isfinite(E) && std::isfinite(nu)) || nu <= -1.0f || nu >= 0.5f)
             return fail(MPM_ERR_INVALID, "E must be finite and nu in (-1, 0.5)");
-        HIP_TRY(hipStreamSynchronize(stream));
         auto& sp = scenes[size_t(s)];
         set_scene_elasticity(sp, E, nu);
-        HIP_TRY(hipMemcpyAsync(d_scenes + s, &sp, sizeof(sp), hipMemcpyHostToDevice, stream));
-        HIP_TRY(hipStreamSynchronize(stream));
+        // in the stream's order, the values in the launch: no wait (a batch sets its scenes one by one)
+        HIP_TRY(nclr_host::launch_set_scene(d_scenes + s, sp, stream));
         return MPM_OK;
     }
 
@@ -1136,10 +1213,17 @@ struct nclr_mpm_sim {
                         hist,     slots, gv, stamps, status,
                         active,   active_sum, stamp,    d_scenes, slots_b, gbar, epart, erange, epartial, gtmp[0],
                         gtmp[1],  tape,       sort_tape, uidx,     ucnt,        upref, ttotal, rtot, line_changes, off_grid,
-                        tile_scene, node_tile_scene, scene_flags, scene_frozen, cslots, cgrid, cmassive, cbox, cinfo,
+                        tile_scene, node_tile_scene, grid_out, cslots, cgrid, cmassive, cbox, cinfo,
                         csubbox, cbar};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
+        if (host_words) (void)hipHostFree(host_words);
+        if (host_read) (void)hipHostFree(host_read);
+        host_words = nullptr;
+        host_read = nullptr;
+        host_read_bytes = 0;
+        grid_out = nullptr;
+        grid_out_floats = 0;
         uidx = ucnt = upref = ttotal = meta = rtot = nullptr;
         p.items = nullptr;
         tile_scene = node_tile_scene = nullptr;
@@ -1281,14 +1365,13 @@ int create_impl(int dim, int nscenes, const mpm_scene* sc, const float* x, const
         dmalloc(&h->hist, size_t(256) * size_t(nclr_host::sort_tiles(int64_t(nn))) + 256) != hipSuccess ||
         dmalloc(&h->slots, slot_nodes) != hipSuccess ||
         dmalloc(&h->gv, gv_nodes) != hipSuccess || dmalloc(&h->stamps, size_t(node_tiles)) != hipSuccess ||
-        dmalloc(&h->status, 1) != hipSuccess || dmalloc(&h->active, size_t(node_tiles)) != hipSuccess ||
+        h->alloc_words(size_t(nscenes)) != hipSuccess || dmalloc(&h->active, size_t(node_tiles)) != hipSuccess ||
         dmalloc(&h->active_sum, 1) != hipSuccess || dmalloc(&h->stamp, 1) != hipSuccess ||
         dmalloc(&h->d_scenes, size_t(nscenes)) != hipSuccess || dmalloc(&h->uidx, nn) != hipSuccess ||
         dmalloc(&h->ucnt, bucket_cells) != hipSuccess || dmalloc(&h->upref, bucket_cells) != hipSuccess ||
         dmalloc(&h->ttotal, nbins) != hipSuccess ||
         dmalloc(&h->rtot, 2 * (size_t(tiles) / nclr_dev::kScanRound + 2)) != hipSuccess ||
-        dmalloc(&h->line_changes, 1) != hipSuccess || dmalloc(&h->off_grid, size_t(nscenes)) != hipSuccess ||
-        dmalloc(&h->scene_flags, size_t(nscenes)) != hipSuccess || dmalloc(&h->scene_frozen, size_t(nscenes)) != hipSuccess)
+        dmalloc(&h->line_changes, 1) != hipSuccess || dmalloc(&h->off_grid, size_t(nscenes)) != hipSuccess)
         return cleanup(fail(MPM_ERR_HIP, "hipMalloc failed (out of device memory?)"));
     p.scenes = h->d_scenes;
     p.stamp = h->stamp;
@@ -1402,28 +1485,7 @@ int mpm_scene_status(mpm_handle h, uint32_t* flags, int64_t* failed_step) {
 int mpm_get_particles(mpm_handle h, float* x, float* v, float* F, float* C, float* Jp, float* mass,
                       float* volume) {
     if (!h) return fail(MPM_ERR_INVALID, "NULL handle");
-    RC_TRY(h->sync());
-    std::vector<float> host;
-    std::vector<uint32_t> ids;
-    RC_TRY(h->download(host, ids));
-    h->unpermute(host, ids);
-    const int D = h->dim;
-    const int64_t n = h->p.n, stride = h->p.stride;
-    const int fX = 0, fV = D, fF = 2 * D, fC = 2 * D + D * D, fJ = 2 * D + 2 * D * D;
-    for (int64_t i = 0; i < n; ++i) {
-        for (int a = 0; a < D; ++a) {
-            if (x) x[i * D + a] = host[(fX + a) * stride + i];
-            if (v) v[i * D + a] = host[(fV + a) * stride + i];
-        }
-        for (int k = 0; k < D * D; ++k) {
-            if (F) F[i * D * D + k] = host[(fF + k) * stride + i];
-            if (C) C[i * D * D + k] = host[(fC + k) * stride + i];
-        }
-        if (Jp) Jp[i] = host[fJ * stride + i];
-        if (mass) mass[i] = host[(fJ + 1) * stride + i];
-        if (volume) volume[i] = host[(fJ + 2) * stride + i];
-    }
-    return MPM_OK;
+    return h->get_particles(x, v, F, C, Jp, mass, volume);
 }
 
 int mpm_set_particles(mpm_handle h, const float* x, const float* v, const float* F, const float* C,
@@ -1440,27 +1502,7 @@ int mpm_set_particles(mpm_handle h, const float* x, const float* v, const float*
 int mpm_get_grid_scene(mpm_handle h, int scene, float* velocity, float* mass) {
     if (!h) return fail(MPM_ERR_INVALID, "NULL handle");
     if (scene < 0 || scene >= int(h->scenes.size())) return fail(MPM_ERR_INVALID, "scene index out of range");
-    RC_TRY(h->sync());
-    const auto& sp = h->scenes[size_t(scene)];
-    const int64_t total = h->scene_nodes(scene);
-    float* dvel = nullptr;
-    float* dmass = nullptr;
-    HIP_TRY(dmalloc(&dvel, size_t(total) * h->dim));
-    if (dmalloc(&dmass, size_t(total)) != hipSuccess) {
-        (void)hipFree(dvel);
-        return fail(MPM_ERR_HIP, "hipMalloc failed");
-    }
-    hipError_t e = nclr_host::launch_export_grid(h->args(h->cur), scene, sp.res, sp.node_tile_base, sp.ntn, dvel,
-                                                 dmass, total);
-    if (e == hipSuccess && velocity)
-        e = hipMemcpyAsync(velocity, dvel, size_t(total) * h->dim * sizeof(float), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess && mass)
-        e = hipMemcpyAsync(mass, dmass, size_t(total) * sizeof(float), hipMemcpyDeviceToHost, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    (void)hipFree(dvel);
-    (void)hipFree(dmass);
-    if (e != hipSuccess) return fail(MPM_ERR_HIP, std::string("grid export: ") + hipGetErrorString(e));
-    return MPM_OK;
+    return h->get_grid(scene, velocity, mass);
 }
 
 int mpm_get_grid(mpm_handle h, float* velocity, float* mass) { return mpm_get_grid_scene(h, 0, velocity, mass); }
@@ -1685,6 +1727,26 @@ int mpm_grad_from_particle_order(mpm_handle h, const float* src, float* dst) {
     HIP_TRY(hipSetDevice(h->opts.device));
     HIP_TRY(nclr_host::launch_permute_channels(h->pid[h->cur], src, h->p.n, dst, h->p.n, h->grad_channels(), h->p.n,
                                                false, h->state[h->cur ^ 1], h->line_changes, h->stream));
+    return MPM_OK;
+}
+
+int64_t mpm_order_bytes(mpm_handle h) { return h ? int64_t(size_t(h->p.stride) * sizeof(uint32_t)) : -1; }
+
+int mpm_save_order(mpm_handle h, void* dst) {
+    if (!h || !dst) return fail(MPM_ERR_INVALID, "NULL argument");
+    HIP_TRY(hipSetDevice(h->opts.device));
+    HIP_TRY(hipMemcpyAsync(dst, h->pid[h->cur], size_t(h->p.stride) * sizeof(uint32_t), hipMemcpyDeviceToDevice,
+                           h->stream));
+    return MPM_OK;
+}
+
+int mpm_grad_to_saved_order(mpm_handle h, const void* order, const float* src, float* dst) {
+    if (!h || !order || ((!src || !dst) && h->p.n > 0)) return fail(MPM_ERR_INVALID, "NULL argument");
+    if (src == dst && h->p.n > 0) return fail(MPM_ERR_INVALID, "src and dst must not alias");
+    HIP_TRY(hipSetDevice(h->opts.device));
+    HIP_TRY(nclr_host::launch_permute_channels(static_cast<const uint32_t*>(order), src, h->p.n, dst, h->p.n,
+                                               h->grad_channels(), h->p.n, false, h->state[h->cur ^ 1],
+                                               h->line_changes, h->stream));
     return MPM_OK;
 }
 

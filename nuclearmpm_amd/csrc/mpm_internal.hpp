@@ -227,6 +227,10 @@ hipError_t launch_p2g_adjoint(const LaunchArgs& a, const AdjointArgs& b);
 hipError_t launch_permute_channels(const uint32_t* pid, const float* src, int64_t src_stride, float* dst,
                                    int64_t dst_stride, int channels, int64_t n, bool to_particle_order, float* rows,
                                    uint32_t* changes, hipStream_t s);
+// A state in slot order as particle-major arrays in particle order, one behind the other (n of each): x, v, F, C,
+// Jp, mass, volume.
+hipError_t launch_particles_out(int dim, const float* st, const uint32_t* pid, int64_t n, int64_t stride, float* out,
+                                hipStream_t s);
 // A large state image is stored in tile order when it is set: its keys and cleared tile bounds
 // (into the radix sort's input), and after launch_key_sort the slots from the sorted order.  a.state_in / a.pid_in:
 // the state before, whose constants (mass, volume) the new one keeps and whose buffer is scratch.
@@ -253,6 +257,7 @@ hipError_t launch_svd(int dim, int mode, const float* A, float* U, float* S, flo
 hipError_t launch_fill_u32(uint32_t* p, int64_t n, uint32_t value, hipStream_t s);
 hipError_t launch_iota_u32(uint32_t* p, int64_t n, hipStream_t s);
 hipError_t launch_bump_u32(uint32_t* p, hipStream_t s);  // *p += 1 on the device
+hipError_t launch_set_scene(nclr_dev::SceneParams* dst, const nclr_dev::SceneParams& sp, hipStream_t s);
 hipError_t launch_zero_f4(float4* p, int64_t n, hipStream_t s);
 hipError_t launch_active_sum(const LaunchArgs& a, uint32_t first_tile, uint32_t tiles, unsigned long long* out);
 // Stable sort by the low `bits` bits of n keys that lie in radix_keys_in(keys, keys_tmp, bits) (the pass

@@ -16,6 +16,8 @@
 // 3.13 -> 2.37 ms.
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "mpm_device.hpp"
 
 namespace nclr_dev {
@@ -181,6 +183,32 @@ __global__ __launch_bounds__(256) void k_sorted_step(StepParams p, uint32_t* __r
     list_grid_tile<D>(p, stops ? p.node_tiles : uint32_t(t), item_offset, tiles, &meta[kMetaGridTiles], active);
 }
 
+// Slots -> particle-major arrays in particle order, for the host: the device does the reordering and the
+// transposition, so that the host only copies.
+template <int D>
+__global__ __launch_bounds__(256) void k_particles_out(const float* __restrict__ st, const uint32_t* __restrict__ pid,
+                                                       int64_t n, int64_t stride, float* __restrict__ out) {
+    const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const int64_t to = pid[i];
+    if (to >= n) return;
+    int row = 0;
+    auto put = [&](auto width) {
+        constexpr int K = decltype(width)::value;
+#pragma unroll
+        for (int k = 0; k < K; ++k) out[row * n + to * K + k] = st[(row + k) * stride + i];
+        row += K;
+    };
+    using std::integral_constant;
+    put(integral_constant<int, D>{});      // x
+    put(integral_constant<int, D>{});      // v
+    put(integral_constant<int, D * D>{});  // F
+    put(integral_constant<int, D * D>{});  // C
+    put(integral_constant<int, 1>{});      // Jp
+    put(integral_constant<int, 1>{});      // mass
+    put(integral_constant<int, 1>{});      // volume
+}
+
 }  // namespace nclr_dev
 
 namespace nclr_host {
@@ -223,6 +251,14 @@ hipError_t launch_sorted_step(const LaunchArgs& a) {
     else
         k_sorted_step<3><<<b, 256, 0, a.stream>>>(a.p, a.stamp, a.off_grid, a.item_offset,
                                                   static_cast<GridTile<3>*>(a.grid_tiles), a.meta, a.active, list);
+    return hipGetLastError();
+}
+
+hipError_t launch_particles_out(int dim, const float* st, const uint32_t* pid, int64_t n, int64_t stride, float* out,
+                                hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    if (dim == 2) k_particles_out<2><<<blocks_of(n, 256), 256, 0, s>>>(st, pid, n, stride, out);
+    else k_particles_out<3><<<blocks_of(n, 256), 256, 0, s>>>(st, pid, n, stride, out);
     return hipGetLastError();
 }
 

@@ -576,6 +576,8 @@ namespace nclr_dev {
 
 __global__ void k_bump_u32(uint32_t* __restrict__ p) { *p = *p + 1u; }
 
+__global__ void k_set_scene(SceneParams* __restrict__ dst, SceneParams sp) { *dst = sp; }
+
 }  // namespace nclr_dev
 
 namespace nclr_host {
@@ -755,6 +757,11 @@ hipError_t launch_fill_u32(uint32_t* p, int64_t n, uint32_t value, hipStream_t s
 
 hipError_t launch_bump_u32(uint32_t* p, hipStream_t s) {
     k_bump_u32<<<1, 1, 0, s>>>(p);
+    return hipGetLastError();
+}
+
+hipError_t launch_set_scene(SceneParams* dst, const SceneParams& sp, hipStream_t s) {
+    k_set_scene<<<1, 1, 0, s>>>(dst, sp);
     return hipGetLastError();
 }
 

@@ -193,3 +193,61 @@ def test_large_state_images_in_any_order(dim, n, mixed):
         b.set_state_image(image)
         b.advance(1)
         b.synchronize()
+
+
+@pytest.mark.parametrize("n,res", [(0, 20), (1, 20), (777, 79), (77_672, 79), (77_673, 80)])
+def test_host_reads_on_both_sides_of_the_pinned_size(n, res):
+    """Particle arrays and grids up to 8 MiB are read through pinned memory (77,672 3D particles, res 79)."""
+    import torch
+
+    p = _cloud(3, n, 11)
+    p.mass = np.linspace(1.0, 2.0, n, dtype=np.float32)
+    p.volume = np.linspace(2.0, 3.0, n, dtype=np.float32)
+    with MPMSimulation(p, MaterialModel.kJelly, res, E=1e3, identity_mode=1) as sim:
+        sim.advance(2)
+        for _ in range(2):  # a first read and one with the buffers kept
+            sim._cache = None
+            got, (vel, mass) = sim.particles(), sim.grid()
+            image = sim.state_image().cpu() if n else torch.empty(25, 0)
+            rows = [getattr(got, k).reshape(n, w) for k, w in (("x", 3), ("v", 3), ("F", 9), ("C", 9), ("Jp", 1))]
+            assert np.array_equal(np.concatenate(rows, 1).T, image.numpy())
+            assert np.array_equal(got.mass, p.mass) and np.array_equal(got.volume, p.volume)
+            # mass on the nodes: n sums of 27 weights, each rounded; empty nodes carry neither mass nor velocity
+            assert mass.shape == (res + 1,) * 3 and vel.shape == (res + 1,) * 3 + (3,)
+            assert abs(float(mass.sum(dtype=np.float64)) - float(p.mass.sum(dtype=np.float64))) <= 1e-5 * n
+            assert not vel[mass == 0].any()
+        assert sim.active_nodes() == int((mass > 0).sum())
+
+
+def test_queued_elasticity_and_saved_order():
+    """set_elasticity between queued steps takes effect in their order, and a cotangent goes to a saved slot order as
+    it did while that order was the current one."""
+    import torch
+
+    from nuclearmpm_amd._lib import check, lib
+
+    a, b = _cloud(3, 5000, 3), _cloud(3, 3001, 4)
+    specs = [SceneSpec(a, MaterialModel.kJelly, 40), SceneSpec(b, MaterialModel.kJelly, 40)]
+    out = []
+    for wait in (False, True):
+        with MPMBatch(specs, identity_mode=1) as sim:
+            for k in range(4):
+                sim.advance(1)
+                for s in range(2):
+                    sim.set_elasticity(s, 1e3 * (1 + k + 5 * s))
+                    if wait:
+                        sim.synchronize()
+            out.append(sim.state_image())
+            if wait:
+                L, h, n = lib(), sim._handle(), sim.n
+                order = torch.empty(int(L.mpm_order_bytes(h)), dtype=torch.uint8, device="cuda")
+                cot = torch.randn(25, n, device="cuda")
+                now, later = torch.empty_like(cot), torch.empty_like(cot)
+                torch.cuda.synchronize()
+                check(L.mpm_save_order(h, order.data_ptr()))
+                check(L.mpm_grad_from_particle_order(h, cot.data_ptr(), now.data_ptr()))
+                sim.advance(3)
+                check(L.mpm_grad_to_saved_order(h, order.data_ptr(), cot.data_ptr(), later.data_ptr()))
+                sim.synchronize()
+                assert torch.equal(now, later) and not torch.equal(now, cot)
+    assert torch.equal(out[0], out[1])
