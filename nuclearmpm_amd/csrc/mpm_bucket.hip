@@ -8,12 +8,18 @@
 //
 //   count    one workgroup per old work item: each particle's new key and neighbour offset
 //            o = new - old (or the off-grid bucket), its rank among the item's particles with the
-//            same offset (in slot order), and the item's count per offset
-//   prefix   one wave per new tile: its <= 3^D source tiles in increasing order, and their items
-//            in order, give each (item, offset) the number of earlier particles bound for the tile
-//   scan     one workgroup: bucket starts (exclusive scan of the tile totals) and the P2G work
-//            items of the new order
+//            same offset (in slot order), the item's count per offset, and the new tiles' totals
+//            (integer atomics, at most one per item and offset)
+//   tables   in one launch, since the totals are there already: bucket starts (exclusive scan of the
+//            tile totals) and the P2G work items of the new order, one workgroup per kScanRound tiles;
+//            and, one wave per new tile, its <= 3^D source tiles in increasing order, and their
+//            items in order, give each (item, offset) the number of earlier particles bound for the tile
 //   scatter  per slot: position = start[new tile] + prefix[item][offset] + rank -> perm, keys
+//
+// Every kernel here takes 3.5 to 5 us up to some 10^5 particles, whatever it does, so launches count.
+// With the totals taken by the prefix waves, the scan waited for them in a launch of its own (two
+// beyond one round): the sort of 30,011 liquid particles 16.4 -> 12.9 us (a step 60 -> 55), of 150,003
+// jelly 19 -> 14.8, of 19,600 in 2D 15.6 -> 11.6, of 256 2D scenes (1.75M particles) 46 -> 39.
 //
 // Positions follow slot order within every tile's bucket, i.e. for particles on their grid the
 // result is the stable sort by key of the current order, identical to the radix sort's
@@ -41,18 +47,34 @@ NCLR_DI int offset_index(const int (&delta)[D]) {
     return o;
 }
 
+// Tile of offset index o relative to its source tile's.
+template <int D>
+NCLR_DI int64_t tile_step(int o, int nt) {
+    int64_t t = 0, stride = 1;
+#pragma unroll
+    for (int a = D - 1; a >= 0; --a) {
+        t += (o % 3 - 1) * stride;
+        o /= 3;
+        stride *= nt;
+    }
+    return t;
+}
+
 template <int D>
 __global__ __launch_bounds__(256) void k_bucket_count(const float* __restrict__ st, StepParams p,
                                                       uint32_t* __restrict__ stamp,
                                                       const uint32_t* __restrict__ item_offset,
                                                       uint32_t* __restrict__ newkey, uint32_t* __restrict__ rankpk,
                                                       uint32_t* __restrict__ uidx, uint32_t* __restrict__ ucnt,
-                                                      uint32_t* __restrict__ status) {
+                                                      uint32_t* __restrict__ old_offset,
+                                                      uint32_t* __restrict__ ttotal) {
     using B = Buckets<D>;
     __shared__ uint32_t running[B::NO];
     __shared__ uint32_t wave_count[4][B::NO];
     const uint32_t item = blockIdx.x;
     if (item == 0 && threadIdx.x == 0) *stamp = *stamp + 1u;
+    // the old order's item offsets, for the prefix waves: the tables may be written over the old ones
+    if (threadIdx.x == 0 && item <= p.ntiles) old_offset[item] = item_offset[item];
     const WorkItem wi = work_item(p, item);  // loaded with the count below, used only if valid
     if (item >= item_offset[p.ntiles]) return;
     for (int o = threadIdx.x; o < B::NO; o += blockDim.x) {
@@ -139,18 +161,20 @@ __global__ __launch_bounds__(256) void k_bucket_count(const float* __restrict__ 
         }
         __syncthreads();
     }
-    for (int o = threadIdx.x; o < B::NO; o += blockDim.x) ucnt[int64_t(item) * B::NO + o] = running[o];
+    for (int o = threadIdx.x; o < B::NO; o += blockDim.x) {
+        const uint32_t c = running[o];
+        ucnt[int64_t(item) * B::NO + o] = c;
+        if (o != B::OFF && c != 0u) atomicAdd(&ttotal[int64_t(tile) + tile_step<D>(o, sp.nt)], c);
+    }
 }
 
 // One wave per new tile k, lane s < 3^D for the source tile kc + d(s) - 1 (d(s) the base-3 digits
 // of s, so that increasing s is increasing source tile): each lane sums its source's items bound
 // for k, a wave scan orders the sources, and each lane then writes its items' prefixes in order.
 template <int D>
-__global__ __launch_bounds__(256) void k_bucket_prefix(StepParams p, const uint32_t* __restrict__ item_offset,
-                                                       const uint32_t* __restrict__ ucnt,
-                                                       uint32_t* __restrict__ upref, uint32_t* __restrict__ ttotal) {
+NCLR_DI void bucket_prefix(const StepParams& p, int64_t k, const uint32_t* __restrict__ item_offset,
+                           const uint32_t* __restrict__ ucnt, uint32_t* __restrict__ upref) {
     using B = Buckets<D>;
-    const int64_t k = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) >> 6;
     const int s = threadIdx.x & 63;
     if (k >= int64_t(p.ntiles)) return;  // whole waves
     const SceneParams sp = p.scenes[p.nscenes == 1 ? 0 : scene_of_tile(p, uint32_t(k))];
@@ -204,8 +228,6 @@ __global__ __launch_bounds__(256) void k_bucket_prefix(StepParams p, const uint3
         upref[int64_t(u) * B::NO + o] = run;
         run += cnt[int64_t(u) * B::NO];
     }
-    const uint32_t total = __shfl(x, B::NEIGH - 1);
-    if (s == 0) ttotal[k] = total;
 }
 
 // Bucket starts (exclusive scan of the tile totals) and the P2G work items of the new order.  On
@@ -216,9 +238,9 @@ __global__ __launch_bounds__(256) void k_bucket_prefix(StepParams p, const uint3
 // no part in P2G and G2P copies them unchanged, so their order within the last bucket cannot
 // affect any result; they are placed by an atomic counter.
 //
-// Up to kScanRound tiles: k_bucket_scan, one workgroup.  More: k_bucket_round_totals and
-// k_bucket_rounds, one workgroup per round of kScanRound tiles (totals, then each round with the
-// sum of the earlier rounds' totals as its carry); the results are the same.
+// One workgroup per round of kScanRound tiles; its carry is the sum of the earlier tiles' totals, which
+// it reads again (16 bytes a thread and round: the last of 71 rounds, 8 scenes of res 128, is done
+// long before the prefix waves of the same launch).
 struct BucketVisit {
     uint32_t *tile_start, *tile_end, *item_offset;
     uint4* items;
@@ -231,64 +253,54 @@ struct BucketVisit {
     }
 };
 
-template <int D>
-__global__ __launch_bounds__(1024) void k_bucket_scan(StepParams p, uint32_t chunk,
-                                                      uint32_t* __restrict__ item_offset,
-                                                      uint32_t* __restrict__ tile_start,
-                                                      uint32_t* __restrict__ tile_end,
-                                                      const uint32_t* __restrict__ ttotal,
-                                                      const uint32_t* prev_meta, uint32_t* meta) {
-    __shared__ uint32_t s_seen;
-    if (threadIdx.x == 0) s_seen = prev_meta[0];
-    __syncthreads();  // meta (possibly the same buffer as prev_meta) is rewritten below
-    const BucketVisit visit{tile_start, tile_end, item_offset, p.items, chunk};
-    auto count = [&](uint32_t tile) { return ttotal[tile]; };
-    uint32_t cp = 0, ci = 0;
-    for (uint32_t b0 = 0; b0 < p.ntiles; b0 += kScanRound) {
-        uint32_t tp, ti;
-        scan_round(b0, p.ntiles, chunk, cp, ci, count, visit, tp, ti);
-        cp += tp;
-        ci += ti;
+NCLR_DI void bucket_tables(const StepParams& p, uint32_t round, uint32_t rounds, uint32_t chunk,
+                           uint32_t* __restrict__ item_offset, uint32_t* __restrict__ tile_start,
+                           uint32_t* __restrict__ tile_end, const uint32_t* __restrict__ ttotal,
+                           const uint32_t* prev_meta, uint32_t* meta) {
+    const uint32_t b0 = round * kScanRound;
+    uint32_t cp = 0, ci = 0, tp, ti;
+    if (round > 0) {
+        uint32_t sp = 0, si = 0, ep, ei;
+        auto add = [&](uint32_t c) {
+            sp += c;
+            si += (c + chunk - 1) / chunk;
+        };
+#pragma unroll 4
+        for (uint32_t t = uint32_t(threadIdx.x) * 4; t < b0; t += kScanRound) {
+            const uint4 c = *reinterpret_cast<const uint4*>(ttotal + t);
+            add(c.x);
+            add(c.y);
+            add(c.z);
+            add(c.w);
+        }
+        block_scan2(sp, si, ep, ei, cp, ci);
     }
-    if (threadIdx.x == 0) {
-        item_offset[p.ntiles] = ci;  // the total
-        meta[0] = cp;
+    const BucketVisit visit{tile_start, tile_end, item_offset, p.items, chunk};
+    scan_round(b0, p.ntiles, chunk, cp, ci, [&](uint32_t tile) { return ttotal[tile]; }, visit, tp, ti);
+    if (round + 1 == rounds && threadIdx.x == 0) {
+        item_offset[p.ntiles] = ci + ti;  // the total
+        const uint32_t seen = prev_meta[0];  // meta may be prev_meta
+        meta[0] = cp + tp;
         meta[1] = 0;
-        meta[2] = s_seen;
+        meta[2] = seen;
         meta[kMetaGridTiles] = 0;
     }
 }
 
-__global__ __launch_bounds__(1024) void k_bucket_round_totals(uint32_t ntiles, uint32_t chunk,
-                                                              const uint32_t* __restrict__ ttotal,
-                                                              uint32_t* __restrict__ rtot, const uint32_t* prev_meta,
-                                                              uint32_t* meta) {
-    uint32_t tp, ti;
-    round_totals(blockIdx.x, ntiles, chunk, [&](uint32_t tile) { return ttotal[tile]; }, tp, ti);
-    if (threadIdx.x == 0) {
-        rtot[2 * blockIdx.x] = tp;
-        rtot[2 * blockIdx.x + 1] = ti;
-        if (blockIdx.x == 0) meta[2] = prev_meta[0];
-    }
-}
-
 template <int D>
-__global__ __launch_bounds__(1024) void k_bucket_rounds(StepParams p, uint32_t chunk, uint32_t* __restrict__ item_offset,
+__global__ __launch_bounds__(1024) void k_bucket_tables(StepParams p, uint32_t rounds, uint32_t chunk,
+                                                        const uint32_t* __restrict__ old_offset,
+                                                        const uint32_t* __restrict__ ucnt,
+                                                        uint32_t* __restrict__ upref,
+                                                        uint32_t* __restrict__ item_offset,
                                                         uint32_t* __restrict__ tile_start,
                                                         uint32_t* __restrict__ tile_end,
                                                         const uint32_t* __restrict__ ttotal,
-                                                        const uint32_t* __restrict__ rtot, uint32_t* __restrict__ meta) {
-    uint32_t cp, ci, tp, ti;
-    round_carries(rtot, blockIdx.x, cp, ci);
-    const BucketVisit visit{tile_start, tile_end, item_offset, p.items, chunk};
-    scan_round(blockIdx.x * kScanRound, p.ntiles, chunk, cp, ci, [&](uint32_t tile) { return ttotal[tile]; }, visit,
-               tp, ti);
-    if (threadIdx.x == 0 && blockIdx.x + 1 == gridDim.x) {
-        item_offset[p.ntiles] = ci + ti;
-        meta[0] = cp + tp;
-        meta[1] = 0;
-        meta[kMetaGridTiles] = 0;
-    }
+                                                        const uint32_t* prev_meta, uint32_t* meta) {
+    if (blockIdx.x < rounds)
+        bucket_tables(p, blockIdx.x, rounds, chunk, item_offset, tile_start, tile_end, ttotal, prev_meta, meta);
+    else
+        bucket_prefix<D>(p, int64_t(blockIdx.x - rounds) * 16 + (threadIdx.x >> 6), old_offset, ucnt, upref);
 }
 
 template <int D>
@@ -303,8 +315,11 @@ __global__ __launch_bounds__(256) void k_bucket_scatter(StepParams p, const uint
                                                         uint32_t list_blocks,
                                                         const uint32_t* __restrict__ item_offset,
                                                         GridTile<D>* __restrict__ tiles,
-                                                        uint32_t* __restrict__ active) {
+                                                        uint32_t* __restrict__ active,
+                                                        uint32_t* __restrict__ ttotal) {
     using B = Buckets<D>;
+    // the next sort counts from zero
+    for (uint32_t t = blockIdx.x * 256 + threadIdx.x; t < p.ntiles; t += gridDim.x * 256) ttotal[t] = 0;
     if (blockIdx.x < list_blocks) {  // the first workgroups list the node tiles (a chain of dependent
                                      // loads: behind the particles' workgroups it made a tail of 4 us)
         list_grid_tile<D>(p, blockIdx.x * 256 + threadIdx.x, item_offset, tiles, &meta[kMetaGridTiles], active);
@@ -344,32 +359,23 @@ template <int D>
 static hipError_t bucket_dispatch(const LaunchArgs& a) {
     const auto& p = a.p;
     hipStream_t s = a.stream;
-    const int64_t items = max_items(p.n, p.ntiles);
-    // the old order's work items (the previous sort's block) are read by the count and prefix
-    // kernels; the scans write the new ones (into the same block or another)
+    // the old order's work items (the previous sort's block) are read by the count; the tables are
+    // the new ones (in the same block or another).  A workgroup per item there may be, and per old offset.
+    const int64_t items = std::max<int64_t>(max_items(p.n, p.ntiles), int64_t(p.ntiles) + 1);
     StepParams prev = p;
     prev.items = const_cast<uint4*>(a.prev_items);
-    k_bucket_count<D><<<unsigned(std::max<int64_t>(items, 1)), 256, 0, s>>>(
-        a.state_in, prev, a.stamp, a.prev_item_offset, a.keys_tmp, a.perm_tmp, a.uidx, a.ucnt, a.status);
-    if (p.ntiles > 0)
-        k_bucket_prefix<D><<<unsigned((int64_t(p.ntiles) + 3) / 4), 256, 0, s>>>(p, a.prev_item_offset, a.ucnt,
-                                                                                a.upref, a.ttotal);
+    k_bucket_count<D><<<unsigned(items), 256, 0, s>>>(a.state_in, prev, a.stamp, a.prev_item_offset, a.keys_tmp,
+                                                      a.perm_tmp, a.uidx, a.ucnt, a.old_offset, a.ttotal);
     const uint32_t rounds = (p.ntiles + kScanRound - 1) / kScanRound;
-    if (rounds <= 1) {
-        k_bucket_scan<D><<<1, 1024, 0, s>>>(p, uint32_t(p.chunk), a.item_offset, a.tile_start, a.tile_end, a.ttotal,
-                                            a.prev_meta, a.meta);
-    } else {
-        k_bucket_round_totals<<<rounds, 1024, 0, s>>>(p.ntiles, uint32_t(p.chunk), a.ttotal, a.rtot, a.prev_meta,
-                                                      a.meta);
-        k_bucket_rounds<D><<<rounds, 1024, 0, s>>>(p, uint32_t(p.chunk), a.item_offset, a.tile_start, a.tile_end,
-                                                   a.ttotal, a.rtot, a.meta);
-    }
+    k_bucket_tables<D><<<rounds + (p.ntiles + 15) / 16, 1024, 0, s>>>(p, rounds, uint32_t(p.chunk), a.old_offset,
+                                                                      a.ucnt, a.upref, a.item_offset, a.tile_start,
+                                                                      a.tile_end, a.ttotal, a.prev_meta, a.meta);
     const unsigned pb = unsigned((p.n + 255) / 256);
     const unsigned tb = grid_tiles_listed(D, p) ? (p.node_tiles + 255) / 256 : 0;
     if (pb + tb > 0)
-        k_bucket_scatter<D><<<pb + tb, 256, 0, s>>>(p, a.keys_tmp, a.perm_tmp, a.uidx, a.upref, a.tile_start, a.pid_in,
+        k_bucket_scatter<D><<<std::max(pb + tb, (p.ntiles + 1023) / 1024), 256, 0, s>>>(p, a.keys_tmp, a.perm_tmp, a.uidx, a.upref, a.tile_start, a.pid_in,
                                                     a.meta, a.perm, a.keys, a.status, tb, a.item_offset,
-                                                    static_cast<GridTile<D>*>(a.grid_tiles), a.active);
+                                                    static_cast<GridTile<D>*>(a.grid_tiles), a.active, a.ttotal);
     return hipGetLastError();
 }
 

@@ -100,7 +100,7 @@ struct nclr_mpm_sim {
     unsigned long long* active_sum = nullptr;
     // incremental sort: valid while the state is stored in the order of the last sort and the
     // tile bounds / work items of that sort are intact (cleared by uploads, loads, re-tuning)
-    uint32_t *uidx = nullptr, *ucnt = nullptr, *upref = nullptr, *ttotal = nullptr, *meta = nullptr;
+    uint32_t *uidx = nullptr, *ucnt = nullptr, *upref = nullptr, *ttotal = nullptr, *old_offset = nullptr, *meta = nullptr;
     uint32_t* rtot = nullptr;
     uint32_t* line_changes = nullptr;  // one word: how incoherent an order is (mpm_order.hip)
     uint32_t *tile_scene = nullptr, *node_tile_scene = nullptr;  // scene maps (batches only)
@@ -209,6 +209,7 @@ struct nclr_mpm_sim {
         a.ucnt = ucnt;
         a.upref = upref;
         a.ttotal = ttotal;
+        a.old_offset = old_offset;
         a.meta = meta;
         a.grid_tiles = grid_tiles;
         a.rtot = rtot;
@@ -1212,7 +1213,7 @@ struct nclr_mpm_sim {
         void* bufs[] = {state[0], state[1], pid[0],  pid[1],   sort_block, keys_tmp, perm_tmp,
                         hist,     slots, gv, stamps, status,
                         active,   active_sum, stamp,    d_scenes, slots_b, gbar, epart, erange, epartial, gtmp[0],
-                        gtmp[1],  tape,       sort_tape, uidx,     ucnt,        upref, ttotal, rtot, line_changes, off_grid,
+                        gtmp[1],  tape,       sort_tape, uidx,     ucnt,        upref, ttotal, old_offset, rtot, line_changes, off_grid,
                         tile_scene, node_tile_scene, grid_out, cslots, cgrid, cmassive, cbox, cinfo,
                         csubbox, cbar};
         for (void* b : bufs)
@@ -1224,7 +1225,7 @@ struct nclr_mpm_sim {
         host_read_bytes = 0;
         grid_out = nullptr;
         grid_out_floats = 0;
-        uidx = ucnt = upref = ttotal = meta = rtot = nullptr;
+        uidx = ucnt = upref = ttotal = old_offset = meta = rtot = nullptr;
         p.items = nullptr;
         tile_scene = node_tile_scene = nullptr;
         scene_flags = scene_frozen = nullptr;
@@ -1369,7 +1370,7 @@ int create_impl(int dim, int nscenes, const mpm_scene* sc, const float* x, const
         dmalloc(&h->active_sum, 1) != hipSuccess || dmalloc(&h->stamp, 1) != hipSuccess ||
         dmalloc(&h->d_scenes, size_t(nscenes)) != hipSuccess || dmalloc(&h->uidx, nn) != hipSuccess ||
         dmalloc(&h->ucnt, bucket_cells) != hipSuccess || dmalloc(&h->upref, bucket_cells) != hipSuccess ||
-        dmalloc(&h->ttotal, nbins) != hipSuccess ||
+        dmalloc(&h->ttotal, nbins) != hipSuccess || dmalloc(&h->old_offset, nbins) != hipSuccess ||
         dmalloc(&h->rtot, 2 * (size_t(tiles) / nclr_dev::kScanRound + 2)) != hipSuccess ||
         dmalloc(&h->line_changes, 1) != hipSuccess || dmalloc(&h->off_grid, size_t(nscenes)) != hipSuccess)
         return cleanup(fail(MPM_ERR_HIP, "hipMalloc failed (out of device memory?)"));
@@ -1402,6 +1403,7 @@ int create_impl(int dim, int nscenes, const mpm_scene* sc, const float* x, const
         nclr_host::launch_fill_u32(h->stamps, int64_t(node_tiles), 0u, h->stream) != hipSuccess ||
         nclr_host::launch_fill_u32(h->stamp, 1, 0u, h->stream) != hipSuccess ||
         nclr_host::launch_fill_u32(h->status, 1, 0u, h->stream) != hipSuccess ||
+        nclr_host::launch_fill_u32(h->ttotal, int64_t(nbins), 0u, h->stream) != hipSuccess ||
         nclr_host::launch_fill_u32(h->active, int64_t(node_tiles), 0u, h->stream) != hipSuccess ||
         nclr_host::launch_fill_u32(h->pid[1], p.stride, 0u, h->stream) != hipSuccess)
         return cleanup(fail(MPM_ERR_HIP, "device initialisation failed"));

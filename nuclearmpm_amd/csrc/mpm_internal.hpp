@@ -188,10 +188,11 @@ struct LaunchArgs {
     uint32_t* uidx;            // n: old work item of each slot
     uint32_t* ucnt;            // max_items * offsets: per old item, particles per neighbour offset
     uint32_t* upref;           // max_items * offsets: per (old item, offset), earlier particles bound alike
-    uint32_t* ttotal;          // ntiles: particles per new tile
+    uint32_t* ttotal;          // ntiles: particles per new tile (zero between sorts)
+    uint32_t* old_offset;      // ntiles + 1: the old order's item offsets
     uint32_t* meta;            // 4 counters
     void* grid_tiles;          // node_tiles GridTile<dim>: the node tiles the sorted particles reach (meta[kMetaGridTiles])
-    uint32_t* rtot;            // 2 per round of the tile scans: particle and work-item totals
+    uint32_t* rtot;            // 2 per round of the radix sort's tile scan: particle and work-item totals
     // the incremental sort's inputs from the step before: its item offsets, item table and meta.
     // The same buffers as item_offset, p.items and meta, unless the step sorts into another block.
     const uint32_t* prev_item_offset;

@@ -251,3 +251,28 @@ def test_queued_elasticity_and_saved_order():
                 sim.synchronize()
                 assert torch.equal(now, later) and not torch.equal(now, cot)
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dim,sizes", [(2, (129,)), (3, (129,)), (3, (129, 9)), (3, (9, 129, 129, 20)), (2, (20,) * 7)])
+def test_sort_tables_at_the_edges_of_their_rounds(dim, sizes):
+    """The sort's tables are built in rounds of 4096 tiles (16 per workgroup for the prefixes): 64, 4096, 4097 and 8202
+    tiles, and 28; every scene of a batch as it is by itself, over steps in which particles change tiles."""
+    clouds = [_cloud(dim, 1500 + 211 * i, 20 + i) for i in range(len(sizes))]
+    for c, res in zip(clouds, sizes):
+        c.v *= np.float32(0.1 * 1e4 / res)  # some tenths of a cell a step
+    specs = [SceneSpec(c, MaterialModel.kJelly, res, E=1.0) for c, res in zip(clouds, sizes)]
+    with MPMBatch(specs, identity_mode=1) as batch:
+        batch.advance(6)
+        got = [batch.particles(s) for s in range(len(sizes))]
+    for c, res, g in zip(clouds, sizes, got):
+        with MPMSimulation(c, MaterialModel.kJelly, res, E=1.0, identity_mode=1) as sim:
+            for _ in range(6):  # the radix sort every step
+                sim.advance(1)
+                image = sim.state_image()
+                sim.set_state_image(image)
+            ref = sim.particles()
+        for k in ("x", "v", "F", "C", "Jp"):
+            # a tile's particles in another order: bitwise up to one work item per tile, else a few
+            # roundings of a node's sum a step
+            a, b = getattr(g, k), getattr(ref, k)
+            assert np.array_equal(a, b) if dim == 3 and res == 129 else np.abs(a - b).max() <= 1e-5 * np.abs(b).max(), k
