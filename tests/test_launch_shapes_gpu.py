@@ -276,3 +276,36 @@ def test_sort_tables_at_the_edges_of_their_rounds(dim, sizes):
             # roundings of a node's sum a step
             a, b = getattr(g, k), getattr(ref, k)
             assert np.array_equal(a, b) if dim == 3 and res == 129 else np.abs(a - b).max() <= 1e-5 * np.abs(b).max(), k
+
+
+@pytest.mark.parametrize("d", [2, 3])
+def test_jacobi_pairs_on_both_sides_of_the_plain_range_are_bitwise_the_oracle(d):
+    """Quotients and roots of operands of ordinary size skip the IEEE range handling (2^-40 of the largest entry up):
+    zeros of either sign, entries and differences around the line, equal diagonals, and matrices of any scale."""
+    from nuclearmpm_amd._lib import check, lib, ptr
+
+    rng = np.random.default_rng(17)
+    n = 3000
+    eye = np.eye(d)[None]
+    tiny = lambda: np.exp2(rng.uniform(-52, -28, (n, d, d))) * rng.choice([-1.0, 1.0], (n, d, d))  # noqa: E731
+    A = [rng.normal(size=(n, d, d)), eye + 0.01 * rng.normal(size=(n, d, d))]
+    A.append(np.where(rng.random((n, d, d)) < 0.4, rng.choice([0.0, -0.0], (n, d, d)), rng.normal(size=(n, d, d))))
+    A.append(eye + tiny())                              # off-diagonals around the line
+    sym = rng.normal(size=(n, d, d))
+    sym = (sym + sym.transpose(0, 2, 1)).astype(np.float32)
+    A.append(sym)                                       # m10 - m01 = 0
+    A.append(sym + 2.0 ** -22 * rng.normal(size=(n, d, d)))
+    eq = rng.normal(size=(n, d, d))
+    eq[:, range(d), range(d)] = rng.normal(size=(n, 1))  # equal diagonals
+    A.append(eq)
+    skew = rng.normal(size=(n, d, d))
+    A.append(skew - skew.transpose(0, 2, 1) + tiny())   # m00 + m11 around the line
+    A.append(rng.normal(size=(n, d, d)) * np.exp2(rng.integers(-148, 126, (n, 1, 1))))
+    A.append(np.exp2(rng.integers(-60, 60, (n, d, d))) * rng.normal(size=(n, d, d)))
+    A = np.ascontiguousarray(np.concatenate(A), np.float32)
+    A = A[np.isfinite(A).all(axis=(1, 2))]
+    U, V, S = np.empty_like(A), np.empty_like(A), np.empty(A.shape[:2], np.float32)
+    check(lib().mpm_svd(d, len(A), ptr(A), ptr(U), ptr(S), ptr(V), 1, 0))
+    Uo, So, Vo = O.svd(A)
+    for a, b in ((U, Uo), (S, So), (V, Vo)):
+        assert np.array_equal(a, b, equal_nan=True)
