@@ -1002,9 +1002,14 @@ struct nclr_mpm_sim {
     int adjoint_steps(int nsteps, const SegTape& T, const SegGuard& g, const float* gout, float* gin,
                       double* grad_E) {
         const size_t gn = gv_nodes();
-        const size_t gbytes = size_t(grad_channels()) * size_t(p.n) * sizeof(float);
-        HIP_TRY(hipMemcpyAsync(gtmp[0], gout, gbytes, hipMemcpyDeviceToDevice, stream));
-        int c = 0, held = 0;
+        // the first step reads gout, the last one writes gin; one step that is both reads a copy (they may alias)
+        const float* from = gout;
+        if (nsteps == 1) {
+            const size_t gbytes = size_t(grad_channels()) * size_t(p.n) * sizeof(float);
+            HIP_TRY(hipMemcpyAsync(gtmp[0], gout, gbytes, hipMemcpyDeviceToDevice, stream));
+            from = gtmp[0];
+        }
+        int held = 0;
         const int room = std::min(nsteps, nclr_dev::kESteps);
         if (grad_E && e_steps < room) {
             HIP_TRY(hipStreamSynchronize(stream));
@@ -1032,14 +1037,14 @@ struct nclr_mpm_sim {
             // the last state is stored in the order of the step before's sort
             const bool order_kept = !kept && t > 0;
             prev_sort = order_kept ? T.sorts + sort_block_bytes * size_t(t - 1) : nullptr;
-            RC_TRY(backward_step(gtmp[c], gtmp[c ^ 1], kept, kept && T.gv, order_kept, held));
-            c ^= 1;
+            float* to = t == 0 ? gin : gtmp[t & 1];
+            RC_TRY(backward_step(from, to, kept, kept && T.gv, order_kept, held));
+            from = to;
             if (grad_E && (++held == e_steps || held == nclr_dev::kESteps || t == 0)) {
                 RC_TRY(sum_e(t + held - 1, held, nsteps, T.sorts, grad_E));
                 held = 0;
             }
         }
-        HIP_TRY(hipMemcpyAsync(gin, gtmp[c], gbytes, hipMemcpyDeviceToDevice, stream));
         return MPM_OK;
     }
 
