@@ -595,6 +595,52 @@ NCLR_DI unsigned long long fixed_point(float y, double scale) {
     return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
 
+// Which lane's particle each lane of a wave takes, so that lanes deposit to different LDS banks: a 64-bit
+// atomic of a wave is 4 cycles when each 16 consecutive lanes hold 16 of the 32 bank pairs, and as many
+// times that as the fullest pair holds lanes (a lattice puts 2 to 8 particles into a cell, neighbours in
+// the order).  first: a particle's first node; all its nodes are at the same distances from it, so lanes
+// whose first nodes differ modulo 32 never meet.  Lanes are ordered by how many earlier ones have their
+// residue.  counts: 32 words of LDS of this wave.
+NCLR_DI uint32_t bank_order(uint32_t* counts, bool valid, int first) {
+    const uint32_t lane = threadIdx.x & 63u;
+    if (lane < 32u) counts[lane] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    uint32_t rank = ~0u;
+    if (valid) rank = atomicAdd(&counts[uint32_t(first) & 31u], 1u);
+    uint32_t pos = 0, base = 0;
+    auto place = [&](bool here) {
+        const uint64_t m = __ballot(here);
+        const uint32_t below = __builtin_amdgcn_mbcnt_hi(uint32_t(m >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(m), 0u));
+        if (here) pos = base + below;
+        base += uint32_t(__popcll(m));
+    };
+#pragma unroll
+    for (uint32_t r = 0; r < 5; ++r) place(rank == r);
+    place(rank >= 5);  // rarely any; and the lanes without a particle
+    return uint32_t(__builtin_amdgcn_ds_permute(int(pos << 2), int(lane)));
+}
+
+// The same for a work item's particles: sorted position j (this lane's by default) and state slot of this lane.
+// Every lane of the wave calls it; only a lane with j < j1 has a particle.
+template <int D>
+NCLR_DI void bank_particles(uint32_t* counts, const float* __restrict__ st, int64_t stride, const SceneParams& sp,
+                            const int (&torg)[D], uint32_t j1, uint32_t& j, uint32_t& slot) {
+    bool here = j < j1;
+    int first = 0;
+    if (here) {
+        float x[D], fx[D], w[D][3];
+        int base[D];
+#pragma unroll
+        for (int a = 0; a < D; ++a) x[a] = ldf(st, stride, Layout<D>::X + a, slot);
+        here = stencil<D>(x, sp, base, fx, w);
+#pragma unroll
+        for (int a = 0; a < D; ++a) first = first * Tile<D>::R + (base[a] - torg[a]);
+    }
+    const uint32_t from = bank_order(counts, here, first);
+    slot = __shfl(slot, int(from));
+    j = j - (threadIdx.x & 63u) + from;
+}
+
 NCLR_DI float fixed_point_value(unsigned long long q, double inv_scale) {
     return float(double((long long)q) * inv_scale);
 }

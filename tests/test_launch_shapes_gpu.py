@@ -342,3 +342,34 @@ def test_backward_leaves_the_first_steps_grid(dim, n, record):
         b.advance(2)
         fresh.advance(1)
         assert np.array_equal(b.particles(0).x, fresh.particles(0).x)
+
+
+@pytest.mark.parametrize("dim,n,spread", [(3, 1, 0.0), (3, 63, 0.0), (3, 65, 0.0), (3, 449, 0.2), (3, 5003, 0.05),
+                                          (3, 530_003, 8.0), (2, 140_003, 6.0), (2, 140_003, 40.0)])
+def test_p2g_lane_order_of_particles_that_share_cells(dim, n, spread):
+    """P2G orders a wave's particles by LDS bank (3D, and 2D with several particles per thread): waves with one particle,
+    with all of them in one cell (spread 0: every rank up to 63), partly filled, and at large against the oracle."""
+    res = 64
+    rng = np.random.default_rng(n)
+    x = (30.3 + spread * (rng.random((n, dim)) - 0.5)) / res
+    p = Particles.from_positions(x.astype(np.float32), identity_mode=1)
+    p.v = rng.normal(0, 1.0, p.v.shape).astype(np.float32)
+    p.C = rng.normal(0, 2.0, p.C.shape).astype(np.float32)
+    p.F = (p.F + rng.normal(0, 0.005, p.F.shape)).astype(np.float32)
+    p.mass = (1.0 + rng.random(n)).astype(np.float32)
+    with MPMSimulation(p, MaterialModel.kJelly, res, E=1e2, identity_mode=1, p2g_chunk=512) as sim:
+        sim.advance(1)
+        got, (vel, mass) = sim.particles(), sim.grid()
+    st = O.State(x=p.x, v=p.v, F=p.F, C=p.C, Jp=p.Jp, mass=p.mass, volume=p.volume)
+    assert_parity(got, O.run(st, O.JELLY, steps=1, res=res, E=1e2, identity_mode=1), inv_dx=float(res),
+                  label=f"{dim}D n={n}")
+    # up to 28,000 particles reach a node: masses against sums in 64 bits (the oracle's FP32 sums round more than the step)
+    X = p.x.astype(np.float64) * res
+    base = (X - 0.5).astype(np.int64)
+    f = X - base
+    w = [0.5 * (1.5 - f) ** 2, 0.75 - (f - 1.0) ** 2, 0.5 * (f - 0.5) ** 2]
+    ref_mass = np.zeros((res + 1,) * dim)
+    for o in np.ndindex(*(3,) * dim):
+        np.add.at(ref_mass, tuple(base[:, a] + o[a] for a in range(dim)),
+                  p.mass * np.prod([w[o[a]][:, a] for a in range(dim)], axis=0))
+    assert np.abs(mass - ref_mass).max() <= 1e-5 * ref_mass.max()
