@@ -683,9 +683,10 @@ static hipError_t sort_dispatch(const LaunchArgs& a) {
 //       faster with it, the 1.75M-particle 2D batch's slower.
 //   3D  fewer than four full work items per CU, which is what the 36 KB of accumulators lets a CU
 //       hold at 256 threads: every item is resident at once and the launch takes as long as its
-//       items.  Chunk 512: 60,007 snow particles 32.8 -> 27.2 us, 150,003 jelly 39.4 -> 35.9,
-//       24 x 9,261 jelly 51.8 -> 48.9; but 680,943 snow (accurate) 81.7 -> 85.4 and 2.1M jelly
-//       214 -> 221, where a CU's next items hide the latency and the wider barriers only cost.
+//       items.  Chunk 512: 30,011 liquid particles 18.2 -> 15.4 us, 60,007 snow 28.9 -> 22.8, 150,003
+//       jelly 33.4 -> 30.4, 24 x 9,261 jelly 40.9 -> 38.7; but 680,943 snow (accurate) 63.7 -> 66.9,
+//       where a CU's next items hide the latency and the wider barriers only cost (1M snow and 2.1M
+//       jelly in the exact mode 131 and 185 us either way).
 template <int D, int MAT, int PPT, int MODE>
 static void p2g_mode(const LaunchArgs& a) {
     const unsigned g = unsigned((a.p.n + 256 * PPT - 1) / (256 * PPT) + a.p.ntiles);
