@@ -117,8 +117,8 @@ int mpm_advance(mpm_handle h, int nsteps);
  * the step (the state the reference's throwing advance() leaves), and the scene stays stopped;
  * later steps advance the other scenes and find the stopped scene again (every later advance() of
  * the reference throws again).  Setting or loading a state (mpm_set_particles, mpm_load_state,
- * mpm_set_state_device) restarts every scene.  A stopped scene's grid export shows its last
- * completed step. */
+ * mpm_set_state_device[_any_order]) restarts every scene.  A stopped scene's grid export shows its
+ * last completed step. */
 int mpm_synchronize(mpm_handle h);
 
 /* Per-scene status without raising it as an error (no reference counterpart: a batch of the
@@ -237,6 +237,11 @@ int mpm_load_state(mpm_handle h, const void* src);
  * volume are kept and the slot order becomes the particle order). */
 int mpm_get_state_device(mpm_handle h, float* dst);
 int mpm_set_state_device(mpm_handle h, const float* src);
+/* mpm_set_state_device, except that the slot order afterwards is the engine's choice: an image of
+ * 2^18 particles or more is stored sorted, so that the first step after it reads the particles in
+ * order.  For callers that read the state and its cotangents through mpm_get_state_device and
+ * mpm_grad_to_particle_order. */
+int mpm_set_state_device_any_order(mpm_handle h, const float* src);
 
 /* Re-indexes a cotangent between particle order and the current slot order (src != dst). */
 int mpm_grad_from_particle_order(mpm_handle h, const float* src, float* dst);

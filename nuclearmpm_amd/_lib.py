@@ -147,7 +147,8 @@ def lib() -> ctypes.CDLL:
     L.mpm_grad_channels.restype = i32
     L.mpm_state_bytes.argtypes = [H]
     L.mpm_state_bytes.restype = i64
-    for name in ("mpm_save_state", "mpm_load_state", "mpm_get_state_device", "mpm_set_state_device"):
+    for name in ("mpm_save_state", "mpm_load_state", "mpm_get_state_device", "mpm_set_state_device",
+                 "mpm_set_state_device_any_order"):
         getattr(L, name).argtypes = [H, _vp]
         getattr(L, name).restype = i32
     L.mpm_order_bytes.argtypes = [H]

@@ -113,7 +113,7 @@ class _Rollout(torch.autograd.Function):
         E_vals = E.detach().double().cpu().tolist()
         for s, e in enumerate(E_vals):
             sim.set_elasticity(s, e)
-        check(L.mpm_set_state_device(h, state0.data_ptr()))
+        check(L.mpm_set_state_device_any_order(h, state0.data_ptr()))
         sb = int(L.mpm_state_bytes(h))
         plan = _record_plan(L, h, steps, every, record, state0.device)
         ckpts = []

@@ -1706,14 +1706,16 @@ int mpm_get_state_device(mpm_handle h, float* dst) {
     return MPM_OK;
 }
 
-int mpm_set_state_device(mpm_handle h, const float* src) {
+// The state from an image in particle order.  any_order: the slot order is the engine's choice (a large image is
+// stored in tile order, with the sort's tables, so that the next step needs no sort); otherwise slots = particles.
+static int set_state_device(mpm_handle h, const float* src, bool any_order) {
     if (!h || (!src && h->p.n > 0)) return fail(MPM_ERR_INVALID, "NULL argument");
     HIP_TRY(hipSetDevice(h->opts.device));
     const int64_t n = h->p.n, stride = h->p.stride;
     if (n == 0) return MPM_OK;
     const int o = h->cur ^ 1, ng = h->grad_channels();
-    if (nclr_host::image_goes_sorted(n)) {
-        // stored in tile order, with the sort's tables: the next step sorts incrementally
+    const bool sorted = any_order && nclr_host::image_goes_sorted(n);
+    if (sorted) {
         const nclr_host::LaunchArgs a = h->args(h->cur);
         HIP_TRY(nclr_host::launch_image_keys(a, src, nclr_host::key_sort_input(a)));
         HIP_TRY(nclr_host::launch_key_sort(a));
@@ -1728,9 +1730,13 @@ int mpm_set_state_device(mpm_handle h, const float* src) {
         HIP_TRY(nclr_host::launch_iota_u32(h->pid[o], stride, h->stream));
     }
     h->cur = o;
-    h->sorted_valid = h->slots_sorted = nclr_host::image_goes_sorted(n);
+    h->sorted_valid = h->slots_sorted = sorted;
     return h->clear_scene_state();
 }
+
+int mpm_set_state_device(mpm_handle h, const float* src) { return set_state_device(h, src, false); }
+
+int mpm_set_state_device_any_order(mpm_handle h, const float* src) { return set_state_device(h, src, true); }
 
 int mpm_grad_from_particle_order(mpm_handle h, const float* src, float* dst) {
     if (!h || ((!src || !dst) && h->p.n > 0)) return fail(MPM_ERR_INVALID, "NULL argument");

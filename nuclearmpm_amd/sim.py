@@ -193,7 +193,7 @@ class _Engine:
         image = image.contiguous()
         torch.cuda.synchronize(image.device)
         self._cache = None
-        check(lib().mpm_set_state_device(self._handle(), image.data_ptr() if self._n else None))
+        check(lib().mpm_set_state_device_any_order(self._handle(), image.data_ptr() if self._n else None))
         check(lib().mpm_synchronize(self._handle()))
 
     def state_image(self):

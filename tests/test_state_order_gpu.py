@@ -1,0 +1,53 @@
+"""Slot order of the engine's state after it is set from a device image."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from nuclearmpm_amd import MaterialModel, MPMSimulation, Particles, autodiff
+from nuclearmpm_amd._lib import check, lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _cloud(dim, n, seed):
+    rng = np.random.default_rng(seed)
+    p = Particles.from_positions((0.2 + 0.5 * rng.random((n, dim))).astype(np.float32), identity_mode=1)
+    p.v = rng.normal(0, 1.0, p.v.shape).astype(np.float32)
+    p.C = rng.normal(0, 1.0, p.C.shape).astype(np.float32)
+    p.F = (p.F + rng.normal(0, 0.01, p.F.shape)).astype(np.float32)
+    return p
+
+
+@pytest.mark.parametrize("dim,n", [(2, 1001), (2, 262143), (2, 262144), (3, 262144), (3, 300007)])
+def test_set_state_device_makes_the_slot_order_the_particle_order(dim, n):
+    """At every size: a cotangent in slot order is one in particle order, and mpm_backward_step returns grad_in in
+    particle order, bit for bit what a one-step rollout returns."""
+    p = _cloud(dim, n, dim)
+    ng = autodiff.channels(dim)
+    with MPMSimulation(p, MaterialModel.kJelly, 64, E=1e3, identity_mode=1) as sim:
+        L, h = lib(), sim._handle()
+        image = sim.state_image()
+        cot = torch.randn(ng, n, generator=torch.Generator("cuda").manual_seed(7), device="cuda")
+        s0 = image.clone().requires_grad_(True)
+        out = autodiff.rollout(sim, s0, torch.tensor([1e3]), steps=1, checkpoint_every=1)
+        want = torch.autograd.grad(out, s0, cot)[0]
+        sim.advance(2)  # slots in tile order
+        snap = torch.empty(int(L.mpm_state_bytes(h)), dtype=torch.uint8, device="cuda")
+        order = torch.empty(int(L.mpm_order_bytes(h)), dtype=torch.uint8, device="cuda")
+        slots, gin = torch.empty_like(cot), torch.empty_like(cot)
+        torch.cuda.synchronize()
+        check(L.mpm_set_state_device(h, image.data_ptr()))
+        check(L.mpm_save_order(h, order.data_ptr()))
+        check(L.mpm_save_state(h, snap.data_ptr()))
+        check(L.mpm_grad_from_particle_order(h, cot.data_ptr(), slots.data_ptr()))
+        sim.synchronize()
+        assert torch.equal(order.view(torch.int32)[:n], torch.arange(n, dtype=torch.int32, device="cuda"))
+        assert torch.equal(slots, cot)
+        sim.advance(1)
+        check(L.mpm_grad_from_particle_order(h, cot.data_ptr(), slots.data_ptr()))
+        check(L.mpm_load_state(h, snap.data_ptr()))
+        check(L.mpm_backward_step(h, slots.data_ptr(), gin.data_ptr(), None))
+        sim.synchronize()
+        assert torch.equal(gin, want)
