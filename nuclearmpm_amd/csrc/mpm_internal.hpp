@@ -150,7 +150,7 @@ struct CompactArgs {
 
 namespace nclr_host {
 
-// Fewer full work items than this (the chip's CUs; 3D P2G: than four times this) make a launch
+// Fewer full work items than this (the chip's CUs; 3D P2G at chunk 512: than four times this) make a launch
 // latency-bound: P2G and the 2D G2P adjoint then run one particle per thread.
 constexpr int kFewItems = 256;
 

@@ -165,8 +165,18 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
     const uint32_t tile = wi.tile;
     const int scene = p.nscenes == 1 ? 0 : scene_of_tile(p, tile);
     if (scene_stopped(p, scene)) return;  // uniform over the workgroup
-    for (int r = threadIdx.x; r < 4 * REG; r += blockDim.x) acc[r] = 0ull;
-    for (int r = threadIdx.x; r < REG; r += blockDim.x) nonfinite[r] = 0u;
+    for (int r = threadIdx.x; r < 4 * REG; r += TPB) acc[r] = 0ull;
+    for (int r = threadIdx.x; r < REG; r += TPB) nonfinite[r] = 0u;
+    // The item's waves: those with particles, and at least 256 threads for the loop over the region.  The
+    // others end here and free their registers (the barriers below wait for the waves that are left).
+    int threads = TPB;
+    if constexpr (TPB > 256) {
+        threads = max(256, int(wi.j1 - wi.j0 + 63u) & ~63);
+        if (__builtin_amdgcn_readfirstlane(int(threadIdx.x)) >= threads) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // the zeros above are in LDS
+            return;
+        }
+    }
     __syncthreads();
     const SceneParams sp = p.scenes[scene];
     const int material = MAT == kMixed ? sp.material : MAT;
@@ -267,7 +277,8 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
         } else {
             bmax = s_bound[0][c];
 #pragma unroll
-            for (int w = 1; w < NW; ++w) bmax = fmaxf(bmax, s_bound[w][c]);
+            for (int w = 1; w < NW; ++w)
+                if (w < 4 || 64 * w < threads) bmax = fmaxf(bmax, s_bound[w][c]);
         }
         fixed_point_scale(bmax, scale[c], inv_scale[c]);
     }
@@ -301,7 +312,7 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
     // every work item owns a slot: plain stores, no global atomics
     float4* dst = slots + int64_t(item) * REG;
     const float nan = __builtin_nanf("");
-    for (int r = threadIdx.x; r < REG; r += blockDim.x) {
+    for (int r = threadIdx.x; r < REG; r += threads) {
         float out[4];
         const uint32_t bad = nonfinite[r];
 #pragma unroll
@@ -676,25 +687,33 @@ static hipError_t sort_dispatch(const LaunchArgs& a) {
     return hipGetLastError();
 }
 
-// 256 threads with chunk / 256 particles each, or, when the particles fill few work items, one
-// particle per thread (a workgroup of chunk threads), which shortens a work item's latency (the
-// results are the same: the sums are exact and the scale is the item's maximum).  The line:
+// 256 threads with chunk / 256 particles each, or one particle per thread (a workgroup of chunk threads, those
+// past the item's particles ended at once), which shortens a work item's latency; the results are the same:
+// the sums are exact and the scale is the item's maximum.  The host knows the particles, not the work items:
+// a lattice has few full ones, spread particles one of a few dozen in every tile.  The lines:
 //   2D  fewer full work items than the chip has CUs.  The 19,600-particle 2D jelly step's P2G is
 //       faster with it, the 1.75M-particle 2D batch's slower.
-//   3D  fewer than four full work items per CU, which is what the 36 KB of accumulators lets a CU
-//       hold at 256 threads: every item is resident at once and the launch takes as long as its
-//       items.  Chunk 512: 30,011 liquid particles 18.2 -> 15.4 us, 60,007 snow 28.9 -> 22.8, 150,003
-//       jelly 33.4 -> 30.4, 24 x 9,261 jelly 40.9 -> 38.7; but 680,943 snow (accurate) 63.7 -> 66.9,
-//       where a CU's next items hide the latency and the wider barriers only cost (1M snow and 2.1M
-//       jelly in the exact mode 131 and 185 us either way).
+//   3D  chunk 512, the exact and the fast mode, fewer than four full work items per CU.  us, one particle per
+//       thread / 256 threads, res 128:
+//         lattice  exact 30,011 22.4 / 28, 150,003 30.5 / 34, 262,144 37 / 40, 400,000 48 / 49, 520,000 55 / 58
+//                  fast  30,011 17.8 / 20, 150,003 25 / 26, 262,144 29 / 30.5, 400,000 38 / 39, 520,000 44 / 46
+//         spread   exact  5,000 47 / 47, 60,000 58 / 58.5, 150,000 59 / 59, 300,000 63 / 63, 500,000 68 / 67
+//                  fast   5,000 36 / 36, 60,000 42 / 42.5, 150,000 42 / 43, 300,000 45 / 46, 500,000 49 / 49
+//       Spread particles took 67 to 75 in the exact mode while the idle waves stayed.  Beyond the line a CU's
+//       next items hide the latency.  Not the accurate mode, whose registers (114) let a CU hold two such
+//       workgroups: lattices 17.2 / 20, 24 / 26 and 31.5 / 30, but spread 51 / 47.  Not chunk 1024, where 1024 threads
+//       leave too few registers: a lattice of 60,007 33 / 48, as many spread 98 / 62.
 template <int D, int MAT, int PPT, int MODE>
 static void p2g_mode(const LaunchArgs& a) {
     const unsigned g = unsigned((a.p.n + 256 * PPT - 1) / (256 * PPT) + a.p.ntiles);
-    if (a.p.n < int64_t(D == 2 ? kFewItems : 4 * kFewItems) * 256 * PPT)
-        k_p2g_tile<D, MAT, 1, MODE, 256 * PPT><<<g, 256 * PPT, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p,
-                                                                             a.slots, a.rot);
-    else
-        k_p2g_tile<D, MAT, PPT, MODE><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p, a.slots, a.rot);
+    if constexpr (D == 2 || (PPT == 2 && MODE != kSvdAccurate)) {
+        if (a.p.n < int64_t(D == 2 ? kFewItems : 4 * kFewItems) * 256 * PPT) {
+            k_p2g_tile<D, MAT, 1, MODE, 256 * PPT><<<g, 256 * PPT, 0, a.stream>>>(a.state_in, a.perm, a.item_offset,
+                                                                                 a.p, a.slots, a.rot);
+            return;
+        }
+    }
+    k_p2g_tile<D, MAT, PPT, MODE><<<g, 256, 0, a.stream>>>(a.state_in, a.perm, a.item_offset, a.p, a.slots, a.rot);
 }
 
 template <int D, int MAT, int PPT>

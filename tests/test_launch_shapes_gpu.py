@@ -373,3 +373,29 @@ def test_p2g_lane_order_of_particles_that_share_cells(dim, n, spread):
         np.add.at(ref_mass, tuple(base[:, a] + o[a] for a in range(dim)),
                   p.mass * np.prod([w[o[a]][:, a] for a in range(dim)], axis=0))
     assert np.abs(mass - ref_mass).max() <= 1e-5 * ref_mass.max()
+
+
+@pytest.mark.parametrize("material,svd", [(MaterialModel.kJelly, "exact"), (MaterialModel.kSnow, "fast"),
+                                          (MaterialModel.kLiquid, "exact")])
+def test_3d_p2g_ends_the_waves_without_particles(material, svd):
+    """One particle per thread (3D, chunk 512, below 1024 full work items: 524,288 particles): work items of 1 to 512
+    particles, whose idle waves end before the barriers, in scenes alone and in a batch above the line."""
+    opts = dict(identity_mode=1, svd=svd, p2g_chunk=512)
+    res, tile, rng = 64, 8, np.random.default_rng(8)
+    counts = (1, 64, 65, 255, 256, 257, 320, 321, 448, 449, 511, 512, 513, 769, 1024)
+    x = []
+    for k, c in enumerate(counts):  # a tile each, every second one along the axes; stencil bases inside the tile
+        first = 0.5 + tile * (1 + 2 * np.array([k % 3, k // 3 % 3, k // 9]))
+        x.append((first + 0.1 + (tile - 0.2) * rng.random((c, 3))) / res)
+    a = Particles.from_positions(np.concatenate(x).astype(np.float32), identity_mode=1)
+    a.v = rng.normal(0, 1.0, a.v.shape).astype(np.float32)
+    a.F = (a.F + rng.normal(0, 0.01, a.F.shape)).astype(np.float32)
+    b = _cloud(3, 1024 * 512, 9)
+    with MPMBatch([SceneSpec(a, material, res), SceneSpec(b, material, res)], **opts) as batch:
+        batch.advance(2)
+        got = batch.particles(0)
+    with MPMSimulation(a, material, res, **opts) as sim:
+        sim.advance(2)
+        ref = sim.particles()
+    for k in ("x", "v", "F", "C", "Jp"):
+        assert np.array_equal(getattr(got, k), getattr(ref, k)), k
