@@ -399,3 +399,32 @@ def test_3d_p2g_ends_the_waves_without_particles(material, svd):
         ref = sim.particles()
     for k in ("x", "v", "F", "C", "Jp"):
         assert np.array_equal(getattr(got, k), getattr(ref, k)), k
+
+
+@pytest.mark.parametrize("dim,sizes", [(2, (129,)), (3, (129,)), (3, (129, 9)), (3, (9, 129, 129, 20)), (2, (20,) * 7),
+                                       (2, (8192,)), (2, (8192, 20)), (3, (512, 20))])
+def test_incremental_sort_tables_are_bitwise_the_radix_sorts(dim, sizes):
+    """Up to 64 rounds of 4096 tiles the sort's carries come from the tiles, above (65 rounds: res 8192 or 512 and a
+    small scene) from the rounds' totals: bit for bit the steps of an engine that saves and loads its state
+    before each one, which keeps the slot order and sorts from scratch."""
+    import torch
+
+    from nuclearmpm_amd._lib import check, lib
+
+    clouds = [_cloud(dim, 1500 + 211 * i, 20 + i) for i in range(len(sizes))]
+    for c, res in zip(clouds, sizes):
+        c.v *= np.float32(0.1 * 1e4 / res)  # some tenths of a cell a step
+    specs = [SceneSpec(c, MaterialModel.kJelly, res, E=1.0) for c, res in zip(clouds, sizes)]
+    with MPMBatch(specs, identity_mode=1) as batch, MPMBatch(specs, identity_mode=1) as fresh:
+        L, h = lib(), fresh._handle()
+        snap = torch.empty(int(L.mpm_state_bytes(h)), dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        for _ in range(6):
+            batch.advance(1)
+            check(L.mpm_save_state(h, snap.data_ptr()))
+            check(L.mpm_load_state(h, snap.data_ptr()))
+            fresh.advance(1)
+        assert torch.equal(batch.state_image(), fresh.state_image())
+        assert not torch.equal(batch.state_image()[:dim], torch.from_numpy(np.concatenate([c.x for c in clouds]).T).cuda())
+        for s in range(len(sizes)):
+            assert batch.active_nodes(s) == fresh.active_nodes(s) > 0
