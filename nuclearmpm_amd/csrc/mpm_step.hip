@@ -156,8 +156,12 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
     // 6.  680,943 snow particles (accurate) 81 -> 63 us, 24 x 9,261 jelly 45.5 -> 38.2, 150,003 jelly 33 -> 29,
     // 30,011 liquid 17.9 -> 15.3, 8 x 262,144 jelly 200 -> 185, 1M spread snow (random order, issue bound) 130
     // either way; 256 2D scenes 48.3 -> 46.7.  Not in 2D launches of one particle per thread, whose nine
-    // nodes do not pay for a second dependent load (8.5 us either way).
+    // nodes do not pay for a second dependent load (8.5 us either way), nor in work items of up to kBankItem
+    // particles, two waves, which have little to collide (us, ordered / not: 60,000 liquid particles spread
+    // over res 128 24.3 / 23.3, 64 such scenes of 20,000 1160 / 1096, 300,000 2D jelly over res 4096 98 / 86,
+    // 128 2D scenes of 2,000 23.9 / 21.5; 256 scenes of a lattice of 100 13.5 / 13.2).
     constexpr bool BANKS = D == 3 || PPT > 1;
+    constexpr uint32_t kBankItem = 128;
     __shared__ uint32_t s_banks[BANKS ? NW : 1][32];
     const uint32_t item = blockIdx.x;
     const WorkItem wi = work_item(p, item);  // loaded with the count below, used only if valid
@@ -201,7 +205,7 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
         rb[k] = 0;
         ms[k] = 0.0f;
         uint32_t slot = j < j1 ? perm[j] : 0u;
-        if constexpr (BANKS) bank_particles<D>(s_banks[threadIdx.x >> 6], st, p.stride, sp, torg, j1, j, slot);
+        if (BANKS && j1 - j0 > kBankItem) bank_particles<D>(s_banks[threadIdx.x >> 6], st, p.stride, sp, torg, j1, j, slot);
         if (j >= j1) continue;
         const int64_t i = slot;
         float x[D], v[D];

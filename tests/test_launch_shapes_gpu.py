@@ -382,7 +382,7 @@ def test_3d_p2g_ends_the_waves_without_particles(material, svd):
     particles, whose idle waves end before the barriers, in scenes alone and in a batch above the line."""
     opts = dict(identity_mode=1, svd=svd, p2g_chunk=512)
     res, tile, rng = 64, 8, np.random.default_rng(8)
-    counts = (1, 64, 65, 255, 256, 257, 320, 321, 448, 449, 511, 512, 513, 769, 1024)
+    counts = (1, 64, 65, 128, 129, 255, 256, 257, 320, 321, 448, 449, 511, 512, 513, 769, 1024)
     x = []
     for k, c in enumerate(counts):  # a tile each, every second one along the axes; stencil bases inside the tile
         first = 0.5 + tile * (1 + 2 * np.array([k % 3, k // 3 % 3, k // 9]))
