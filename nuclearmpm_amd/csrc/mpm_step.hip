@@ -139,10 +139,17 @@ __global__ __launch_bounds__(1024) void k_items_rounds(const uint32_t* __restric
 // ---------------------------------------------------------------------------------------------
 
 // A work item of TPB * PPT particles, PPT per thread.
+// kLateAffine (the exact mode's 512 threads): C, Jp, mass and volume are loaded behind the SVD instead of held
+// through it, which fits eight waves per SIMD and so four workgroups per CU, as many as of 256 threads: 64 VGPRs
+// instead of 74.  60,000 snow particles spread over two thirds of res 128 40 -> 32 us (three workgroups per CU
+// made a second round of their 1,300 work items), a lattice of 150,003 31 -> 30.6.
+template <int D, int MODE, int TPB>
+constexpr bool kLateAffine = D == 3 && MODE == kSvdExact && TPB == 512;
+
 template <int D, int MAT, int PPT, int MODE, int TPB = 256>
-__global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, const uint32_t* __restrict__ perm,
-                                                  const uint32_t* __restrict__ item_offset, StepParams p,
-                                                  float4* __restrict__ slots, float* __restrict__ rot) {
+__global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(kLateAffine<D, MODE, TPB> ? 8 : 1))) void k_p2g_tile(
+    const float* __restrict__ st, const uint32_t* __restrict__ perm, const uint32_t* __restrict__ item_offset,
+    StepParams p, float4* __restrict__ slots, float* __restrict__ rot) {
     using TL = Tile<D>;
     using L = Layout<D>;
     constexpr int REG = TL::REGION;
@@ -162,6 +169,7 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
     // 128 2D scenes of 2,000 23.9 / 21.5; 256 scenes of a lattice of 100 13.5 / 13.2).
     constexpr bool BANKS = D == 3 || PPT > 1;
     constexpr uint32_t kBankItem = 128;
+    constexpr bool LATE = kLateAffine<D, MODE, TPB>;
     __shared__ uint32_t s_banks[BANKS ? NW : 1][32];
     const uint32_t item = blockIdx.x;
     const WorkItem wi = work_item(p, item);  // loaded with the count below, used only if valid
@@ -220,11 +228,14 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
 #pragma unroll
             for (int b = 0; b < D; ++b) {
                 F.a[a][b] = ldf(st, p.stride, L::F + a * D + b, i);
-                C.a[a][b] = ldf(st, p.stride, L::C + a * D + b, i);
+                if constexpr (!LATE) C.a[a][b] = ldf(st, p.stride, L::C + a * D + b, i);
             }
-        const float Jp = ldf(st, p.stride, L::JP, i);
-        const float mass = ldf(st, p.stride, L::MASS, i);
-        const float vol = ldf(st, p.stride, L::VOL, i);
+        float Jp, mass, vol;
+        if constexpr (!LATE) {
+            Jp = ldf(st, p.stride, L::JP, i);
+            mass = ldf(st, p.stride, L::MASS, i);
+            vol = ldf(st, p.stride, L::VOL, i);
+        }
         int base[D];
         float fx[D], w[D][3];
         if (!stencil<D>(x, sp, base, fx, w)) continue;  // keyed into this tile, so never taken
@@ -236,6 +247,17 @@ __global__ __launch_bounds__(TPB) void k_p2g_tile(const float* __restrict__ st, 
             for (int a = 0; a < D; ++a)
 #pragma unroll
                 for (int b = 0; b < D; ++b) rot[int64_t(a * D + b) * p.stride + j] = keep.a[a][b];
+        if constexpr (LATE) {
+            const float* st2 = st;
+            asm volatile("" : "+s"(st2));
+#pragma unroll
+            for (int a = 0; a < D; ++a)
+#pragma unroll
+                for (int b = 0; b < D; ++b) C.a[a][b] = ldf(st2, p.stride, L::C + a * D + b, i);
+            Jp = ldf(st2, p.stride, L::JP, i);
+            mass = ldf(st2, p.stride, L::MASS, i);
+            vol = ldf(st2, p.stride, L::VOL, i);
+        }
         As[k] = fused_affine_from<D>(material, F, FmR, C, Jp, mass, vol, sp);
         ms[k] = mass;
         float wsum = 1.0f;
@@ -699,14 +721,14 @@ static hipError_t sort_dispatch(const LaunchArgs& a) {
 //       faster with it, the 1.75M-particle 2D batch's slower.
 //   3D  chunk 512, the exact and the fast mode, fewer than four full work items per CU.  us, one particle per
 //       thread / 256 threads, res 128:
-//         lattice  exact 30,011 22.4 / 28, 150,003 30.5 / 34, 262,144 37 / 40, 400,000 48 / 49, 520,000 55 / 58
-//                  fast  30,011 17.8 / 20, 150,003 25 / 26, 262,144 29 / 30.5, 400,000 38 / 39, 520,000 44 / 46
-//         spread   exact  5,000 47 / 47, 60,000 58 / 58.5, 150,000 59 / 59, 300,000 63 / 63, 500,000 68 / 67
-//                  fast   5,000 36 / 36, 60,000 42 / 42.5, 150,000 42 / 43, 300,000 45 / 46, 500,000 49 / 49
-//       Spread particles took 67 to 75 in the exact mode while the idle waves stayed.  Beyond the line a CU's
-//       next items hide the latency.  Not the accurate mode, whose registers (114) let a CU hold two such
-//       workgroups: lattices 17.2 / 20, 24 / 26 and 31.5 / 30, but spread 51 / 47.  Not chunk 1024, where 1024 threads
-//       leave too few registers: a lattice of 60,007 33 / 48, as many spread 98 / 62.
+//         lattice  exact 30,011 21 / 27, 150,003 31 / 34, 262,144 37.5 / 39.5, 400,000 46.5 / 49.5, 520,000 53.5 / 59
+//                  fast  30,011 17 / 20, 150,003 24.5 / 26, 262,144 29 / 31, 400,000 36.5 / 38.5, 520,000 42 / 46
+//         spread   exact  5,000 43.5 / 44, 60,000 53 / 53, 150,000 54 / 54.5, 262,000 59.5 / 59.5, 520,000 69 / 69
+//                  fast   5,000 33 / 33.5, 60,000 38 / 39, 150,000 39.5 / 41, 262,000 44 / 44.5, 520,000 51 / 51.5
+//       Beyond the line a CU's next items hide the latency.  Not the accurate mode, whose registers (114) let a
+//       CU hold two such workgroups: lattices 16.5 / 19, 24 / 25.5 and 31.5 / 30.5, but spread 46 to 49 / 43.  Not
+//       chunk 1024, where 1024 threads leave too few registers: lattices of the exact mode 31 / 46 and 56 / 56,
+//       spread 90 / 55; of the fast mode 24 / 31 and 60 / 54.
 template <int D, int MAT, int PPT, int MODE>
 static void p2g_mode(const LaunchArgs& a) {
     const unsigned g = unsigned((a.p.n + 256 * PPT - 1) / (256 * PPT) + a.p.ntiles);
