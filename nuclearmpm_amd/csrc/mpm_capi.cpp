@@ -1032,6 +1032,8 @@ struct nclr_mpm_sim {
             if (kept && T.gv && t == 0) {
                 HIP_TRY(nclr_host::launch_restore_grid(args(cur), T.gv, T.gpre));
                 stamp_host += 1;
+            } else if (kept && t == 0) {
+                HIP_TRY(nclr_host::launch_clear_counts(args(cur)));  // its grid update follows, its sort does not
             }
             rot = T.gv && dim == 3 && kept ? T.rot + size_t(t) * rot_floats() : nullptr;
             // the last state is stored in the order of the step before's sort

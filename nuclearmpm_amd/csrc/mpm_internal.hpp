@@ -251,6 +251,9 @@ hipError_t launch_sort_incremental(const LaunchArgs& a);
 int bucket_offsets(int dim);
 hipError_t launch_p2g(const LaunchArgs& a);
 hipError_t launch_grid(const LaunchArgs& a);
+// Zeroes the node counts of node tiles that a grid update of the sort in a does not visit (a step without a
+// sort of its own, after steps whose particles reached other node tiles).
+hipError_t launch_clear_counts(const LaunchArgs& a);
 // Bumps the step stamp and makes a recorded step's grid (its sort in a) the engine's own.
 hipError_t launch_restore_grid(const LaunchArgs& a, const float4* kept_gv, const float4* kept_gpre);
 hipError_t launch_g2p(const LaunchArgs& a);

@@ -815,6 +815,11 @@ hipError_t launch_grid(const LaunchArgs& a) {
     return hipGetLastError();
 }
 
+hipError_t launch_clear_counts(const LaunchArgs& a) {
+    if (!grid_tiles_listed(a.dim, a.p)) return hipSuccess;  // the grid update visits every node tile
+    return launch_fill_u32(a.active, a.p.node_tiles, 0u, a.stream);
+}
+
 hipError_t launch_restore_grid(const LaunchArgs& a, const float4* kept_gv, const float4* kept_gpre) {
     if (a.p.node_tiles == 0) return hipSuccess;
     hipError_t e = launch_bump_u32(a.stamp, a.stream);

@@ -428,3 +428,31 @@ def test_incremental_sort_tables_are_bitwise_the_radix_sorts(dim, sizes):
         assert not torch.equal(batch.state_image()[:dim], torch.from_numpy(np.concatenate([c.x for c in clouds]).T).cuda())
         for s in range(len(sizes)):
             assert batch.active_nodes(s) == fresh.active_nodes(s) > 0
+
+
+@pytest.mark.parametrize("dim,n", [(3, 4001), (2, 66_000)])
+@pytest.mark.parametrize("record", ["none", "grid", "nogrid"])
+def test_backward_drops_the_node_counts_of_later_steps(dim, n, record):
+    """As above, where the second step reaches node tiles that the first one does not list (the particles move down an
+    axis, out of the lowest tile they are in): their counts must not stay."""
+    import torch
+
+    from nuclearmpm_amd import autodiff
+
+    res, S = 128, 8 if dim == 3 else 16
+    c = _cloud(dim, n, 33)
+    base = 40 + c.x.astype(np.float64) * 20  # clear of the walls
+    base[:, 0] += 4 * S + 0.05 - base[:, 0].min()  # the lowest stencil base is 4 S, a step later 4 S - 1
+    c.x = ((base + 0.5) / res).astype(np.float32)
+    c.v, c.C, c.F = c.v * 0, c.C * 0, c.F * 0 + np.eye(dim, dtype=np.float32)
+    c.v[:, 0] = -60.0  # 0.77 cells a step
+    tiles = ((c.x * np.float32(res) - np.float32(0.5)).astype(np.int64)) // S
+    listed = {tuple(t + d) for t in np.unique(tiles, axis=0) for d in np.ndindex(*(2,) * dim)}
+    opts = dict(identity_mode=1, E=1.0, p2g_chunk=256)
+    with MPMSimulation(c, MaterialModel.kJelly, res, **opts) as b, MPMSimulation(c, MaterialModel.kJelly, res, **opts) as fresh:
+        fresh.advance(2)
+        assert not {tuple(t) for t in np.unique(np.argwhere(fresh.grid()[1] > 0) // S, axis=0)} <= listed
+        x0 = autodiff.pack(*(torch.from_numpy(getattr(c, k)).cuda() for k in ("x", "v", "F", "C", "Jp"))).requires_grad_(True)
+        out = autodiff.rollout(b, x0, torch.tensor([1.0], requires_grad=True), 2, 2, record=record)
+        out.square().sum().backward()
+        assert b.active_nodes() == int((b.grid()[1] > 0).sum()) > 0
