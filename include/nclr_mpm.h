@@ -278,7 +278,9 @@ int mpm_backward_segment(mpm_handle h, int nsteps, const float* grad_out, float*
  * forward grid and its pre-update {momentum, mass} (32 bytes per node of every scene's node tiles)
  * with, in 3D, nsteps - 1 entries of the particles' polar factors (36 bytes per particle); kept
  * only while they leave a quarter of the free device memory, else each adjoint step recomputes
- * them. */
+ * them.  Also, where grad_E is given, the dL/dE contributions of up to 32 steps between two sums, less one
+ * step's, which every engine has that ran a backward pass (per step 4 bytes per particle, and per
+ * scene 16 bytes and 8 per 2,048 particles of the largest scene). */
 int64_t mpm_tape_bytes(mpm_handle h, int nsteps);
 
 /* Recorded segments: no counterpart in the reference (whose checkpointing recomputes every

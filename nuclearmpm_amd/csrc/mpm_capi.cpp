@@ -828,6 +828,10 @@ struct nclr_mpm_sim {
     // Room for the dL/dE contributions of `steps` adjoint steps between two sums.
     hipError_t grow_e_steps(int steps) {
         if (e_steps >= steps) return hipSuccess;
+        if (epart) {
+            const hipError_t e = hipStreamSynchronize(stream);
+            if (e != hipSuccess) return e;
+        }
         if (epart) (void)hipFree(epart);
         if (erange) (void)hipFree(erange);
         if (epartial) (void)hipFree(epartial);
@@ -842,13 +846,31 @@ struct nclr_mpm_sim {
         return e;
     }
 
+    // Device bytes of one such step.
+    int64_t e_step_bytes() {
+        const int64_t ns = int64_t(scenes.size());
+        return int64_t(sizeof(float)) * std::max<int64_t>(p.n, 1) + int64_t(sizeof(int64_t)) * 2 * ns +
+               int64_t(sizeof(double)) * ns * echunks_for_scenes();
+    }
+
+    // Room for the dL/dE contributions of up to kESteps of `steps` adjoint steps if that is to be had (else of one:
+    // sums step by step).  Allocated once a segment's state and sort tapes are, which it needs, and before
+    // its grid tape, which takes its share of what is free.
+    int ensure_e_steps(int steps) {
+        steps = std::max(1, std::min(steps, nclr_dev::kESteps));
+        if (grow_e_steps(steps) == hipSuccess) return MPM_OK;
+        (void)hipGetLastError();
+        if (grow_e_steps(1) == hipSuccess) return MPM_OK;
+        return fail(MPM_ERR_HIP, "hipMalloc of the adjoint buffers failed (out of device memory?)");
+    }
+
     int ensure_adjoint() {
         if (adjoint_ready) return MPM_OK;
         const size_t slot_nodes = size_t(nclr_host::max_items(p.n, p.ntiles)) * nclr_host::region_nodes(dim);
         const size_t gfl = size_t(grad_channels()) * size_t(std::max<int64_t>(p.n, 1));
         auto alloc = [](auto** q, size_t count) { return *q ? hipSuccess : dmalloc(q, count); };
         if (alloc(&slots_b, slot_nodes) != hipSuccess || alloc(&gbar, gv_nodes()) != hipSuccess ||
-            grow_e_steps(1) != hipSuccess || alloc(&rot_own, rot_floats()) != hipSuccess ||
+            alloc(&rot_own, rot_floats()) != hipSuccess ||
             alloc(&gtmp[0], gfl) != hipSuccess || alloc(&gtmp[1], gfl) != hipSuccess)
             return fail(MPM_ERR_HIP, "hipMalloc of the adjoint buffers failed (out of device memory?)");
         adjoint_ready = true;
@@ -865,6 +887,7 @@ struct nclr_mpm_sim {
     int backward_step(const float* gout, float* gin, bool presorted = false, bool grid_kept = false,
                       bool order_kept = false, int slot = 0) {
         RC_TRY(ensure_adjoint());
+        RC_TRY(ensure_e_steps(1));
         if (p.n == 0) return MPM_OK;
         nclr_host::LaunchArgs a = args(cur);
         if (!(presorted && grid_kept)) a.rot = rot_own;  // P2G is recomputed below
@@ -1010,14 +1033,6 @@ struct nclr_mpm_sim {
             from = gtmp[0];
         }
         int held = 0;
-        const int room = std::min(nsteps, nclr_dev::kESteps);
-        if (grad_E && e_steps < room) {
-            HIP_TRY(hipStreamSynchronize(stream));
-            if (grow_e_steps(room) != hipSuccess) {  // no room: sums step by step
-                (void)hipGetLastError();
-                HIP_TRY(grow_e_steps(1));
-            }
-        }
         struct PrevReset {
             char*& prev;
             ~PrevReset() { prev = nullptr; }
@@ -1055,8 +1070,8 @@ struct nclr_mpm_sim {
     // (adjoint_steps); no state copies.  The engine's own buffers, pointers and step counter are
     // restored at the end, so the state is the checkpoint again.
     int backward_segment(int nsteps, const float* gout, float* gin, double* grad_E) {
-        RC_TRY(ensure_adjoint());
         if (nsteps < 1) return fail(MPM_ERR_INVALID, "nsteps must be >= 1");
+        RC_TRY(ensure_adjoint());
         if (p.n == 0) return MPM_OK;
         const size_t sb = state_bytes();
         if (tape_states < nsteps - 1) {
@@ -1069,6 +1084,7 @@ struct nclr_mpm_sim {
             HIP_TRY(hipMalloc(reinterpret_cast<void**>(&sort_tape), sort_block_bytes * size_t(nsteps - 1)));
             tape_states = nsteps - 1;
         }
+        RC_TRY(ensure_e_steps(grad_E ? nsteps : 1));
         const size_t gn = gv_nodes();
         if (tape_grid_states < nsteps) {
             // the grid tape: every step of the segment, if it leaves a quarter of the free device memory
@@ -1184,14 +1200,15 @@ struct nclr_mpm_sim {
     // backward_segment over a segment recorded by advance_recorded from the current state (the
     // caller restores the segment's first state): no recomputation of the recorded steps.
     int backward_recorded(int nsteps, char* rec, bool with_grid, const float* gout, float* gin, double* grad_E) {
-        RC_TRY(ensure_adjoint());
         if (nsteps < 1) return fail(MPM_ERR_INVALID, "nsteps must be >= 1");
+        RC_TRY(ensure_adjoint());
         auto it = std::find_if(records.begin(), records.end(), [&](const RecordInfo& r) { return r.base == rec; });
         if (it == records.end() || it->nsteps != nsteps || it->with_grid != with_grid)
             return fail(MPM_ERR_INVALID, "the tape was not recorded by mpm_advance_recorded with these nsteps and with_grid");
         if (it->params != params_digest())
             return fail(MPM_ERR_INVALID, "the engine's parameters (tuning or elasticity) changed since the tape was recorded");
         if (p.n == 0) return MPM_OK;
+        RC_TRY(ensure_e_steps(grad_E ? nsteps : 1));
         SegTape T{};
         (void)record_layout(nsteps, with_grid, rec, &T);
         SegGuard g(*this);
@@ -1798,7 +1815,8 @@ int64_t mpm_tape_bytes(mpm_handle h, int nsteps) {
     if (!h || nsteps < 1) return -1;
     const int64_t grid = 2 * int64_t(h->p.node_tiles) * int64_t(nclr_host::tile_nodes(h->dim)) * int64_t(sizeof(float4));
     const int64_t rot = int64_t(h->rot_floats() * sizeof(float));
-    return int64_t(nsteps - 1) * (int64_t(h->state_bytes() + h->sort_block_bytes) + rot) + int64_t(nsteps) * grid;
+    const int64_t e = int64_t(std::min(nsteps, nclr_dev::kESteps) - 1) * h->e_step_bytes();
+    return int64_t(nsteps - 1) * (int64_t(h->state_bytes() + h->sort_block_bytes) + rot) + int64_t(nsteps) * grid + e;
 }
 
 int64_t mpm_record_bytes(mpm_handle h, int nsteps, int with_grid) {

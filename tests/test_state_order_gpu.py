@@ -51,3 +51,22 @@ def test_set_state_device_makes_the_slot_order_the_particle_order(dim, n):
         check(L.mpm_backward_step(h, slots.data_ptr(), gin.data_ptr(), None))
         sim.synchronize()
         assert torch.equal(gin, want)
+
+
+@pytest.mark.parametrize("dim,n", [(2, 300_000), (3, 200_000)])
+def test_a_segment_takes_the_memory_that_tape_bytes_says(dim, n):
+    """The first backward segment of an engine allocates what mpm_tape_bytes counts beyond a one-step segment, the
+    dL/dE contributions of its steps among it (31 x 4 bytes per particle here)."""
+    p, steps, taken = _cloud(dim, n, 5), 33, []
+    for k in (1, steps):
+        with MPMSimulation(p, MaterialModel.kJelly, 32, E=1.0, identity_mode=1) as sim:
+            L, h = lib(), sim._handle()
+            cot = torch.zeros(autodiff.channels(dim), n, device="cuda")
+            gE = torch.zeros(1, dtype=torch.float64, device="cuda")
+            torch.cuda.synchronize()
+            bytes_k = int(L.mpm_tape_bytes(h, k))
+            free = torch.cuda.mem_get_info()[0]
+            check(L.mpm_backward_segment(h, k, cot.data_ptr(), cot.data_ptr(), gE.data_ptr()))
+            sim.synchronize()
+            taken.append(free - torch.cuda.mem_get_info()[0] - bytes_k)
+    assert abs(taken[1] - taken[0]) < 20 << 20, taken  # some ten allocations, each rounded up to 2 MiB
