@@ -959,7 +959,7 @@ struct nclr_mpm_sim {
             : e(s), state{s.state[0], s.state[1]}, pid{s.pid[0], s.pid[1]}, cur(s.cur), steps(s.steps),
               graph(s.opts.graph), gv(s.gv) {
             s.opts.graph = 0;
-            s.slots_sorted = false;  // the segment's first step sorts into its tape entry
+            s.slots_sorted = false;
         }
         ~SegGuard() {
             for (int k = 0; k < 2; ++k) {
@@ -991,6 +991,14 @@ struct nclr_mpm_sim {
             state[slot] = reinterpret_cast<float*>(entry);
             pid[slot] = reinterpret_cast<uint32_t*>(entry + state_floats() * sizeof(float));
         }
+    }
+
+    // Before a segment that steps from the current state: its first step sorts into its tape entry also where the
+    // state's own sort stands (a sorted image).
+    int segment_sorts() {
+        if (sorted_valid && slots_sorted) HIP_TRY(nclr_host::launch_stop_off_grid(args(cur)));
+        slots_sorted = false;
+        return MPM_OK;
     }
 
     // Steps 0 .. nsteps - 2 of a segment from the current state, each into its tape entries: step t
@@ -1113,6 +1121,7 @@ struct nclr_mpm_sim {
         const bool grid_tape = tape_grid_states >= nsteps;
         const SegTape T{tape, sort_tape, grid_tape ? tape_gv : nullptr, grid_tape ? tape_gpre : nullptr,
                         grid_tape ? tape_rot : nullptr};
+        RC_TRY(segment_sorts());
         SegGuard g(*this);
         RC_TRY(record_steps(nsteps, T, g));
         return adjoint_steps(nsteps, T, g, gout, gin, grad_E);
@@ -1174,6 +1183,7 @@ struct nclr_mpm_sim {
         if (p.n == 0) {
             RC_TRY(advance(nsteps));
         } else {
+            RC_TRY(segment_sorts());
             SegGuard g(*this);
             RC_TRY(record_steps(nsteps, T, g));
             const int own = g.cur ^ 1;

@@ -241,6 +241,8 @@ hipError_t launch_image_to_slots(const LaunchArgs& a, const float* image, int ch
                                  uint32_t* changes);
 // The sort of the first step after that (perm is the identity, the tables stand).
 hipError_t launch_sorted_step(const LaunchArgs& a);
+// Ahead of a sort of that state all the same (a segment's first step sorts into its tape entry).
+hipError_t launch_stop_off_grid(const LaunchArgs& a);
 // The radix sort of a.p.n tile keys (in radix_keys_in's buffer), tile bounds (cleared) and work items.
 hipError_t launch_key_sort(const LaunchArgs& a);
 uint32_t* key_sort_input(const LaunchArgs& a);

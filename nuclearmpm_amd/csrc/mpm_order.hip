@@ -167,6 +167,14 @@ __global__ __launch_bounds__(256) void k_image_to_slots(uint32_t* __restrict__ p
     for (int c = 0; c < channels; ++c) st[int64_t(c) * stride + j] = image[int64_t(c) * n + i];
 }
 
+// Stops the scenes with a particle off their grid, ahead of an incremental sort from a sorted image: the sort
+// finds such particles itself, but in the launch that lists the node tiles, which leaves a stopped
+// scene's counts as they are.
+__global__ __launch_bounds__(256) void k_stop_off_grid(StepParams p, const uint32_t* __restrict__ off_grid) {
+    const int64_t s = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (s < p.nscenes && off_grid[s]) stop_scene(p, int(s), kStatusOutOfRange);
+}
+
 // The sort of the step after a sorted image: the slots are in order and the tables stand; the step's stamp,
 // the scenes with a particle off their grid and the node tiles are left to do.
 template <int D>
@@ -239,6 +247,11 @@ hipError_t launch_permute_channels(const uint32_t* pid, const float* src, int64_
         k_rows_to_channels<<<b, 256, 0, s>>>(to_particle_order ? nullptr : pid, rows, dst, dst_stride, channels, n,
                                              changes);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_stop_off_grid(const LaunchArgs& a) {
+    k_stop_off_grid<<<blocks_of(a.p.nscenes, 256), 256, 0, a.stream>>>(a.p, a.off_grid);
     return hipGetLastError();
 }
 

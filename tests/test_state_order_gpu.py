@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from nuclearmpm_amd import MaterialModel, MPMSimulation, Particles, autodiff
+from nuclearmpm_amd import MaterialModel, MPMBatch, MPMSimulation, Particles, SceneSpec, autodiff
 from nuclearmpm_amd._lib import check, lib
 
 pytestmark = pytest.mark.gpu
@@ -70,3 +70,45 @@ def test_a_segment_takes_the_memory_that_tape_bytes_says(dim, n):
             sim.synchronize()
             taken.append(free - torch.cuda.mem_get_info()[0] - bytes_k)
     assert abs(taken[1] - taken[0]) < 20 << 20, taken  # some ten allocations, each rounded up to 2 MiB
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("recorded", [0, 1, 3])
+def test_a_large_image_with_a_particle_off_one_scenes_grid(dim, recorded):
+    """The image of a batch, stored in tile order: its first step (of mpm_advance, or of a recorded segment of 1 or 3
+    steps, which sorts from that order) stops that scene alone.  The scene keeps its particles, grid and
+    active nodes; the others step as they do alone, bit for bit."""
+    sizes, res, steps = (100_001, 130_007, 40_003), 64, max(recorded, 1)
+    before = [_cloud(dim, n, 40 + s) for s, n in enumerate(sizes)]
+    for c in before:
+        c.x = (c.x * np.float32(0.4) + np.float32(0.1)).astype(np.float32)
+    after = [_cloud(dim, n, 50 + s) for s, n in enumerate(sizes)]
+    for c in after:
+        c.x = (c.x * np.float32(0.4) + np.float32(0.5)).astype(np.float32)  # no node tile in common
+    after[1].x[777, 0] = 2.0
+    rows = (torch.from_numpy(np.concatenate([getattr(c, k) for c in after])).cuda() for k in ("x", "v", "F", "C", "Jp"))
+    image = autodiff.pack(*rows)
+    with MPMBatch([SceneSpec(c, MaterialModel.kJelly, res, E=1.0) for c in before], identity_mode=1) as batch:
+        L, h = lib(), batch._handle()
+        batch.advance(2)
+        grid, active = batch.grid(1), batch.active_nodes(1)
+        tape = torch.empty(int(L.mpm_record_bytes(h, steps, 1)), dtype=torch.uint8, device="cuda")
+        torch.cuda.synchronize()
+        batch.set_state_image(image)
+        if recorded:
+            check(L.mpm_advance_recorded(h, steps, tape.data_ptr(), 1))
+        else:
+            batch.advance(steps)
+        assert batch.scene_status() == {1: {"flags": 1, "step": 3}}
+        assert batch.active_nodes(1) == active > 0
+        for a, b in zip(batch.grid(1), grid):
+            assert np.array_equal(a, b)
+        got = [batch.particles(s) for s in range(3)]
+    for k in ("x", "v", "F", "C", "Jp"):
+        assert np.array_equal(getattr(got[1], k), getattr(after[1], k)), k
+    for s in (0, 2):
+        with MPMSimulation(after[s], MaterialModel.kJelly, res, E=1.0, identity_mode=1) as sim:
+            sim.advance(steps)
+            alone = sim.particles()
+        for k in ("x", "v", "F", "C", "Jp"):
+            assert np.array_equal(getattr(got[s], k), getattr(alone, k)), (s, k)
