@@ -69,7 +69,7 @@ hipError_t dmalloc(T** p, size_t count) {
     return hipMalloc(reinterpret_cast<void**>(p), std::max<size_t>(count, 1) * sizeof(T));
 }
 
-bool valid_chunk(int c) { return c == 256 || c == 512 || c == 1024; }
+bool valid_chunk(int c) { return c == nclr_dev::kMinChunk || c == 512 || c == nclr_dev::kMaxChunk; }
 bool valid_threads(int t) { return t == 64 || t == 128 || t == 256; }
 
 }  // namespace

@@ -39,7 +39,7 @@ struct Tile<3> {
 };
 
 // Smallest P2G work item (particles per workgroup); the slot buffer is sized for it.
-constexpr int kMinChunk = 256;
+constexpr int kMinChunk = 256, kMaxChunk = 1024;
 
 // One scene (an independent simulation) of a batch.
 struct SceneParams {

@@ -182,11 +182,10 @@ __global__ __launch_bounds__(256) void k_sorted_step(StepParams p, uint32_t* __r
                                                      const uint32_t* __restrict__ off_grid,
                                                      const uint32_t* __restrict__ item_offset,
                                                      GridTile<D>* __restrict__ tiles, uint32_t* meta,
-                                                     uint32_t* __restrict__ active, int list) {
+                                                     uint32_t* __restrict__ active) {
     const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (t == 0) *stamp = *stamp + 1u;
     if (t < p.nscenes && off_grid[t]) stop_scene(p, int(t), kStatusOutOfRange);
-    if (!list) return;
     const bool stops = t < p.node_tiles && off_grid[p.nscenes == 1 ? 0 : scene_of_node_tile(p, uint32_t(t))] != 0u;
     list_grid_tile<D>(p, stops ? p.node_tiles : uint32_t(t), item_offset, tiles, &meta[kMetaGridTiles], active);
 }
@@ -229,6 +228,8 @@ static unsigned row_blocks(int64_t n) { return unsigned(std::min<int64_t>((n + k
 // Below this count the set fits the L2 caches and the direct form is as fast in any order (150,003
 // particles at random: 36 us, by rows 23 and the two launches that decide).
 constexpr int64_t kMinByRows = int64_t(1) << 18;
+// A sorted image's first step lists the node tiles: launches of that size do (grid_tiles_listed).
+static_assert(kMinByRows >= int64_t(kFewItems) * kMaxChunk, "sorted images have listed node tiles");
 
 hipError_t launch_permute_channels(const uint32_t* pid, const float* src, int64_t src_stride, float* dst,
                                    int64_t dst_stride, int channels, int64_t n, bool to_particle_order, float* rows,
@@ -257,13 +258,12 @@ hipError_t launch_stop_off_grid(const LaunchArgs& a) {
 
 hipError_t launch_sorted_step(const LaunchArgs& a) {
     const unsigned b = std::max(1u, blocks_of(std::max<int64_t>(a.p.node_tiles, a.p.nscenes), 256));
-    const int list = grid_tiles_listed(a.dim, a.p) ? 1 : 0;
     if (a.dim == 2)
         k_sorted_step<2><<<b, 256, 0, a.stream>>>(a.p, a.stamp, a.off_grid, a.item_offset,
-                                                  static_cast<GridTile<2>*>(a.grid_tiles), a.meta, a.active, list);
+                                                  static_cast<GridTile<2>*>(a.grid_tiles), a.meta, a.active);
     else
         k_sorted_step<3><<<b, 256, 0, a.stream>>>(a.p, a.stamp, a.off_grid, a.item_offset,
-                                                  static_cast<GridTile<3>*>(a.grid_tiles), a.meta, a.active, list);
+                                                  static_cast<GridTile<3>*>(a.grid_tiles), a.meta, a.active);
     return hipGetLastError();
 }
 
