@@ -487,9 +487,12 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(D == 3 && P
             float s = 0.0f;
 #pragma unroll
             for (int b = 0; b < D; ++b) s += fabsf(Cb[k].a[a][b]);
-            // |off - fx| <= 1.5 on every axis
-            const float bc = wsum * (fabsf(vb[k][a]) + 1.5f * four_inv_dx * s);
-            finite[k] = (a == 0 || finite[k]) && bc < 3.0e38f;
+            // |off - fx| is at most 1.5 on every axis, except in the half cell at the lower walls (stencil base 0,
+            // fx from -0.5 to 0.5): up to 2.5 there, but beyond 1.5 only at the third node, whose weight is at
+            // most an eighth of the axis's |weights|, so that no contribution exceeds the bound there either
+            const float vc = fabsf(vb[k][a]), bc = wsum * (vc + 1.5f * four_inv_dx * s);
+            // the unchecked deposits also need every bracket finite, which the weight is multiplied to
+            finite[k] = (a == 0 || finite[k]) && bc < 3.0e38f && vc + 2.5f * four_inv_dx * s < 3.0e38f;
             if (bc < 3.0e38f) bound[a] = fmaxf(bound[a], bc);
         }
     }

@@ -456,3 +456,53 @@ def test_backward_drops_the_node_counts_of_later_steps(dim, n, record):
         out = autodiff.rollout(b, x0, torch.tensor([1.0], requires_grad=True), 2, 2, record=record)
         out.square().sum().backward()
         assert b.active_nodes() == int((b.grid()[1] > 0).sum()) > 0
+
+
+@pytest.mark.parametrize("dim", [2, 3])
+@pytest.mark.parametrize("material", [MaterialModel.kJelly, MaterialModel.kSnow])
+def test_adjoint_of_particles_in_the_half_cell_at_the_lower_walls(dim, material):
+    """Stencil base 0 with an offset below 0.5, where a node is up to 2.5 cells away: gradients against the FP64
+    adjoint, and a cotangent whose bound is finite but whose bracket at the third node is not leaves that node
+    NaN, as every contribution out of range does."""
+    import torch
+
+    from nuclearmpm_amd import autodiff
+
+    res, n = 24, 64
+    rng = np.random.default_rng(dim)
+    s = 8.0 + 4.0 * rng.random((n, dim))
+    s[:, 0] = rng.uniform(0.02, 0.98, n)  # in cells: base 0, offset as it is
+    s[0] = [0.2] + [10.9] * (dim - 1)
+    s[1] = [3.0] + [10.9] * (dim - 1)     # shares the third node with it, no other on that axis
+    p = Particles.from_positions((s / res).astype(np.float32), identity_mode=1)
+    p.F = (p.F + rng.normal(0, 0.01, p.F.shape)).astype(np.float32)
+    p.v = rng.normal(0, 0.5, p.v.shape).astype(np.float32)
+    cot = rng.normal(size=(autodiff.channels(dim), n)).astype(np.float32)
+    with MPMSimulation(p, material, res, identity_mode=1) as sim:
+        image = sim.state_image()
+
+        def grad(c):
+            s0 = image.clone().requires_grad_(True)
+            out = autodiff.rollout(sim, s0, torch.tensor([1e4]), steps=1, checkpoint_every=1)
+            return torch.autograd.grad(out, s0, torch.from_numpy(c).cuda())[0].cpu().numpy()
+
+        got = grad(cot)
+        huge = np.zeros_like(cot)
+        huge[2 * dim + dim * dim, 0] = 1.95e38 / (4.0 * res)  # C_00: 1.5 of it in cells is in range, 1.8 is not
+        lost = grad(huge)
+    assert np.isnan(lost[dim, 1]), lost[dim, :4]
+    if material != MaterialModel.kJelly:
+        return
+    parts, at = [], 0
+    for shape in ((dim,), (dim,), (dim, dim), (dim, dim)):
+        w = int(np.prod(shape))
+        parts.append(np.ascontiguousarray(cot[at:at + w].T).reshape((n,) + shape).astype(np.float64))
+        at += w
+    ref = O.adjoint_jelly(O.State(x=p.x, v=p.v, F=p.F, C=p.C, Jp=p.Jp, mass=p.mass, volume=p.volume),
+                          O.Grads(*parts, Jp=cot[at].astype(np.float64)), res=res, E=1e4, identity_mode=1)
+    at = 0
+    for k in ("x", "v", "F", "C"):
+        r = getattr(ref, k).reshape(n, -1)
+        g = got[at:at + r.shape[1]].T
+        at += r.shape[1]
+        assert np.abs(g - r).max() <= 1e-4 * np.abs(r).max(), k  # the bound of the one-step gradient tests
