@@ -9,7 +9,7 @@
 //               consecutive original indices.
 //   tiles       particles are keyed by the tile of their stencil base cell (S^D cells, S = 16 in
 //               2D, 8 in 3D), tiles numbered scene after scene, and counting-sorted every step
-//               (mpm_sort.hip): perm maps sorted position -> slot, [tile_start, tile_end) per tile.
+//               (mpm_bucket.hip; the first step mpm_sort.hip): perm maps sorted position -> slot, [tile_start, tile_end) per tile.
 //   slots       per P2G work item (a chunk of one tile), its region of (S+2)^D nodes as float4
 //               {momentum, mass}.
 //   gv          the updated grid in node tiles of S^D nodes, float4 {v, m}; stamps[node tile] ==
@@ -22,8 +22,8 @@
 //          stamp), the radix sort of mpm_sort.hip, tile bounds and P2G work items
 //   p2g    one workgroup per work item: fused affine matrix per particle, quantised 3^D
 //          stencil contributions summed exactly with 64-bit LDS integer atomics, region -> slot
-//   grid   one workgroup per node tile: sums the slots covering each node, grid_op
-//          (src/nclr.h:263-310)
+//   grid   workgroups over the node tiles that particles reach, listed by the sort (small 2D launches:
+//          one per node tile): sums the slots covering each node, grid_op (src/nclr.h:263-310)
 //   g2p    per sorted position j: particle perm[j] -> slot j of the other buffer (the state stays
 //          physically sorted by tile)
 #include <hip/hip_runtime.h>
