@@ -257,7 +257,8 @@ int mpm_grad_to_saved_order(mpm_handle h, const void* order, const float* src, f
  *
  * Vector-Jacobian product of one step taken from the current state (every material: jelly; snow
  * with the backward pass of its singular-value clamp, its Jp update and its hardening; liquid):
- * grad_out is the cotangent of the state after the step in ITS slot order,
+ * grad_out is the cotangent of the state after the step in ITS slot order (the tiled step's; the
+ * compact step orders its slots differently),
  * grad_in (must not alias grad_out) receives the cotangent of the current state in the current
  * slot order, and grad_E[s] += dL/dE of scene s (nscenes doubles; NULL: not accumulated).  The
  * state and the step counter are unchanged; the grid export afterwards shows this step's grid. */
@@ -266,9 +267,13 @@ int mpm_backward_step(mpm_handle h, const float* grad_out, float* grad_in, doubl
 /* Vector-Jacobian product of `nsteps` steps from the current state (a checkpoint): recomputes
  * the states inside the segment on the device into a tape of nsteps - 1 states and their sorts
  * (device memory, allocated on first use and grown to the longest segment), then runs nsteps
- * backward steps in reverse on the tape.  grad_out is in the slot order of the state nsteps steps ahead, grad_in in
- * the current slot order (they may alias).  The current state is left as it was. */
+ * backward steps in reverse on the tape.  grad_out is in the slot order of the state nsteps tiled steps
+ * ahead (the compact step leaves another order), grad_in in the current slot order (they may alias).
+ * The current state is left as it was. */
 int mpm_backward_segment(mpm_handle h, int nsteps, const float* grad_out, float* grad_in, double* grad_E);
+/* The same with grad_out and grad_in in particle order, whatever order the forward steps left: for
+ * engines that advance with the compact step. */
+int mpm_backward_segment_particles(mpm_handle h, int nsteps, const float* grad_out, float* grad_in, double* grad_E);
 
 /* Device bytes of the tape mpm_backward_segment keeps for segments of `nsteps` steps (-1 for a
  * NULL handle or nsteps < 1): nsteps - 1 entries of one state snapshot (mpm_state_bytes) and one

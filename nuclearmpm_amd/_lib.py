@@ -164,6 +164,8 @@ def lib() -> ctypes.CDLL:
     L.mpm_backward_step.restype = i32
     L.mpm_backward_segment.argtypes = [H, i32, _vp, _vp, _vp]
     L.mpm_backward_segment.restype = i32
+    L.mpm_backward_segment_particles.argtypes = [H, i32, _vp, _vp, _vp]
+    L.mpm_backward_segment_particles.restype = i32
     L.mpm_tape_bytes.argtypes = [H, i32]
     L.mpm_tape_bytes.restype = i64
     L.mpm_record_bytes.argtypes = [H, i32, i32]

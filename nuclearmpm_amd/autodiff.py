@@ -13,11 +13,15 @@ states, sorts and optionally grids the recomputation would produce, on a device 
 and their backward skips the recomputation (mpm_backward_recorded); the gradients are bitwise the
 same, the device memory grows by one tape per recorded segment.
 
+The backward pass takes tiled steps.  Where the forward pass takes the compact step, which orders its slots
+differently, cotangents go from segment to segment in particle order (mpm_backward_segment_particles).
+
 State tensors are (channels, n) float32 on the engine's device: rows x[d], v[d], F[d*d], C[d*d]
 (matrices row-major), Jp, particles in the order the simulation was created with.
 """
 from __future__ import annotations
 
+import ctypes
 from typing import Optional, Tuple
 
 import torch
@@ -116,6 +120,15 @@ class _Rollout(torch.autograd.Function):
         check(L.mpm_set_state_device_any_order(h, state0.data_ptr()))
         sb = int(L.mpm_state_bytes(h))
         plan = _record_plan(L, h, steps, every, record, state0.device)
+        ppt = ctypes.c_int()
+        check(L.mpm_get_compact(h, ctypes.byref(ppt)))
+        compact = ppt.value > 0
+
+        def slot_order():
+            order = torch.empty(int(L.mpm_order_bytes(h)), dtype=torch.uint8, device=state0.device)
+            check(L.mpm_save_order(h, order.data_ptr()))
+            return order
+
         ckpts = []
         done = 0
         for mode in plan:
@@ -128,18 +141,18 @@ class _Rollout(torch.autograd.Function):
             else:
                 rec = torch.empty(int(L.mpm_record_bytes(h, k, mode)), dtype=torch.uint8, device=state0.device)
                 check(L.mpm_advance_recorded(h, k, rec.data_ptr(), mode))
-            ckpts.append((buf, k, rec, mode))
             done += k
-        # the final state's slot order, in which its cotangent is wanted
-        order = torch.empty(int(L.mpm_order_bytes(h)), dtype=torch.uint8, device=state0.device)
-        check(L.mpm_save_order(h, order.data_ptr()))
+            # the slot order in which the segment's backward pass wants its cotangent: with tiled steps only
+            # at the end (in between it is the next segment's first)
+            last = slot_order() if (rec is not None if compact else done == steps) else None
+            ckpts.append((buf, k, rec, mode, last))
         out = torch.empty_like(state0)
         check(L.mpm_get_state_device(h, out.data_ptr()))
         check(L.mpm_synchronize(h))
         sim._cache = None
         ctx.sim = sim
         ctx.ckpts = ckpts
-        ctx.order = order
+        ctx.compact = compact
         ctx.E_meta = (E.dtype, E.device, E.shape)
         ctx.E_vals = E_vals
         ctx.nu_vals = list(sim._nus)
@@ -156,17 +169,28 @@ class _Rollout(torch.autograd.Function):
         # this rollout's E (another rollout or set_elasticity may have changed it since)
         for s, (e, nu) in enumerate(zip(ctx.E_vals, ctx.nu_vals)):
             sim.set_elasticity(s, e, nu)
-        g = torch.empty_like(g_user)
-        check(L.mpm_grad_to_saved_order(h, ctx.order.data_ptr(), g_user.data_ptr(), g.data_ptr()))
-        for buf, k, rec, mode in reversed(ctx.ckpts):
+        g, g0 = torch.empty_like(g_user), torch.empty_like(g_user)
+        if ctx.compact:
+            g0.copy_(g_user)
+            _ready(g0)
+        for buf, k, rec, mode, last in reversed(ctx.ckpts):
+            if ctx.compact and rec is None:
+                check(L.mpm_load_state(h, buf.data_ptr()))
+                check(L.mpm_backward_segment_particles(h, int(k), g0.data_ptr(), g0.data_ptr(), gE.data_ptr()))
+                continue
+            if last is not None:
+                src = g0 if ctx.compact else g_user
+                check(L.mpm_grad_to_saved_order(h, last.data_ptr(), src.data_ptr(), g.data_ptr()))
             check(L.mpm_load_state(h, buf.data_ptr()))
             if rec is None:
                 check(L.mpm_backward_segment(h, int(k), g.data_ptr(), g.data_ptr(), gE.data_ptr()))
             else:
                 check(L.mpm_backward_recorded(h, int(k), rec.data_ptr(), mode, g.data_ptr(), g.data_ptr(),
                                               gE.data_ptr()))
-        g0 = torch.empty_like(g)
-        check(L.mpm_grad_to_particle_order(h, g.data_ptr(), g0.data_ptr()))
+            if ctx.compact:
+                check(L.mpm_grad_to_particle_order(h, g.data_ptr(), g0.data_ptr()))
+        if not ctx.compact:
+            check(L.mpm_grad_to_particle_order(h, g.data_ptr(), g0.data_ptr()))
         check(L.mpm_synchronize(h))
         sim._cache = None
         dtype, device, shape = ctx.E_meta

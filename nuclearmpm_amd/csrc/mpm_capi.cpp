@@ -884,8 +884,9 @@ struct nclr_mpm_sim {
     // forward grid (a backward segment's recomputed step wrote them): only the adjoint kernels run.
     // order_kept: the state is stored in the order of prev_sort's sort (a segment's last state): the
     // sort is the incremental one.  slot: where the step's dL/dE contributions go (sum_e adds them up).
+    // particles: gout's values in particle order; gout itself is written, in the slot order after the step.
     int backward_step(const float* gout, float* gin, bool presorted = false, bool grid_kept = false,
-                      bool order_kept = false, int slot = 0) {
+                      bool order_kept = false, int slot = 0, const float* particles = nullptr) {
         RC_TRY(ensure_adjoint());
         RC_TRY(ensure_e_steps(1));
         if (p.n == 0) return MPM_OK;
@@ -904,6 +905,11 @@ struct nclr_mpm_sim {
                 if (order_kept) RC_TRY(timed(kSort, [&] { return nclr_host::launch_sort_incremental(a); }));
                 else RC_TRY(timed(kSort, [&] { return nclr_host::launch_sort(a); }));
                 sorted_valid = false;
+            }
+            if (particles) {  // uidx is free between sorts
+                HIP_TRY(nclr_host::launch_sorted_order(a, uidx));
+                HIP_TRY(nclr_host::launch_permute_channels(uidx, particles, p.n, const_cast<float*>(gout), p.n,
+                                                           grad_channels(), p.n, false, nullptr, nullptr, stream));
             }
             RC_TRY(timed(kP2G, [&] { return nclr_host::launch_p2g(a); }));
             RC_TRY(timed(kGrid, [&] { return nclr_host::launch_grid(a); }));
@@ -1030,12 +1036,15 @@ struct nclr_mpm_sim {
     // they run only the adjoint kernels.  The last state was never stepped, so its adjoint step
     // sorts and recomputes its grid; the first one's (t = 0) grid becomes the engine's own, so the
     // grid export and active-node count afterwards show a step from the segment's start.
+    // particles: gout and gin are in particle order.
     int adjoint_steps(int nsteps, const SegTape& T, const SegGuard& g, const float* gout, float* gin,
-                      double* grad_E) {
+                      double* grad_E, bool particles = false) {
         const size_t gn = gv_nodes();
         // the first step reads gout, the last one writes gin; one step that is both reads a copy (they may alias)
         const float* from = gout;
-        if (nsteps == 1) {
+        if (particles) {
+            from = gtmp[nsteps & 1];
+        } else if (nsteps == 1) {
             const size_t gbytes = size_t(grad_channels()) * size_t(p.n) * sizeof(float);
             HIP_TRY(hipMemcpyAsync(gtmp[0], gout, gbytes, hipMemcpyDeviceToDevice, stream));
             from = gtmp[0];
@@ -1062,14 +1071,17 @@ struct nclr_mpm_sim {
             // the last state is stored in the order of the step before's sort
             const bool order_kept = !kept && t > 0;
             prev_sort = order_kept ? T.sorts + sort_block_bytes * size_t(t - 1) : nullptr;
-            float* to = t == 0 ? gin : gtmp[t & 1];
-            RC_TRY(backward_step(from, to, kept, kept && T.gv, order_kept, held));
+            float* to = t == 0 && !particles ? gin : gtmp[t & 1];
+            RC_TRY(backward_step(from, to, kept, kept && T.gv, order_kept, held, particles && !kept ? gout : nullptr));
             from = to;
             if (grad_E && (++held == e_steps || held == nclr_dev::kESteps || t == 0)) {
                 RC_TRY(sum_e(t + held - 1, held, nsteps, T.sorts, grad_E));
                 held = 0;
             }
         }
+        if (particles)
+            HIP_TRY(nclr_host::launch_permute_channels(pid[cur], from, p.n, gin, p.n, grad_channels(), p.n, true, nullptr,
+                                                       nullptr, stream));
         return MPM_OK;
     }
 
@@ -1077,7 +1089,7 @@ struct nclr_mpm_sim {
     // recomputed straight into the engine's tape (record_steps) and the adjoint steps run on it
     // (adjoint_steps); no state copies.  The engine's own buffers, pointers and step counter are
     // restored at the end, so the state is the checkpoint again.
-    int backward_segment(int nsteps, const float* gout, float* gin, double* grad_E) {
+    int backward_segment(int nsteps, const float* gout, float* gin, double* grad_E, bool particles = false) {
         if (nsteps < 1) return fail(MPM_ERR_INVALID, "nsteps must be >= 1");
         RC_TRY(ensure_adjoint());
         if (p.n == 0) return MPM_OK;
@@ -1124,7 +1136,7 @@ struct nclr_mpm_sim {
         RC_TRY(segment_sorts());
         SegGuard g(*this);
         RC_TRY(record_steps(nsteps, T, g));
-        return adjoint_steps(nsteps, T, g, gout, gin, grad_E);
+        return adjoint_steps(nsteps, T, g, gout, gin, grad_E, particles);
     }
 
     // A recorded segment's tape inside caller memory: states, sort blocks, then (with_grid) the
@@ -1819,6 +1831,13 @@ int mpm_backward_segment(mpm_handle h, int nsteps, const float* grad_out, float*
     HIP_TRY(hipSetDevice(h->opts.device));
     RC_TRY(h->require_live());
     return h->backward_segment(nsteps, grad_out, grad_in, grad_E);
+}
+
+int mpm_backward_segment_particles(mpm_handle h, int nsteps, const float* grad_out, float* grad_in, double* grad_E) {
+    if (!h || ((!grad_out || !grad_in) && h->p.n > 0)) return fail(MPM_ERR_INVALID, "NULL argument");
+    HIP_TRY(hipSetDevice(h->opts.device));
+    RC_TRY(h->require_live());
+    return h->backward_segment(nsteps, grad_out, grad_in, grad_E, true);
 }
 
 int64_t mpm_tape_bytes(mpm_handle h, int nsteps) {

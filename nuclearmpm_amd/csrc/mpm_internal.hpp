@@ -228,6 +228,8 @@ hipError_t launch_p2g_adjoint(const LaunchArgs& a, const AdjointArgs& b);
 hipError_t launch_permute_channels(const uint32_t* pid, const float* src, int64_t src_stride, float* dst,
                                    int64_t dst_stride, int channels, int64_t n, bool to_particle_order, float* rows,
                                    uint32_t* changes, hipStream_t s);
+// order[j] = the particle of sorted position j, after a sort of a.state_in (the slot order of the state a step on).
+hipError_t launch_sorted_order(const LaunchArgs& a, uint32_t* order);
 // A state in slot order as particle-major arrays in particle order, one behind the other (n of each): x, v, F, C,
 // Jp, mass, volume.
 hipError_t launch_particles_out(int dim, const float* st, const uint32_t* pid, int64_t n, int64_t stride, float* out,

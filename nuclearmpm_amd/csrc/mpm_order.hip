@@ -190,6 +190,13 @@ __global__ __launch_bounds__(256) void k_sorted_step(StepParams p, uint32_t* __r
     list_grid_tile<D>(p, stops ? p.node_tiles : uint32_t(t), item_offset, tiles, &meta[kMetaGridTiles], active);
 }
 
+// order[j] = the particle of sorted position j.
+__global__ __launch_bounds__(256) void k_sorted_order(const uint32_t* __restrict__ pid, const uint32_t* __restrict__ perm,
+                                                      uint32_t* __restrict__ order, int64_t n) {
+    const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (j < n) order[j] = pid[perm[j]];
+}
+
 // Slots -> particle-major arrays in particle order, for the host: the device does the reordering and the
 // transposition, so that the host only copies.
 template <int D>
@@ -272,6 +279,12 @@ hipError_t launch_particles_out(int dim, const float* st, const uint32_t* pid, i
     if (n <= 0) return hipSuccess;
     if (dim == 2) k_particles_out<2><<<blocks_of(n, 256), 256, 0, s>>>(st, pid, n, stride, out);
     else k_particles_out<3><<<blocks_of(n, 256), 256, 0, s>>>(st, pid, n, stride, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_sorted_order(const LaunchArgs& a, uint32_t* order) {
+    if (a.p.n <= 0) return hipSuccess;
+    k_sorted_order<<<blocks_of(a.p.n, 256), 256, 0, a.stream>>>(a.pid_in, a.perm, order, a.p.n);
     return hipGetLastError();
 }
 
