@@ -9,7 +9,8 @@
 //               consecutive original indices.
 //   tiles       particles are keyed by the tile of their stencil base cell (S^D cells, S = 16 in
 //               2D, 8 in 3D), tiles numbered scene after scene, and counting-sorted every step
-//               (mpm_bucket.hip; the first step mpm_sort.hip): perm maps sorted position -> slot, [tile_start, tile_end) per tile.
+//               (mpm_bucket.hip; the first step mpm_sort.hip): perm maps sorted position ->
+//               slot, [tile_start, tile_end) per tile.
 //   slots       per P2G work item (a chunk of one tile), its region of (S+2)^D nodes as float4
 //               {momentum, mass}.
 //   gv          the updated grid in node tiles of S^D nodes, float4 {v, m}; stamps[node tile] ==
